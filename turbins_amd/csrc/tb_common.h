@@ -276,6 +276,8 @@ struct ConcSlot {
     double *cin = nullptr, *cout = nullptr, *cout_old = nullptr;
 };
 
+constexpr int XFER_TEAM = 8;   // threads of a large host transfer, each with a pinned slot
+
 struct tb_ctx {
     tb_config cfg;
     std::string err;
@@ -330,6 +332,8 @@ struct tb_ctx {
     double *hscal = nullptr;     // pinned host mirror of scal
     unsigned long long *hseq = nullptr;   // pinned word the device writes after publishing scalars
     unsigned long long pub_seq = 0;       // last sequence number asked for
+    char *xfer_pin = nullptr;             // pinned slots of the host transfers (allocated on the first large one)
+    hipEvent_t xfer_ev[XFER_TEAM] = {};
 
     // multigrid
     int nlev = 0;

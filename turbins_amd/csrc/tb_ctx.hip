@@ -3,6 +3,8 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <exception>
+#include <thread>
 
 #include "tb_common.h"
 
@@ -191,6 +193,9 @@ extern "C" void tb_destroy(tb_ctx *c) {
     hipFree(c->scal);
     if (c->hscal) hipHostFree(c->hscal);
     if (c->hseq) hipHostFree(c->hseq);
+    if (c->xfer_pin) hipHostFree(c->xfer_pin);
+    for (int w = 0; w < XFER_TEAM; w++)
+        if (c->xfer_ev[w]) hipEventDestroy(c->xfer_ev[w]);
     for (int e = 0; e < 2; e++)
         if (c->net_ev[e]) hipEventDestroy(c->net_ev[e]);
     if (c->ev0) hipEventDestroy(c->ev0);
@@ -227,11 +232,95 @@ extern "C" int tb_grid_array(tb_ctx *c, int which, double *out, int capacity) {
 }
 
 // ---------------------------------------------------------------------------
+// Field transfers.  The host side is dense (NX points a row), the device side
+// padded to px.  A strided copy of pageable memory goes row by row (7.5 us a
+// row, whatever its length: 247 ms for a 135 MB field of 33 k rows), so a
+// kernel packs the rows into the scratch vector kv[4] (or unpacks them from
+// it) and the dense block crosses the bus in one piece.  kv[4] is free between
+// calls and no solver presumes anything of its contents.
+template <typename T>
+__global__ void __launch_bounds__(256) k_pack_rows(const T *__restrict__ src, int spitch, T *__restrict__ dst,
+                                                   int dpitch, int nx, long rows) {
+    const long r = blockIdx.x * 4L + threadIdx.y;
+    if (r >= rows) return;
+    for (int i = threadIdx.x; i < nx; i += 64) dst[r * dpitch + i] = src[r * spitch + i];
+}
+
+template <typename T>
+static int pack_rows(tb_ctx *c, const T *src, int spitch, T *dst, int dpitch) {
+    const long rows = (long)c->d.NY * c->d.NZ;
+    hipLaunchKernelGGL(k_pack_rows<T>, dim3((unsigned)((rows + 3) / 4)), dim3(64, 4), 0, c->s, src, spitch, dst,
+                       dpitch, c->d.NX, rows);
+    TB_LAUNCH_CHECK(c);
+    return 0;
+}
+
+// A dense device block <-> pageable host memory.  One stream of host copies
+// (the runtime's own staging) reaches 17 GB/s, the bus 57 GB/s: from
+// XFER_MIN bytes up XFER_TEAM threads each move every XFER_TEAM-th chunk
+// through a pinned slot of their own, so that one chunk is on the bus while
+// the others are copied and their pages first touched.  The copies are
+// queued on the context's stream, behind the kernel that packed the block
+// and ahead of the one that unpacks it; the team has ended on return.
+constexpr size_t XFER_CHUNK = 2u << 20;
+constexpr size_t XFER_MIN = 8u << 20;
+
+static int xfer_slots(tb_ctx *c) {
+    if (c->xfer_pin) return 0;
+    for (int w = 0; w < XFER_TEAM; w++)
+        if (!c->xfer_ev[w]) TB_CHECK(c, hipEventCreateWithFlags(&c->xfer_ev[w], hipEventDisableTiming));
+    TB_CHECK(c, hipHostMalloc((void **)&c->xfer_pin, XFER_CHUNK * XFER_TEAM, hipHostMallocDefault));
+    return 0;
+}
+
+// worker w's chunks; returns the first HIP error
+static hipError_t xfer_worker(tb_ctx *c, int w, int dev, char *host, char *block, size_t bytes, bool up) {
+    hipError_t e = hipSetDevice(dev);
+    char *slot = c->xfer_pin + XFER_CHUNK * w;
+    for (size_t o = XFER_CHUNK * w; e == hipSuccess && o < bytes; o += XFER_CHUNK * XFER_TEAM) {
+        const size_t m = bytes - o < XFER_CHUNK ? bytes - o : XFER_CHUNK;
+        if (up) memcpy(slot, host + o, m);
+        e = up ? hipMemcpyAsync(block + o, slot, m, hipMemcpyHostToDevice, c->s)
+               : hipMemcpyAsync(slot, block + o, m, hipMemcpyDeviceToHost, c->s);
+        if (e == hipSuccess) e = hipEventRecord(c->xfer_ev[w], c->s);
+        if (e == hipSuccess) e = hipEventSynchronize(c->xfer_ev[w]);   // the slot is used again
+        if (e == hipSuccess && !up) memcpy(host + o, slot, m);
+    }
+    return e;
+}
+
+static int xfer(tb_ctx *c, void *host, void *block, size_t bytes, bool up) {
+    if (bytes < XFER_MIN) {
+        TB_CHECK(c, up ? hipMemcpyAsync(block, host, bytes, hipMemcpyHostToDevice, c->s)
+                       : hipMemcpyAsync(host, block, bytes, hipMemcpyDeviceToHost, c->s));
+        if (!up) TB_CHECK(c, hipStreamSynchronize(c->s));
+        return 0;
+    }
+    if (xfer_slots(c)) return -1;
+    int dev = 0;
+    TB_CHECK(c, hipGetDevice(&dev));
+    hipError_t err[XFER_TEAM];
+    std::thread team[XFER_TEAM];
+    for (int w = 0; w < XFER_TEAM; w++) {
+        auto work = [=, &err] { err[w] = xfer_worker(c, w, dev, (char *)host, (char *)block, bytes, up); };
+        try {
+            if (w + 1 < XFER_TEAM) team[w] = std::thread(work);
+            else work();
+        } catch (const std::exception &) {
+            work();   // no thread to be had: this one moves the chunks
+        }
+    }
+    for (std::thread &t : team)
+        if (t.joinable()) t.join();
+    for (hipError_t e : err) TB_CHECK(c, e);
+    return 0;
+}
+
 extern "C" int tb_upload_field(tb_ctx *c, int f, const double *host) {
     if (!c || f < 0 || f >= TB_F_COUNT || !host) { if (c) c->err = "tb_upload_field: bad argument"; return -1; }
     const Dims &d = c->d;
-    TB_CHECK(c, hipMemcpy2DAsync(c->f[f], sizeof(double) * d.px, host, sizeof(double) * d.NX,
-                                 sizeof(double) * d.NX, (size_t)d.NY * d.NZ, hipMemcpyHostToDevice, c->s));
+    if (xfer(c, const_cast<double *>(host), c->kv[4], sizeof(double) * d.NX * (size_t)d.NY * d.NZ, true)) return -1;
+    if (pack_rows<double>(c, c->kv[4], d.NX, c->f[f], d.px)) return -1;
     TB_CHECK(c, hipStreamSynchronize(c->s));
     if (f == TB_F_PHI) c->n_hist = c->gram_n = c->guess_nr = 0;
     tb_field_written(c, f);
@@ -241,18 +330,15 @@ extern "C" int tb_upload_field(tb_ctx *c, int f, const double *host) {
 extern "C" int tb_download_field(tb_ctx *c, int f, double *host) {
     if (!c || f < 0 || f >= TB_F_COUNT || !host) { if (c) c->err = "tb_download_field: bad argument"; return -1; }
     const Dims &d = c->d;
-    TB_CHECK(c, hipMemcpy2DAsync(host, sizeof(double) * d.NX, c->f[f], sizeof(double) * d.px,
-                                 sizeof(double) * d.NX, (size_t)d.NY * d.NZ, hipMemcpyDeviceToHost, c->s));
-    TB_CHECK(c, hipStreamSynchronize(c->s));
-    return 0;
+    if (pack_rows<double>(c, c->f[f], d.px, c->kv[4], d.NX)) return -1;
+    return xfer(c, host, c->kv[4], sizeof(double) * d.NX * (size_t)d.NY * d.NZ, false);
 }
 
 extern "C" int tb_download_flags(tb_ctx *c, int q, uint8_t *out) {
     if (!c || q < 0 || q > 3 || !out) { if (c) c->err = "tb_download_flags: bad argument"; return -1; }
     const Dims &d = c->d;
-    TB_CHECK(c, hipMemcpy2DAsync(out, d.NX, c->st[q], d.px, d.NX, (size_t)d.NY * d.NZ, hipMemcpyDeviceToHost, c->s));
-    TB_CHECK(c, hipStreamSynchronize(c->s));
-    return 0;
+    if (pack_rows<uint8_t>(c, c->st[q], d.px, (uint8_t *)c->kv[4], d.NX)) return -1;
+    return xfer(c, out, c->kv[4], (size_t)d.NX * d.NY * d.NZ, false);
 }
 
 extern "C" int tb_ib_count(tb_ctx *c, int q) {

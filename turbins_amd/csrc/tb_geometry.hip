@@ -551,8 +551,7 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
             hipLaunchKernelGGL(k_ls_norm, tiles_grid(all), tiles_block(), 0, c->s, d, c->g, sdf_c, pold, part, all);
             hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, c->s, part, all.per_xcd * NXCD, c->scal + S_TMP0);
             TB_LAUNCH_CHECK(c);
-            TB_CHECK(c, hipMemcpyAsync(c->hscal + S_TMP0, c->scal + S_TMP0, sizeof(double), hipMemcpyDeviceToHost, c->s));
-            TB_CHECK(c, hipStreamSynchronize(c->s));
+            if (tb_read_scalars(c, S_TMP0, 1)) return -1;
             double W_E = sqrt(c->hscal[S_TMP0]);
             int flag = (W_E < 1.0e-5);
             if ((it > max_iterations + 1) || flag) converged = 1;
@@ -598,7 +597,7 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
     for (int q = 0; q < 4; q++) {
         tb_free_ib(c, q);
         if (!c->has_geometry) continue;
-        TB_CHECK(c, hipMemcpy2D(hf.data(), d.NX, c->st[q], d.px, d.NX, (size_t)d.NY * d.NZ, hipMemcpyDeviceToHost));
+        if (tb_download_flags(c, q, hf.data())) return -1;
         std::vector<tb_ib_node> nodes;
         for (int k = 0; k < d.NZ; k++)
             for (int j = 0; j < d.NY; j++)
