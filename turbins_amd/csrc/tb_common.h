@@ -120,12 +120,14 @@ __device__ inline bool tile_point_kfast(const Tiles &t, int &i, int &j, int &k) 
 // column 512 and row 256) are listed 256 to a block, and the last k chunk
 // takes up to KCHUNK/2 extra planes (129 planes: 8 chunks, not 9).  Each
 // block is a chain of plane steps, so nearly empty tiles would cost as much
-// time as full ones.
+// time as full ones; for the same reason grids with fewer than
+// KTILES_BLOCKS blocks (four per CU) are walked in shorter chunks.
 constexpr int KCHUNK = 16;
+constexpr int KTILES_BLOCKS = 1024;
 
 struct KTiles {
     int nx, ny, nz;
-    int tx, ty, kc;     // full tiles per axis, k chunks
+    int tx, ty, kc, ch; // full tiles per axis, k chunks, planes per chunk
     int fx, fy;         // extent of the full tiles
     int ne, eb;         // columns outside the full tiles, blocks listing them (per chunk)
     long n, per_xcd;    // blocks: (tx * ty + eb) * kc
@@ -140,8 +142,11 @@ inline KTiles make_ktiles(int nx, int ny, int nz) {
     t.fy = t.ty * TILE_Y;
     t.ne = nx * ny - t.fx * t.fy;
     t.eb = (t.ne + TILE_X * TILE_Y - 1) / (TILE_X * TILE_Y);
-    t.kc = (nz + KCHUNK / 2) / KCHUNK;
-    if (t.kc < 1) t.kc = 1;
+    for (t.ch = KCHUNK;; t.ch /= 2) {
+        t.kc = (nz + t.ch / 2) / t.ch;
+        if (t.kc < 1) t.kc = 1;
+        if (t.ch == 2 || (t.tx * t.ty + t.eb) * t.kc >= KTILES_BLOCKS) break;
+    }
     t.n = (long)(t.tx * t.ty + t.eb) * t.kc;
     t.per_xcd = (t.n + NXCD - 1) / NXCD;
     return t;
@@ -166,8 +171,8 @@ __device__ inline void ktile_column(const KTiles &t, int &i, int &j, int &k0, in
     // do not form the tail of the launch
     const int r0 = lt - kc * per_chunk;
     const int r = r0 < t.eb ? r0 + nmain : r0 - t.eb;
-    k0 = kc * KCHUNK;
-    k1 = (kc == t.kc - 1) ? t.nz : k0 + KCHUNK;
+    k0 = kc * t.ch;
+    k1 = (kc == t.kc - 1) ? t.nz : k0 + t.ch;
     if (r < nmain) {
         i = (r % t.tx) * TILE_X + threadIdx.x;
         j = (r / t.tx) * TILE_Y + threadIdx.y;

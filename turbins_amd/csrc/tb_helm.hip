@@ -364,7 +364,7 @@ __device__ inline double gs_value(const HelmOp &H, const AxisGS &X, const AxisGS
 // axis, see AxisGS), while xo and b are read from HBM once and xn written
 // once (the in-place form streams both arrays twice).
 //
-// A 512-thread block owns a 64 x 16 column tile and a chunk of GS_TK planes
+// A 512-thread block owns a 64 x 16 column tile and a chunk of T.tk planes
 // and walks k upwards through two LDS rings: four planes of xo with a
 // two-point halo, and three of the red-pass values (black positions holding
 // xo) with a one-point halo.  Per plane m, with two barriers: store plane m-2
@@ -375,14 +375,18 @@ __device__ inline double gs_value(const HelmOp &H, const AxisGS &X, const AxisGS
 // xo plane, statuses and right-hand sides of the next plane are fetched into
 // registers one step ahead, so their latency overlaps the passes; row
 // coefficients come from per-axis tables built in LDS once per block.
-// 32-plane chunks: at 512 x 256 x 128 the 8 x 16 x 4 tiles are exactly the
-// blocks resident at once (two per CU at 75 KB of LDS), so no second round
-// runs on a partly idle chip, and the chunk ends recompute 1/16 of the
-// planes instead of 1/8 (126 -> 115 us per pair against 16-plane chunks).
-constexpr int GS_TX = 64, GS_TY = 16, GS_TK = 32;
+// Chunks of up to 32 planes: a block is a chain of tk + 3 plane steps behind
+// a start of about three more, and 512 blocks are resident at once (two per
+// CU at 75 KB of LDS; two of a CU take 8/5 of the time per step that one does:
+// 2.9 against 1.8 us), so make_gs_tiles takes the chunk with the least time in
+// sequence.  At 512 x 256 x 128 that is 32 (8 x 16 x 4 tiles, one round;
+// 126 -> 115 us per pair against 16 planes); small grids fill the chip with
+// short chains instead of leaving most of it idle (64 -> 11 us a pair at
+// 128x64x32).
+constexpr int GS_TX = 64, GS_TY = 16, GS_TK_MAX = 32;
 constexpr int GS_OX = GS_TX + 4, GS_OY = GS_TY + 4;   // xo ring: halo 2
 constexpr int GS_HX = GS_TX + 2, GS_HY = GS_TY + 2;   // red-pass ring: halo 1
-constexpr int GS_OZ = GS_TK + 4;                      // z table: k0-2 .. k0+GS_TK+1
+constexpr int GS_OZ = GS_TK_MAX + 4;                  // z table: k0-2 .. k0+tk+1
 constexpr int GS_ORING = 4;                           // xo planes staged: m-1, m, m+1 and the next
 constexpr int GS_THREADS = 512;
 constexpr int GS_OLD_PER = (GS_OY * GS_OX + GS_THREADS - 1) / GS_THREADS;
@@ -392,9 +396,12 @@ static_assert(GS_TX * GS_TY == 2 * GS_THREADS, "one black point per thread");
 static_assert(GS_TX % 2 == 0, "tile origins must be even");
 
 struct GsTiles {
-    int tx, ty, kc;
+    int tx, ty, kc, tk;   // tiles per axis, planes per chunk
     int n, per_xcd;
 };
+
+constexpr long GS_RESIDENT = 512;   // blocks resident at once
+constexpr int GS_START = 3;         // plane steps a block's start takes
 
 // The tiles cover the box without its last plane along each axis (see
 // k_gs_last_planes), so 512 x 256 x 128 cells take exactly 8 x 16 x 4 tiles
@@ -403,7 +410,13 @@ static GsTiles make_gs_tiles(const Dims &d) {
     GsTiles t;
     t.tx = (d.NX - 1 + GS_TX - 1) / GS_TX;
     t.ty = (d.NY - 1 + GS_TY - 1) / GS_TY;
-    t.kc = (d.NZ - 1 + GS_TK - 1) / GS_TK;
+    long best = 0;
+    for (int tk = GS_TK_MAX; tk >= 1; tk--) {
+        const long kc = (d.NZ - 1 + tk - 1) / tk, n = t.tx * t.ty * kc;
+        const long step = n <= GS_RESIDENT / 2 ? 5 : 8 * ((n + GS_RESIDENT - 1) / GS_RESIDENT);
+        const long cost = step * (tk + 3 + GS_START);
+        if (best == 0 || cost < best) { best = cost; t.tk = tk; t.kc = (int)kc; }
+    }
     t.n = t.tx * t.ty * t.kc;
     t.per_xcd = (t.n + NXCD - 1) / NXCD;
     return t;
@@ -431,8 +444,8 @@ __global__ void __launch_bounds__(GS_THREADS) k_helm_gs_pair(HelmOp H, const dou
     if (lt >= T.n) return;                                  // whole block
     const int tx = lt % T.tx, rest = lt / T.tx;
     const int i0 = tx * GS_TX, j0 = (rest % T.ty) * GS_TY;
-    const int k0 = (rest / T.ty) * GS_TK;
-    const int k1 = k0 + GS_TK < NZ - 1 ? k0 + GS_TK : NZ - 1;   // the last plane: k_gs_last_planes
+    const int k0 = (rest / T.ty) * T.tk;
+    const int k1 = k0 + T.tk < NZ - 1 ? k0 + T.tk : NZ - 1;   // the last plane: k_gs_last_planes
     const int t = threadIdx.x;
     const uint8_t *__restrict__ st = H.st;
 
