@@ -236,7 +236,8 @@ struct MomArgs {
 
 __device__ inline bool vel_row(int s) { return s == TB_FLUID || s == TB_BUFFER_SOLID; }
 
-template <int R, bool RHS>
+// the node's u, v and w (Q = -1), or one of them
+template <int R, bool RHS, int Q = -1>
 __device__ inline void mom_point(const MomArgs &a, int i, int j, int k) {
     const Dims &d = a.d;
     const GridDev &g = a.g;
@@ -246,7 +247,7 @@ __device__ inline void mom_point(const MomArgs &a, int i, int j, int k) {
     const int wm = a.Wmax;
     const long pidx = (long)k * d.NY + j;
     // u node
-    {
+    if constexpr (Q < 0 || Q == 0) {
         double r = 0.0;
         const int s = a.su[id];
         if (s != TB_BOUNDARY) {
@@ -262,7 +263,7 @@ __device__ inline void mom_point(const MomArgs &a, int i, int j, int k) {
         if constexpr (RHS) st_stream(&a.ru[id], vel_row(s) ? u[id] * a.a_dt - r - a.dpx[id] : 0.0);
     }
     // v node
-    {
+    if constexpr (Q < 0 || Q == 1) {
         double r = 0.0;
         const int s = a.sv[id];
         if (s != TB_BOUNDARY) {
@@ -288,7 +289,7 @@ __device__ inline void mom_point(const MomArgs &a, int i, int j, int k) {
         }
     }
     // w node
-    {
+    if constexpr (Q < 0 || Q == 2) {
         double r = 0.0;
         const int s = a.sw[id];
         if (s != TB_BOUNDARY) {
@@ -471,7 +472,7 @@ static int eno_weights(tb_ctx *c) {
 // ---------------------------------------------------------------------------
 // Second-order ENO of u, v, w and c in one k-marching pass (the workloads'
 // order) on power-of-two uniform grids.  A block owns a 64 x 4 tile of (i, j)
-// columns and walks EF_KC planes of it.  The planes k-1, k, k+1 of u, v, w, c
+// columns and walks up to EF_KC planes of it.  The planes k-1, k, k+1 of u, v, w, c
 // sit in an LDS ring with a two-point x / y halo, so the x and y windows, the
 // z neighbours k +- 1 and the transposes read LDS; each thread keeps k - 2 and
 // k + 2 of its own column in registers.  It computes the nodes at least
@@ -487,7 +488,7 @@ constexpr int EF_THREADS = EF_TX * EF_TY;
 constexpr int EF_STAGE = (EF_PLANE + EF_THREADS - 1) / EF_THREADS;
 
 struct EfTiles {
-    int tx, ty, kc;     // tiles per axis from i, j = 0, k chunks from k = EF_SHELL
+    int tx, ty, kc, ch; // tiles per axis from i, j = 0, k chunks from k = EF_SHELL, planes per chunk
     long n, per_xcd;
 };
 
@@ -495,8 +496,14 @@ static EfTiles make_ef_tiles(const Dims &d, int shell) {
     EfTiles t;
     t.tx = (d.NX - shell + EF_TX - 1) / EF_TX;
     t.ty = (d.NY - shell + EF_TY - 1) / EF_TY;
-    t.kc = (d.NZ - 2 * shell + EF_KC - 1) / EF_KC;
-    t.n = (long)t.tx * t.ty * t.kc;
+    // a block is a chain of ch plane steps behind the staging of its first
+    // three: short chains where the grid has fewer blocks than the 768 that
+    // are resident at once
+    for (t.ch = EF_KC;; t.ch /= 2) {
+        t.kc = (d.NZ - 2 * shell + t.ch - 1) / t.ch;
+        t.n = (long)t.tx * t.ty * t.kc;
+        if (t.ch == 2 || t.n >= 512) break;
+    }
     t.per_xcd = (t.n + NXCD - 1) / NXCD;
     return t;
 }
@@ -539,6 +546,7 @@ struct FusedArgs {
 // the fused kernel's nodes: at least EF_SHELL from every box face, where
 // every window of every quantity lies inside its line's interior span
 constexpr int EF_SHELL = 3;
+constexpr long EF_SHELL_SPLIT = 1L << 18;   // shells of fewer nodes run one quantity per thread
 
 // a value every lane of the wave holds (j is one per wave: a 64-wide row of
 // the 64 x 4 block), moved to scalar registers, bits unchanged
@@ -566,8 +574,8 @@ __global__ void __launch_bounds__(EF_THREADS, 3) k_eno_fused2(FusedArgs A, EfTil
     const int txi = (int)(r1 % T.tx);
     const int kci = (int)(r1 / T.tx);
     const int i0 = txi * EF_TX, j0 = tyi * EF_TY;
-    const int k0 = EF_SHELL + kci * EF_KC;
-    const int k1 = (k0 + EF_KC < d.NZ - EF_SHELL) ? k0 + EF_KC : d.NZ - EF_SHELL;
+    const int k0 = EF_SHELL + kci * T.ch;
+    const int k1 = (k0 + T.ch < d.NZ - EF_SHELL) ? k0 + T.ch : d.NZ - EF_SHELL;
     for (int e = threadIdx.y * EF_TX + threadIdx.x; e < 6 * (k1 - k0 + 1); e += EF_THREADS) {
         const int m = e / 6, f = e - 6 * m, kk = k0 + m;   // kk <= k1 < NZ
         const int tab[4] = {W_WU_Z, W_WV_Z, W_UW_Z, W_VW_Z};
@@ -747,7 +755,11 @@ __global__ void __launch_bounds__(EF_THREADS, 3) k_eno_fused2(FusedArgs A, EfTil
 
 // the nodes within EF_SHELL of a box face (the fused kernel leaves them):
 // each with the per-point code, over the x slabs, then the y slabs between
-// them, then the z slabs between those
+// them, then the z slabs between those.  Small shells take one quantity per
+// row of the grid: the four together are a chain of twelve dependent windows
+// per thread, which few waves do not hide (64x16x16: 30 -> 17 us).  Large ones
+// take all four per thread and share their loads (512x256x128: 151 against
+// 177 us split).
 template <bool RHS>
 __global__ void __launch_bounds__(256) k_eno_shell(MomArgs a, ConcArgs ca, long nx_slab, long ny_slab, long nz_slab) {
     const Dims &d = a.d;
@@ -777,8 +789,17 @@ __global__ void __launch_bounds__(256) k_eno_shell(MomArgs a, ConcArgs ca, long 
     } else {
         return;
     }
-    mom_point<2, RHS>(a, i, j, k);
-    conc_point<2, RHS>(ca, i, j, k);
+    if (gridDim.y == 1) {
+        mom_point<2, RHS>(a, i, j, k);
+        conc_point<2, RHS>(ca, i, j, k);
+        return;
+    }
+    switch (blockIdx.y) {
+    case 0: mom_point<2, RHS, 0>(a, i, j, k); break;
+    case 1: mom_point<2, RHS, 1>(a, i, j, k); break;
+    case 2: mom_point<2, RHS, 2>(a, i, j, k); break;
+    default: conc_point<2, RHS>(ca, i, j, k); break;
+    }
 }
 
 
@@ -938,12 +959,13 @@ static int eno_fused(tb_ctx *c, double rhs_dt, bool store_conv) {
     const long nxs = 2 * H * d.NY * d.NZ, nys = (d.NX - 2 * H) * 2 * H * d.NZ,
                nzs = (d.NX - 2 * H) * (d.NY - 2 * H) * 2 * H;
     const long np = nxs + nys + nzs;
+    const dim3 sgrid((unsigned)((np + 255) / 256), np < EF_SHELL_SPLIT ? 4 : 1);
     if (c->prof_on) tb_prof_begin(c, TB_K_ENO_CONC);
     if (rhs)
-        hipLaunchKernelGGL(k_eno_shell<true>, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->s, m, ca, nxs,
+        hipLaunchKernelGGL(k_eno_shell<true>, sgrid, dim3(256), 0, c->s, m, ca, nxs,
                            nys, nzs);
     else
-        hipLaunchKernelGGL(k_eno_shell<false>, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->s, m, ca, nxs,
+        hipLaunchKernelGGL(k_eno_shell<false>, sgrid, dim3(256), 0, c->s, m, ca, nxs,
                            nys, nzs);
     if (c->prof_on) tb_prof_end(c, TB_K_ENO_CONC);
     TB_LAUNCH_CHECK(c);
