@@ -26,7 +26,10 @@
 //              transposed in (c, n), applied to the output gradient;
 //   backward weights: dW[t*C + c][n] = sum_v X[v + off(t)][c] * dY[v][n]
 //              M = (t, c), N = n, K = voxels.
-// The 1-output-channel head uses plain FP32 kernels.
+// The 1-output-channel head uses plain FP32 kernels, except its weight
+// gradient, which runs through the same matrix-core kernel on the output
+// gradient split exactly into three BF16 parts.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -64,6 +67,7 @@ struct LayerDef {
 };
 static const LayerDef LAYERS[NLAYER] = {{16, 16}, {16, 32}, {32, 32}, {32, 64},
                                         {64, 64}, {96, 32}, {48, 16}, {16, 1}};
+static const int LAYER_LEVEL[NLAYER] = {0, 1, 1, 2, 2, 1, 0, 0};   // halvings of the grid each runs on
 enum { L_IN = 0, L_E1, L_E1B, L_E2, L_E2B, L_D1, L_D0, L_OUT };
 
 // ---------------------------------------------------------------------------
@@ -104,15 +108,6 @@ __device__ inline v4u gather8(const Src &s, int t, int c, int x, int y, int z, i
     int stride;
     long o = src_offset(s, c, xx, yy, zz, nx, ny, base, stride);
     return *(const v4u *)(base + o);
-}
-
-__device__ inline bf16_t gather1(const Src &s, int t, int c, int x, int y, int z, int nx, int ny, int nz) {
-    int xx, yy, zz;
-    if (!tap_neighbour(t, x, y, z, nx, ny, nz, xx, yy, zz)) return 0;
-    const bf16_t *base;
-    int stride;
-    long o = src_offset(s, c, xx, yy, zz, nx, ny, base, stride);
-    return base[o];
 }
 
 __device__ inline void vox_xyz(long v, int nx, int ny, int &x, int &y, int &z) {
@@ -196,102 +191,231 @@ __global__ void __launch_bounds__(256) k_conv_fwd(ConvFwd a) {
 }
 
 // ---------------------------------------------------------------------------
-// backward weights: dW[kk][n] += sum_v X[v + off(t)][c] * dY[v][n],
-// kk = t * cin + c.  Each wave owns KBW 16-row blocks of kk and all n; a
-// workgroup sweeps one voxel range and adds its partial with FP32 atomics.
-constexpr int KBW = 2;
+// backward weights: dW[t][c][n] = sum_v X[v + off(t)][c] * dY[v][n], a
+// product over the voxels.  The matrix cores want eight consecutive voxels of
+// one channel per lane, so both operands are first turned channel-planar
+// (k_planar: rows padded with zeros to 8 voxels).  A wave owns a 16 x 16 block
+// of (c, n), four groups of eight x neighbours, and marches through a chunk
+// of z planes: the nine rows (dy, dz) of X around its dY row stay in
+// registers, three new ones per plane fetched a plane ahead, and the three x
+// shifts are formed on the dY row by funnel shifts with its neighbours' end
+// values, so 27 products (28 with the ones row that sums dY for the bias)
+// follow three 16-byte row loads.  Bound by the matrix cores; the partial sums of a
+// block's four waves meet in LDS, those of the blocks in k_wgrad_sum, in a fixed
+// order.  64^3 voxels, 48 -> 16 channels: 466 -> 24 us (the scalar gathers of
+// the voxel-major form bound it).
+constexpr int WG_TILES = 28;                 // 27 taps and the bias
+constexpr int WG_ELEMS = WG_TILES * 256;
+constexpr long WG_WAVES = 1536;              // waves wanted per launch
 
-struct ConvW {
-    Src s;
-    int nx, ny, nz;
-    long nvox;
-    const bf16_t *gy;   // [nvox][NB*16]
-    float *dW;          // [27 * cin][NB*16]
-    int kblocks;        // 27 * cin / 16
-    long vsplit;        // voxels per workgroup row of the grid (multiple of 32)
+struct WgShape {
+    int nx8;            // groups of 8 voxels per row
+    long plane;         // elements per channel
+    int quads;          // sets of four groups per z plane
+    int zc, nzc;        // planes per chunk, chunks
+    int pairs, nblk;    // (c, n) blocks, workgroups per pair
 };
 
-template <int NB>
-__global__ void __launch_bounds__(256) k_conv_wgrad(ConvW a) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int cin = a.s.Ca + a.s.Cb, cout = NB * 16;
-    const int kb0 = (blockIdx.x * 4 + wave) * KBW;
-    const long vbeg = (long)blockIdx.y * a.vsplit;
-    const long vend = vbeg + a.vsplit < a.nvox ? vbeg + a.vsplit : a.nvox;
-    int tk[KBW], ck[KBW];
-    bool kok[KBW];
-#pragma unroll
-    for (int kb = 0; kb < KBW; kb++) {
-        kok[kb] = kb0 + kb < a.kblocks;
-        const int kk = (kb0 + kb) * 16 + (lane & 15);
-        tk[kb] = kk / cin;
-        ck[kb] = kk - tk[kb] * cin;
-    }
-    v4f acc[KBW][NB];
-#pragma unroll
-    for (int kb = 0; kb < KBW; kb++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) acc[kb][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
-    for (long vs = vbeg; vs < vend; vs += 32) {
-        bf16_t bv[NB][8], av[KBW][8];
+static WgShape wg_shape(int nx, int ny, int nz, int cin, int cout) {
+    WgShape w;
+    w.nx8 = (nx + 7) / 8;
+    w.plane = 8L * w.nx8 * ny * nz;
+    w.quads = (w.nx8 * ny + 3) / 4;
+    w.pairs = (cin / 16) * ((cout + 15) / 16);
+    long chunks = WG_WAVES / ((long)w.quads * w.pairs);
+    if (chunks < 1) chunks = 1;
+    if (chunks > nz) chunks = nz;
+    w.zc = (int)((nz + chunks - 1) / chunks);
+    w.nzc = (nz + w.zc - 1) / w.zc;
+    w.nblk = (int)(((long)w.quads * w.nzc + 3) / 4);
+    return w;
+}
+
+// channel-planar copy [C][nz][ny][8 nx8] of a (concatenated, upsampled)
+// operand, zeros past nx: a thread transposes 8 voxels x 8 channels
+__global__ void __launch_bounds__(256) k_planar(Src s, int nx, int ny, int nz, int nx8, bf16_t *__restrict__ out) {
+    const int C8 = (s.Ca + s.Cb) / 8;
+    const long plane = 8L * nx8 * ny * nz, total = (long)nx8 * ny * nz * C8;
+    for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < total; q += (long)gridDim.x * blockDim.x) {
+        const int c = 8 * (int)(q % C8);
+        const long gidx8 = q / C8;
+        int x8, y, z;
+        vox_xyz(gidx8, nx8, ny, x8, y, z);
+        uint32_t w[8][4];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const long v = vs + 8 * (lane >> 4) + i;
-            const bool ok = v < vend;
-            int x, y, z;
-            vox_xyz(ok ? v : 0, a.nx, a.ny, x, y, z);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) bv[nb][i] = ok ? a.gy[v * cout + nb * 16 + (lane & 15)] : (bf16_t)0;
-#pragma unroll
-            for (int kb = 0; kb < KBW; kb++)
-                av[kb][i] = (ok && kok[kb]) ? gather1(a.s, tk[kb], ck[kb], x, y, z, a.nx, a.ny, a.nz) : (bf16_t)0;
+            v4u v = {0u, 0u, 0u, 0u};
+            const int x = 8 * x8 + i;
+            if (x < nx) {
+                const bf16_t *base;
+                int stride;
+                const long o = src_offset(s, c, x, y, z, nx, ny, base, stride);
+                v = *(const v4u *)(base + o);
+            }
+            w[i][0] = v.x; w[i][1] = v.y; w[i][2] = v.z; w[i][3] = v.w;
         }
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            v4u bw;
-            bw.x = bv[nb][0] | ((uint32_t)bv[nb][1] << 16);
-            bw.y = bv[nb][2] | ((uint32_t)bv[nb][3] << 16);
-            bw.z = bv[nb][4] | ((uint32_t)bv[nb][5] << 16);
-            bw.w = bv[nb][6] | ((uint32_t)bv[nb][7] << 16);
+        for (int e = 0; e < 8; e++) {
+            uint32_t r[4];
 #pragma unroll
-            for (int kb = 0; kb < KBW; kb++) {
-                v4u aw;
-                aw.x = av[kb][0] | ((uint32_t)av[kb][1] << 16);
-                aw.y = av[kb][2] | ((uint32_t)av[kb][3] << 16);
-                aw.z = av[kb][4] | ((uint32_t)av[kb][5] << 16);
-                aw.w = av[kb][6] | ((uint32_t)av[kb][7] << 16);
-                acc[kb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, aw),
-                                                                      __builtin_bit_cast(v8bf, bw), acc[kb][nb], 0, 0, 0);
+            for (int p = 0; p < 4; p++) {
+                const uint32_t a = w[2 * p][e >> 1], b = w[2 * p + 1][e >> 1];
+                r[p] = (e & 1) ? (a >> 16) | (b & 0xffff0000u) : (a & 0xffffu) | (b << 16);
             }
+            *(v4u *)(out + (c + e) * plane + 8 * gidx8) = (v4u){r[0], r[1], r[2], r[3]};
         }
-    }
-#pragma unroll
-    for (int kb = 0; kb < KBW; kb++) {
-        if (!kok[kb]) continue;
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int kk = (kb0 + kb) * 16 + 4 * (lane >> 4) + i;
-                const int n = nb * 16 + (lane & 15);
-                atomicAdd(&a.dW[(long)kk * cout + n], acc[kb][nb][i]);
-            }
     }
 }
 
-// db[n] += sum_v g[v][n]
-__global__ void __launch_bounds__(256) k_bias_grad(const bf16_t *__restrict__ g, long nvox, int cout, float *db) {
-    __shared__ float sh[256];
-    const int n = threadIdx.x % cout, lanes = 256 / cout, r = threadIdx.x / cout;
-    float s = 0.f;
-    for (long v = (long)blockIdx.x * lanes + r; v < nvox; v += (long)gridDim.x * lanes) s += bf2f(g[v * cout + n]);
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x < cout) {
-        float tot = 0.f;
-        for (int q = 0; q < lanes; q++) tot += sh[q * cout + threadIdx.x];
-        atomicAdd(&db[threadIdx.x], tot);
+// an FP32 field as three planar BF16 channels whose sum is exact (8 + 8 + 8
+// significant bits)
+__global__ void __launch_bounds__(256) k_planar_split(const float *__restrict__ g, int nx, int ny, int nz, int nx8,
+                                                      bf16_t *__restrict__ out) {
+    const long total = (long)nx8 * ny * nz, plane = 8 * total;
+    for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < total; q += (long)gridDim.x * blockDim.x) {
+        int x8, y, z;
+        vox_xyz(q, nx8, ny, x8, y, z);
+        uint32_t h[3][4] = {};
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int x = 8 * x8 + i;
+            float v = x < nx ? g[((long)z * ny + y) * nx + x] : 0.f;
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                const bf16_t b = f2bf(v);
+                h[a][i >> 1] |= (uint32_t)b << (16 * (i & 1));
+                v -= bf2f(b);
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < 3; a++) *(v4u *)(out + a * plane + 8 * q) = (v4u){h[a][0], h[a][1], h[a][2], h[a][3]};
     }
+}
+
+struct ConvW {
+    const bf16_t *x, *g;    // channel-planar input and output gradient
+    WgShape w;
+    int ny, nz;
+    int nb;                 // 16-channel blocks of the gradient
+    int gch;                // its channels (the rest of the last block counts as 0)
+    float *part;            // [pairs][nblk][WG_ELEMS]
+};
+
+__device__ inline v4f mfma_bf16(v4u a, v4u b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
+__global__ void __launch_bounds__(256, 2) k_conv_wgrad(ConvW a) {
+    constexpr int STEP = 7;                  // tiles summed over the waves at a time
+    __shared__ float sh[4][STEP * 256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int cb = blockIdx.y / a.nb, nb = blockIdx.y - cb * a.nb;
+    const long wid = (long)blockIdx.x * 4 + wave;
+    const int quad = (int)(wid % a.w.quads), zi = (int)(wid / a.w.quads);
+    const int col = quad * 4 + (lane >> 4);
+    const int x8 = col % a.w.nx8, y = col / a.w.nx8;
+    const int z0 = zi * a.w.zc, z1 = zi < a.w.nzc ? (z0 + a.w.zc < a.nz ? z0 + a.w.zc : a.nz) : z0;
+    const bool ok = y < a.ny;
+    const int n = nb * 16 + (lane & 15);
+    const long row = 8L * a.w.nx8, pl = row * a.ny;
+    const v4u zero = {0u, 0u, 0u, 0u};
+    const bf16_t *X = a.x + (cb * 16 + (lane & 15)) * a.w.plane + y * row + 8 * x8;
+    const bf16_t *G = a.g + (n < a.gch ? n : 0) * a.w.plane + y * row + 8 * x8;
+    const bool gok = ok && n < a.gch, gl = gok && x8 > 0, gr = gok && x8 + 1 < a.w.nx8;
+    const bool ys = ok && y > 0, yn = ok && y + 1 < a.ny;
+    auto xrow = [&](int z, int dy, bool in) -> v4u {
+        return in && z >= 0 && z < a.nz ? *(const v4u *)(X + z * pl + dy * row) : zero;
+    };
+    v4f acc[WG_TILES];
+#pragma unroll
+    for (int t = 0; t < WG_TILES; t++) acc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+    if (z0 < z1) {
+        // X rows (dy = -1, 0, 1) of planes z-1, z, z+1 and, in flight, z+2
+        v4u f0[3], f1[3], f2[3], f3[3];
+        auto fetch = [&](int z, v4u (&f)[3]) {
+            f[0] = xrow(z, -1, ys);
+            f[1] = xrow(z, 0, ok);
+            f[2] = xrow(z, 1, yn);
+        };
+        v4u b, bn;
+        uint32_t l, ln, r, rn;
+        auto fetch_g = [&](int z, v4u &v, uint32_t &lo, uint32_t &hi) {
+            const bf16_t *p = G + z * pl;
+            v = gok && z < z1 ? *(const v4u *)p : zero;
+            lo = gl && z < z1 ? *(const uint32_t *)(p - 2) : 0u;
+            hi = gr && z < z1 ? *(const uint32_t *)(p + 8) : 0u;
+        };
+        fetch(z0 - 1, f0);
+        fetch(z0, f1);
+        fetch(z0 + 1, f2);
+        fetch_g(z0, b, l, r);
+        // row 0 of the bias tile's left operand is 1
+        const uint32_t one = (lane & 15) == 0 ? 0x3f803f80u : 0u;
+        const v4u ones = {one, one, one, one};
+        for (int z = z0; z < z1; z++) {
+            fetch(z + 2, f3);
+            fetch_g(z + 1, bn, ln, rn);
+            const uint32_t m0 = __builtin_amdgcn_alignbit(b.y, b.x, 16), m1 = __builtin_amdgcn_alignbit(b.z, b.y, 16),
+                           m2 = __builtin_amdgcn_alignbit(b.w, b.z, 16);
+            // dY[x + 1], dY[x], dY[x - 1]: the operands of dx = -1, 0, 1
+            const v4u sft[3] = {{m0, m1, m2, (uint32_t)__builtin_amdgcn_alignbit(r, b.w, 16)},
+                                b,
+                                {(uint32_t)__builtin_amdgcn_alignbit(b.x, l, 16), m0, m1, m2}};
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+                for (int dx = 0; dx < 3; dx++) {
+                    acc[dy * 3 + dx] = mfma_bf16(f0[dy], sft[dx], acc[dy * 3 + dx]);
+                    acc[9 + dy * 3 + dx] = mfma_bf16(f1[dy], sft[dx], acc[9 + dy * 3 + dx]);
+                    acc[18 + dy * 3 + dx] = mfma_bf16(f2[dy], sft[dx], acc[18 + dy * 3 + dx]);
+                }
+            acc[27] = mfma_bf16(ones, b, acc[27]);
+#pragma unroll
+            for (int e = 0; e < 3; e++) { f0[e] = f1[e]; f1[e] = f2[e]; f2[e] = f3[e]; }
+            b = bn; l = ln; r = rn;
+        }
+    }
+    float *out = a.part + ((long)blockIdx.y * a.w.nblk + blockIdx.x) * WG_ELEMS;
+#pragma unroll
+    for (int t0 = 0; t0 < WG_TILES; t0 += STEP) {
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < STEP; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                sh[wave][t * 256 + (4 * (lane >> 4) + i) * 16 + (lane & 15)] = acc[t0 + t][i];
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < STEP; t++) {
+            const int e = t * 256 + threadIdx.x;
+            out[t0 * 256 + e] = (sh[0][e] + sh[1][e]) + (sh[2][e] + sh[3][e]);
+        }
+    }
+}
+
+// dW, db += the blocks' partial sums: 64 weights per workgroup, each summed by
+// four threads over a quarter of the blocks and then in order; the head (cout =
+// 1) adds its three split columns
+__global__ void __launch_bounds__(256) k_wgrad_sum(const float *__restrict__ part, int nblk, int nb, int cin, int cout,
+                                                   float *__restrict__ dW, float *__restrict__ db) {
+    __shared__ float sh[4][64];
+    const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
+    const int e = blockIdx.x * 64 + lane;
+    const int pair = e / WG_ELEMS, q = e - pair * WG_ELEMS;
+    const int per = (nblk + 3) / 4, b0 = quarter * per, b1 = b0 + per < nblk ? b0 + per : nblk;
+    const float *p = part + (long)pair * nblk * WG_ELEMS + q;
+    float v = 0.f;
+#pragma unroll 8
+    for (int b = b0; b < b1; b++) v += p[(long)b * WG_ELEMS];
+    sh[quarter][lane] = v;
+    __syncthreads();
+    const int t = q >> 8, r = (q >> 4) & 15, n = (pair % nb) * 16 + (q & 15), c = (pair / nb) * 16 + r;
+    if (quarter || n >= cout || (t == 27 && c > 0)) return;
+    float s = 0.f;
+    for (int k = 0; k < (cout == 1 ? 3 : 1); k++)
+        s += (sh[0][lane + k] + sh[1][lane + k]) + (sh[2][lane + k] + sh[3][lane + k]);
+    if (t == 27) db[n] += s;
+    else dW[((long)t * cin + c) * cout + n] += s;
 }
 
 // ---------------------------------------------------------------------------
@@ -441,30 +565,6 @@ __global__ void __launch_bounds__(256) k_head_bwd_data(const float *__restrict__
         unpack16(y0 + v * 16, m);
         for (int c = 0; c < 16; c++) gy0[v * 16 + c] = f2bf(m[c] > 0.f ? s[c] : 0.f);
     }
-}
-
-// dW[t][c] += sum_v y0[v + off(t)][c] * g_out[v] ; db += sum_v g_out[v]
-// 448 threads: thread q < 432 owns (t = q / 16, c = q % 16), q == 432 the bias
-__global__ void __launch_bounds__(448) k_head_wgrad(const bf16_t *__restrict__ y0, const float *__restrict__ gout,
-                                                    int nx, int ny, int nz, long vsplit, float *dW, float *db) {
-    const int q = threadIdx.x;
-    const long n = (long)nx * ny * nz;
-    const long vb = (long)blockIdx.x * vsplit, ve = vb + vsplit < n ? vb + vsplit : n;
-    const int t = q / 16, c = q % 16;
-    float s = 0.f;
-    for (long v = vb; v < ve; v++) {
-        const float g = gout[v];
-        if (q < 432) {
-            int x, y, z, xx, yy, zz;
-            vox_xyz(v, nx, ny, x, y, z);
-            if (tap_neighbour(t, x, y, z, nx, ny, nz, xx, yy, zz))
-                s += bf2f(y0[(((long)zz * ny + yy) * nx + xx) * 16 + c]) * g;
-        } else if (q == 432) {
-            s += g;
-        }
-    }
-    if (q < 432) atomicAdd(&dW[q], s);
-    else if (q == 432) atomicAdd(db, s);
 }
 
 // loss = mean (out - target)^2 ; g_out = 2 (out - target) / n
@@ -629,6 +729,8 @@ struct Acts {
     float *out = nullptr, *tgt = nullptr, *gout = nullptr;
     bf16_t *gy0 = nullptr, *du0 = nullptr, *gy1 = nullptr, *gx0 = nullptr, *du1 = nullptr, *gx2b = nullptr,
            *gx1b = nullptr, *gx2 = nullptr, *gp1 = nullptr, *gx1 = nullptr, *gp0 = nullptr;
+    bf16_t *plx = nullptr, *plg = nullptr;   // channel-planar operands of one weight gradient
+    float *wpart = nullptr;                  // its per-block partial sums
     std::vector<void *> owned;
 };
 
@@ -724,6 +826,17 @@ static int acts_ensure(tb_net *net, Acts &A, int nx, int ny, int nz, bool train)
             {&A.gp1, A.v2 * 32}, {&A.gx1, A.v1 * 32}, {&A.gp0, A.v1 * 16}};
         for (auto &e : gb)
             if (net_alloc(net, A, (void **)e.p, b2 * e.n)) return -1;
+        long px = 0, pg = 0, pp = 0;
+        for (int l = 0; l < NLAYER; l++) {
+            const int lev = LAYER_LEVEL[l];
+            const WgShape w = wg_shape(nx >> lev, ny >> lev, nz >> lev, LAYERS[l].cin, LAYERS[l].cout);
+            px = std::max(px, w.plane * LAYERS[l].cin);
+            pg = std::max(pg, w.plane * std::max(LAYERS[l].cout, 3));
+            pp = std::max(pp, (long)w.pairs * w.nblk * WG_ELEMS);
+        }
+        if (net_alloc(net, A, (void **)&A.plx, b2 * px) || net_alloc(net, A, (void **)&A.plg, b2 * pg) ||
+            net_alloc(net, A, (void **)&A.wpart, sizeof(float) * pp))
+            return -1;
         if (net_alloc(net, A, (void **)&A.tgt, sizeof(float) * A.v0)) return -1;
         if (net_alloc(net, A, (void **)&A.gout, sizeof(float) * A.v0)) return -1;
     }
@@ -768,35 +881,6 @@ static int conv(tb_net *net, hipStream_t s, const Src &src, int nx, int ny, int 
     return 0;
 }
 
-static int wgrad(tb_net *net, hipStream_t s, const Src &src, int nx, int ny, int nz, const bf16_t *gy, int cout,
-                 float *dW, float *db) {
-    ConvW a;
-    a.s = src;
-    a.nx = nx; a.ny = ny; a.nz = nz;
-    a.nvox = (long)nx * ny * nz;
-    a.gy = gy;
-    a.dW = dW;
-    const int cin = src.Ca + src.Cb;
-    a.kblocks = 27 * cin / 16;
-    const int gx = (a.kblocks + 4 * KBW - 1) / (4 * KBW);
-    long splits = 2048 / gx;
-    if (splits < 1) splits = 1;
-    long maxs = (a.nvox + 255) / 256;
-    if (splits > maxs) splits = maxs;
-    a.vsplit = ((a.nvox + splits - 1) / splits + 31) / 32 * 32;
-    splits = (a.nvox + a.vsplit - 1) / a.vsplit;
-    const dim3 grid((unsigned)gx, (unsigned)splits);
-    switch (cout) {
-        case 16: hipLaunchKernelGGL(k_conv_wgrad<1>, grid, dim3(256), 0, s, a); break;
-        case 32: hipLaunchKernelGGL(k_conv_wgrad<2>, grid, dim3(256), 0, s, a); break;
-        case 64: hipLaunchKernelGGL(k_conv_wgrad<4>, grid, dim3(256), 0, s, a); break;
-        default: net->err = "unsupported channel count"; return -1;
-    }
-    hipLaunchKernelGGL(k_bias_grad, grid1d(a.nvox, 256, 512), dim3(256), 0, s, gy, a.nvox, cout, db);
-    NET_LAUNCH(net);
-    return 0;
-}
-
 static Src src1(const bf16_t *A, int C) {
     Src s;
     s.A = A; s.Ca = C; s.a_up = 0; s.B = nullptr; s.Cb = 0;
@@ -806,6 +890,33 @@ static Src src2(const bf16_t *A, int Ca, const bf16_t *B, int Cb) {
     Src s;
     s.A = A; s.Ca = Ca; s.a_up = 1; s.B = B; s.Cb = Cb;
     return s;
+}
+
+// dW, db of one layer += from its input src and output gradient gy (gout: the
+// head's FP32 one)
+static int wgrad(tb_net *net, hipStream_t s, Acts &A, const Src &src, int nx, int ny, int nz, const bf16_t *gy,
+                 const float *gout, int cout, float *dW, float *db) {
+    const int cin = src.Ca + src.Cb;
+    const WgShape w = wg_shape(nx, ny, nz, cin, cout);
+    const long groups = (long)w.nx8 * ny * nz;
+    hipLaunchKernelGGL(k_planar, grid1d(groups * (cin / 8)), dim3(256), 0, s, src, nx, ny, nz, w.nx8, A.plx);
+    if (gout)
+        hipLaunchKernelGGL(k_planar_split, grid1d(groups), dim3(256), 0, s, gout, nx, ny, nz, w.nx8, A.plg);
+    else
+        hipLaunchKernelGGL(k_planar, grid1d(groups * (cout / 8)), dim3(256), 0, s, src1(gy, cout), nx, ny, nz, w.nx8,
+                           A.plg);
+    ConvW a;
+    a.x = A.plx; a.g = A.plg;
+    a.w = w;
+    a.ny = ny; a.nz = nz;
+    a.nb = (cout + 15) / 16;
+    a.gch = gout ? 3 : cout;
+    a.part = A.wpart;
+    hipLaunchKernelGGL(k_conv_wgrad, dim3((unsigned)w.nblk, (unsigned)w.pairs), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_wgrad_sum, dim3((unsigned)(w.pairs * WG_ELEMS / 64)), dim3(256), 0, s,
+                       (const float *)A.wpart, w.nblk, a.nb, cin, cout, dW, db);
+    NET_LAUNCH(net);
+    return 0;
 }
 
 static int forward(tb_net *net, hipStream_t s, Acts &A) {
@@ -854,50 +965,44 @@ static int backward(tb_net *net, hipStream_t s, Acts &A) {
     // head
     hipLaunchKernelGGL(k_head_bwd_data, grid1d(A.v0), dim3(256), 0, s, (const float *)A.gout,
                        (const float *)(net->w + net->woff[L_OUT]), (const bf16_t *)A.y0, nx, ny, nz, A.gy0);
-    {
-        long vs = (A.v0 + 255) / 256;
-        if (vs < 64) vs = 64;
-        const unsigned nb = (unsigned)((A.v0 + vs - 1) / vs);
-        hipLaunchKernelGGL(k_head_wgrad, dim3(nb), dim3(448), 0, s, (const bf16_t *)A.y0, (const float *)A.gout, nx, ny,
-                           nz, vs, GW(L_OUT), GB(L_OUT));
-    }
+    if (wgrad(net, s, A, src1(A.y0, 16), nx, ny, nz, nullptr, A.gout, 1, GW(L_OUT), GB(L_OUT))) return -1;
     NET_LAUNCH(net);
     // y0 = relu(conv([up(y1), x0]))  (gy0 already masked)
-    if (wgrad(net, s, src2(A.y1, 32, A.x0, 16), nx, ny, nz, A.gy0, 16, GW(L_D0), GB(L_D0))) return -1;
+    if (wgrad(net, s, A, src2(A.y1, 32, A.x0, 16), nx, ny, nz, A.gy0, nullptr, 16, GW(L_D0), GB(L_D0))) return -1;
     if (conv(net, s, src1(A.gy0, 16), nx, ny, nz, net->fragT[L_D0], net->nchT[L_D0], 48, nullptr, 0, nullptr, A.du0)) return -1;
     hipLaunchKernelGGL(k_up_bwd, grid1d(A.v1 * 32), dim3(256), 0, s, (const bf16_t *)A.du0, 32, 16, A.gy1,
                        (const bf16_t *)A.y1, nx, ny, nz);
     hipLaunchKernelGGL(k_take_channels, grid1d(A.v0 * 16), dim3(256), 0, s, (const bf16_t *)A.du0, 48, 32, 16, A.gx0, A.v0);
     NET_LAUNCH(net);
     // y1 = relu(conv([up(x2b), x1b]))
-    if (wgrad(net, s, src2(A.x2b, 64, A.x1b, 32), mx, my, mz, A.gy1, 32, GW(L_D1), GB(L_D1))) return -1;
+    if (wgrad(net, s, A, src2(A.x2b, 64, A.x1b, 32), mx, my, mz, A.gy1, nullptr, 32, GW(L_D1), GB(L_D1))) return -1;
     if (conv(net, s, src1(A.gy1, 32), mx, my, mz, net->fragT[L_D1], net->nchT[L_D1], 96, nullptr, 0, nullptr, A.du1)) return -1;
     hipLaunchKernelGGL(k_up_bwd, grid1d(A.v2 * 64), dim3(256), 0, s, (const bf16_t *)A.du1, 64, 32, A.gx2b,
                        (const bf16_t *)A.x2b, mx, my, mz);
     hipLaunchKernelGGL(k_take_channels, grid1d(A.v1 * 32), dim3(256), 0, s, (const bf16_t *)A.du1, 96, 64, 32, A.gx1b, A.v1);
     NET_LAUNCH(net);
     // x2b = relu(conv(x2))
-    if (wgrad(net, s, src1(A.x2, 64), qx, qy, qz, A.gx2b, 64, GW(L_E2B), GB(L_E2B))) return -1;
+    if (wgrad(net, s, A, src1(A.x2, 64), qx, qy, qz, A.gx2b, nullptr, 64, GW(L_E2B), GB(L_E2B))) return -1;
     if (conv(net, s, src1(A.gx2b, 64), qx, qy, qz, net->fragT[L_E2B], net->nchT[L_E2B], 64, nullptr, 0, A.x2, A.gx2)) return -1;
     // x2 = relu(conv(p1))
-    if (wgrad(net, s, src1(A.p1, 32), qx, qy, qz, A.gx2, 64, GW(L_E2), GB(L_E2))) return -1;
+    if (wgrad(net, s, A, src1(A.p1, 32), qx, qy, qz, A.gx2, nullptr, 64, GW(L_E2), GB(L_E2))) return -1;
     if (conv(net, s, src1(A.gx2, 64), qx, qy, qz, net->fragT[L_E2], net->nchT[L_E2], 32, nullptr, 0, nullptr, A.gp1)) return -1;
     // p1 = pool(x1b): gx1b += up(gp1)/8, then the x1b ReLU mask
     hipLaunchKernelGGL(k_pool_bwd, grid1d(A.v1 * 32), dim3(256), 0, s, (const bf16_t *)A.gp1, A.gx1b,
                        (const bf16_t *)A.x1b, mx, my, mz, 32);
     NET_LAUNCH(net);
     // x1b = relu(conv(x1))
-    if (wgrad(net, s, src1(A.x1, 32), mx, my, mz, A.gx1b, 32, GW(L_E1B), GB(L_E1B))) return -1;
+    if (wgrad(net, s, A, src1(A.x1, 32), mx, my, mz, A.gx1b, nullptr, 32, GW(L_E1B), GB(L_E1B))) return -1;
     if (conv(net, s, src1(A.gx1b, 32), mx, my, mz, net->fragT[L_E1B], net->nchT[L_E1B], 32, nullptr, 0, A.x1, A.gx1)) return -1;
     // x1 = relu(conv(p0))
-    if (wgrad(net, s, src1(A.p0, 16), mx, my, mz, A.gx1, 32, GW(L_E1), GB(L_E1))) return -1;
+    if (wgrad(net, s, A, src1(A.p0, 16), mx, my, mz, A.gx1, nullptr, 32, GW(L_E1), GB(L_E1))) return -1;
     if (conv(net, s, src1(A.gx1, 32), mx, my, mz, net->fragT[L_E1], net->nchT[L_E1], 16, nullptr, 0, nullptr, A.gp0)) return -1;
     // p0 = pool(x0)
     hipLaunchKernelGGL(k_pool_bwd, grid1d(A.v0 * 16), dim3(256), 0, s, (const bf16_t *)A.gp0, A.gx0,
                        (const bf16_t *)A.x0, nx, ny, nz, 16);
     NET_LAUNCH(net);
     // x0 = relu(conv(in))
-    if (wgrad(net, s, src1(A.in16, 16), nx, ny, nz, A.gx0, 16, GW(L_IN), GB(L_IN))) return -1;
+    if (wgrad(net, s, A, src1(A.in16, 16), nx, ny, nz, A.gx0, nullptr, 16, GW(L_IN), GB(L_IN))) return -1;
     return 0;
 }
 
