@@ -99,17 +99,6 @@ __device__ inline long src_offset(const Src &s, int c, int xx, int yy, int zz, i
     return (((long)zz * ny + yy) * nx + xx) * s.Cb + (c - s.Ca);
 }
 
-// 8 consecutive channels (c multiple of 8) of the tap-t neighbour, 0 outside
-__device__ inline v4u gather8(const Src &s, int t, int c, int x, int y, int z, int nx, int ny, int nz) {
-    v4u r = {0u, 0u, 0u, 0u};
-    int xx, yy, zz;
-    if (!tap_neighbour(t, x, y, z, nx, ny, nz, xx, yy, zz)) return r;
-    const bf16_t *base;
-    int stride;
-    long o = src_offset(s, c, xx, yy, zz, nx, ny, base, stride);
-    return *(const v4u *)(base + o);
-}
-
 __device__ inline void vox_xyz(long v, int nx, int ny, int &x, int &y, int &z) {
     x = (int)(v % nx);
     long r = v / nx;
@@ -123,7 +112,6 @@ __device__ inline void vox_xyz(long v, int nx, int ny, int &x, int &y, int &z) {
 struct ConvFwd {
     Src s;
     int nx, ny, nz;
-    long nvox;
     const v4u *frag;        // [nchunks][NB][64 lanes] x 8 bf16
     int nchunks;            // ceil(27 * cin / 32)
     const float *bias;      // [cout] or null
@@ -132,62 +120,152 @@ struct ConvFwd {
     bf16_t *out;            // [nvox][cout]
 };
 
-// 4 waves per workgroup, each wave 32 voxels (two 16-row M blocks) x all
-// NB*16 output channels; K walks (tap, channel) in steps of 32.
-template <int NB>
+// A workgroup computes a box of 16 x TY x TZ voxels, four rows of MT tiles of
+// 16 x neighbours, for NBW blocks of 16 output channels.  The input box with
+// its one-voxel halo sits in LDS, all channels, so that each voxel leaves
+// memory once instead of once per tap; K walks (tap, channel) in steps of 32,
+// a lane's LDS offset per step coming from a table, and a step's weights serve
+// the MT tiles.  The voxel pitch (conv_pitch) spreads eight neighbours over
+// different banks.  The voxel-major form gathered its operand from L1 per tap
+// and was bound there at 7 % of the matrix cores' rate.  Boxes of 16 x 4 x 4
+// (MT = 4) where they fill the chip, else 16 x 2 x 2 with one channel block
+// per workgroup.  128^3 voxels, 48 -> 16 channels: 530 -> 200 us; 16^3, 64 ->
+// 64: 49 -> 14 us.
+constexpr int CONV_LDS = 150 * 1024;
+constexpr int CONV_KMAX = 96;                // steps of 32: at most 27 * 96 / 32 = 81
+
+__host__ __device__ inline int conv_pitch(int cin) {   // bytes per voxel in LDS
+    return 2 * cin + (cin == 16 || cin == 48 ? 0 : 16);
+}
+
+template <int MT, int NBW>
 __global__ void __launch_bounds__(256) k_conv_fwd(ConvFwd a) {
+    constexpr int TY = MT == 4 ? 4 : 2, TZ = TY;
+    constexpr int HX = 18, HY = TY + 2, HZ = TZ + 2;
+    extern __shared__ __align__(16) char tile[];
+    __shared__ int off[CONV_KMAX * 4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long v0 = ((long)blockIdx.x * 4 + wave) * 32;
-    const int cin = a.s.Ca + a.s.Cb;
-    int vx[2], vy[2], vz[2];
-    bool vok[2];
-#pragma unroll
-    for (int mb = 0; mb < 2; mb++) {
-        long v = v0 + mb * 16 + (lane & 15);
-        vok[mb] = v < a.nvox;
-        vox_xyz(vok[mb] ? v : 0, a.nx, a.ny, vx[mb], vy[mb], vz[mb]);
+    const int cin = a.s.Ca + a.s.Cb, c8n = cin / 8, vs = conv_pitch(cin);
+    const unsigned inv = ((1u << 20) + c8n - 1) / c8n;
+    const int tx = (a.nx + 15) / 16, ty = (a.ny + TY - 1) / TY;
+    const int bx = blockIdx.x % tx, br = blockIdx.x / tx;
+    const int x0 = bx * 16, y0 = (br % ty) * TY, z0 = (br / ty) * TZ;
+    const int nb0 = blockIdx.y * NBW, NB = gridDim.y * NBW;
+    for (int e = threadIdx.x; e < a.nchunks * 4; e += 256) {
+        const int kk = (e >> 2) * 32 + 8 * (e & 3);
+        const int t = kk / cin, c = kk - t * cin;
+        off[e] = t < 27 ? (((t / 9) * HY + (t / 3) % 3) * HX + t % 3) * vs + 2 * c : -1;
     }
-    v4f acc[2][NB];
+    for (int e = threadIdx.x; e < HX * HY * HZ * c8n; e += 256) {
+        const int v = (int)((unsigned)e * inv >> 20), c = 8 * (e - v * c8n);   // e / c8n, e < 7776
+        const int hx = v % HX, r = v / HX;
+        const int x = x0 - 1 + hx, y = y0 - 1 + r % HY, z = z0 - 1 + r / HY;
+        v4u w = {0u, 0u, 0u, 0u};
+        if (x >= 0 && y >= 0 && z >= 0 && x < a.nx && y < a.ny && z < a.nz) {
+            const bf16_t *base;
+            int stride;
+            const long o = src_offset(a.s, c, x, y, z, a.nx, a.ny, base, stride);
+            w = *(const v4u *)(base + o);
+        }
+        *(v4u *)(tile + v * vs + 2 * c) = w;
+    }
+    __syncthreads();
+    // this wave's tiles: rows (y, z) of the box, consecutive in y
+    int lb[MT];
 #pragma unroll
-    for (int mb = 0; mb < 2; mb++)
+    for (int m = 0; m < MT; m++) {
+        const int row = wave * MT + m;
+        lb[m] = (((row / TY) * HY + row % TY) * HX + (lane & 15)) * vs;
+    }
+    v4f acc[MT][NBW];
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) acc[mb][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
-    int kk = 8 * (lane >> 4);
-    int t = kk / cin, c = kk - (kk / cin) * cin;
-    for (int ch = 0; ch < a.nchunks; ch++) {
-        v4u av[2];
+    for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int mb = 0; mb < 2; mb++) {
-            av[mb] = (v4u){0u, 0u, 0u, 0u};
-            if (vok[mb]) av[mb] = gather8(a.s, t, c, vx[mb], vy[mb], vz[mb], a.nx, a.ny, a.nz);
+        for (int q = 0; q < NBW; q++) acc[m][q] = (v4f){0.f, 0.f, 0.f, 0.f};
+    const v4u *frag = a.frag + (long)nb0 * 64 + lane;
+    auto products = [&](const v4u (&av)[MT], const v4u (&bw)[NBW]) {
+#pragma unroll
+        for (int q = 0; q < NBW; q++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+                acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, av[m]),
+                                                                    __builtin_bit_cast(v8bf, bw[q]), acc[m][q], 0, 0, 0);
+    };
+    // steps in groups of G: a group's weights are fetched while the one before
+    // it runs (a step alone is shorter than their way from L2)
+    constexpr int G = NBW == 1 ? 4 : 2;
+    const int full = 27 * cin / 32 / G * G;
+    v4u bw[G][NBW], bn[G][NBW];
+    auto fetch = [&](int ch, v4u (&f)[G][NBW]) {
+#pragma unroll
+        for (int j = 0; j < G; j++)
+#pragma unroll
+            for (int q = 0; q < NBW; q++) {
+                const int k = ch + j < a.nchunks ? ch + j : a.nchunks - 1;
+                f[j][q] = frag[((long)k * NB + q) * 64];
+            }
+    };
+    fetch(0, bw);
+    for (int g = 0; g < full; g += G) {
+        fetch(g + G, bn);
+#pragma unroll
+        for (int j = 0; j < G; j++) {
+            const int o = off[(g + j) * 4 + (lane >> 4)];
+            v4u av[MT];
+#pragma unroll
+            for (int m = 0; m < MT; m++) av[m] = *(const v4u *)(tile + lb[m] + o);
+            products(av, bw[j]);
         }
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            const v4u bw = a.frag[((long)ch * NB + nb) * 64 + lane];
+        for (int j = 0; j < G; j++)
 #pragma unroll
-            for (int mb = 0; mb < 2; mb++)
-                acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, av[mb]),
-                                                                      __builtin_bit_cast(v8bf, bw), acc[mb][nb], 0, 0, 0);
-        }
-        c += 32;
-        while (c >= cin) { c -= cin; t++; }
+            for (int q = 0; q < NBW; q++) bw[j][q] = bn[j][q];
     }
-    const int cout = NB * 16;
 #pragma unroll
-    for (int mb = 0; mb < 2; mb++)
+    for (int j = 0; j < G; j++) {
+        if (full + j >= a.nchunks) break;
+        const int o = off[(full + j) * 4 + (lane >> 4)];   // -1 past the last tap
+        v4u av[MT];
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++)
+        for (int m = 0; m < MT; m++) av[m] = o >= 0 ? *(const v4u *)(tile + lb[m] + o) : (v4u){0u, 0u, 0u, 0u};
+        products(av, bw[j]);
+    }
+    // through LDS to 16-byte stores (8 channels of a voxel): [row][x][channel]
+    constexpr int OC = NBW * 16, OP = OC + 8;   // channels, their pitch
+    __syncthreads();
+    bf16_t *ob = reinterpret_cast<bf16_t *>(tile);
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int q = 0; q < NBW; q++) {
+            const float bias = a.bias ? a.bias[(nb0 + q) * 16 + (lane & 15)] : 0.f;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const long v = v0 + mb * 16 + 4 * (lane >> 4) + i;
-                if (v >= a.nvox) continue;
-                const int n = nb * 16 + (lane & 15);
-                float val = acc[mb][nb][i] + (a.bias ? a.bias[n] : 0.f);
+                float val = acc[m][q][i] + bias;
                 if (a.relu) val = val > 0.f ? val : 0.f;
-                const long o = v * cout + n;
-                if (a.mask && !(bf2f(a.mask[o]) > 0.f)) val = 0.f;
-                a.out[o] = f2bf(val);
+                ob[((wave * MT + m) * 16 + 4 * (lane >> 4) + i) * OP + q * 16 + (lane & 15)] = f2bf(val);
             }
+        }
+    __syncthreads();
+    const int cout = NB * 16;
+    for (int e = threadIdx.x; e < 4 * MT * 16 * (OC / 8); e += 256) {
+        const int v = e / (OC / 8), c = 8 * (e - v * (OC / 8));
+        const int row = v / 16, x = x0 + v % 16, y = y0 + row % TY, z = z0 + row / TY;
+        if (x >= a.nx || y >= a.ny || z >= a.nz) continue;
+        v4u w = *(const v4u *)(ob + v * OP + c);
+        const long o = (((long)z * a.ny + y) * a.nx + x) * cout + nb0 * 16 + c;
+        if (a.mask) {
+            const v4u mk = *(const v4u *)(a.mask + o);
+            uint32_t *wp = (uint32_t *)&w;
+            const uint32_t mw[4] = {mk.x, mk.y, mk.z, mk.w};
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                if (!(bf2f((bf16_t)(mw[p] & 0xffff)) > 0.f)) wp[p] &= 0xffff0000u;
+                if (!(bf2f((bf16_t)(mw[p] >> 16)) > 0.f)) wp[p] &= 0xffffu;
+            }
+        }
+        *(v4u *)(a.out + o) = w;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -861,22 +939,27 @@ static int conv(tb_net *net, hipStream_t s, const Src &src, int nx, int ny, int 
     ConvFwd a;
     a.s = src;
     a.nx = nx; a.ny = ny; a.nz = nz;
-    a.nvox = (long)nx * ny * nz;
     a.frag = (const v4u *)frag;
     a.nchunks = nchunks;
     a.bias = bias;
     a.mask = mask;
     a.relu = relu;
     a.out = out;
-    const dim3 grid((unsigned)((a.nvox + 127) / 128));
-    switch (cout) {
-        case 16: hipLaunchKernelGGL(k_conv_fwd<1>, grid, dim3(256), 0, s, a); break;
-        case 32: hipLaunchKernelGGL(k_conv_fwd<2>, grid, dim3(256), 0, s, a); break;
-        case 48: hipLaunchKernelGGL(k_conv_fwd<3>, grid, dim3(256), 0, s, a); break;
-        case 64: hipLaunchKernelGGL(k_conv_fwd<4>, grid, dim3(256), 0, s, a); break;
-        case 96: hipLaunchKernelGGL(k_conv_fwd<6>, grid, dim3(256), 0, s, a); break;
-        default: net->err = "unsupported channel count"; return -1;
-    }
+    const int cin = src.Ca + src.Cb, NB = cout / 16;
+    if (cout % 16 || cin % 16 || nchunks > CONV_KMAX) { net->err = "unsupported channel count"; return -1; }
+    auto boxes = [&](int t) { return (long)((nx + 15) / 16) * ((ny + t - 1) / t) * ((nz + t - 1) / t); };
+    // input box, reused for the output rows of up to 64 channels
+    auto lds = [&](int t) { return std::max(18 * (t + 2) * (t + 2) * conv_pitch(cin), 16 * t * t * 2 * (64 + 8)); };
+    // large boxes where they alone fill the chip's 256 CUs twice and fit LDS
+    const bool big = boxes(4) >= 512 && lds(4) <= CONV_LDS;
+    const int nbw = !big ? 1 : NB % 4 == 0 ? 4 : NB % 3 == 0 ? 3 : NB % 2 == 0 ? 2 : 1;
+    const dim3 grid((unsigned)boxes(big ? 4 : 2), (unsigned)(NB / nbw));
+    const int bytes = lds(big ? 4 : 2);
+    if (!big) hipLaunchKernelGGL((k_conv_fwd<1, 1>), grid, dim3(256), bytes, s, a);
+    else if (nbw == 4) hipLaunchKernelGGL((k_conv_fwd<4, 4>), grid, dim3(256), bytes, s, a);
+    else if (nbw == 3) hipLaunchKernelGGL((k_conv_fwd<4, 3>), grid, dim3(256), bytes, s, a);
+    else if (nbw == 2) hipLaunchKernelGGL((k_conv_fwd<4, 2>), grid, dim3(256), bytes, s, a);
+    else hipLaunchKernelGGL((k_conv_fwd<4, 1>), grid, dim3(256), bytes, s, a);
     NET_LAUNCH(net);
     return 0;
 }
@@ -1043,6 +1126,9 @@ extern "C" tb_net *tb_net_create(uint64_t seed) {
     tb_net *net = new tb_net();
     net->np = param_layout(net->woff, net->boff);
     bool ok = hipStreamCreate(&net->s) == hipSuccess;
+    for (const void *k : {(const void *)k_conv_fwd<1, 1>, (const void *)k_conv_fwd<4, 1>, (const void *)k_conv_fwd<4, 2>,
+                          (const void *)k_conv_fwd<4, 3>, (const void *)k_conv_fwd<4, 4>})
+        ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, CONV_LDS) == hipSuccess;
     ok = ok && hipMalloc((void **)&net->w, sizeof(float) * net->np) == hipSuccess;
     ok = ok && hipMalloc((void **)&net->g, sizeof(float) * net->np) == hipSuccess;
     ok = ok && hipMalloc((void **)&net->m, sizeof(float) * net->np) == hipSuccess;
