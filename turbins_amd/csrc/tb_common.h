@@ -291,7 +291,15 @@ struct ConcSlot {
     double *cin = nullptr, *cout = nullptr, *cout_old = nullptr;
 };
 
-constexpr int XFER_TEAM = 8;   // threads of a large host transfer, each with a pinned slot
+// host transfers (tb_ctx.hip): the pinned slots of a large one's threads,
+// allocated on the first
+constexpr int XFER_TEAM = 8;
+struct HostXfer {
+    char *pin = nullptr;
+    hipEvent_t ev[XFER_TEAM] = {};
+};
+int tb_xfer(HostXfer &x, hipStream_t s, std::string &err, void *host, void *block, size_t bytes, bool up);
+void tb_xfer_free(HostXfer &x);
 
 struct tb_ctx {
     tb_config cfg;
@@ -347,8 +355,7 @@ struct tb_ctx {
     double *hscal = nullptr;     // pinned host mirror of scal
     unsigned long long *hseq = nullptr;   // pinned word the device writes after publishing scalars
     unsigned long long pub_seq = 0;       // last sequence number asked for
-    char *xfer_pin = nullptr;             // pinned slots of the host transfers (allocated on the first large one)
-    hipEvent_t xfer_ev[XFER_TEAM] = {};
+    HostXfer xfer;
 
     // multigrid
     int nlev = 0;

@@ -193,9 +193,7 @@ extern "C" void tb_destroy(tb_ctx *c) {
     hipFree(c->scal);
     if (c->hscal) hipHostFree(c->hscal);
     if (c->hseq) hipHostFree(c->hseq);
-    if (c->xfer_pin) hipHostFree(c->xfer_pin);
-    for (int w = 0; w < XFER_TEAM; w++)
-        if (c->xfer_ev[w]) hipEventDestroy(c->xfer_ev[w]);
+    tb_xfer_free(c->xfer);
     for (int e = 0; e < 2; e++)
         if (c->net_ev[e]) hipEventDestroy(c->net_ev[e]);
     if (c->ev0) hipEventDestroy(c->ev0);
@@ -265,55 +263,69 @@ static int pack_rows(tb_ctx *c, const T *src, int spitch, T *dst, int dpitch) {
 constexpr size_t XFER_CHUNK = 2u << 20;
 constexpr size_t XFER_MIN = 8u << 20;
 
-static int xfer_slots(tb_ctx *c) {
-    if (c->xfer_pin) return 0;
-    for (int w = 0; w < XFER_TEAM; w++)
-        if (!c->xfer_ev[w]) TB_CHECK(c, hipEventCreateWithFlags(&c->xfer_ev[w], hipEventDisableTiming));
-    TB_CHECK(c, hipHostMalloc((void **)&c->xfer_pin, XFER_CHUNK * XFER_TEAM, hipHostMallocDefault));
-    return 0;
-}
-
 // worker w's chunks; returns the first HIP error
-static hipError_t xfer_worker(tb_ctx *c, int w, int dev, char *host, char *block, size_t bytes, bool up) {
+static hipError_t xfer_worker(HostXfer &x, hipStream_t s, int w, int dev, char *host, char *block, size_t bytes,
+                              bool up) {
     hipError_t e = hipSetDevice(dev);
-    char *slot = c->xfer_pin + XFER_CHUNK * w;
+    char *slot = x.pin + XFER_CHUNK * w;
     for (size_t o = XFER_CHUNK * w; e == hipSuccess && o < bytes; o += XFER_CHUNK * XFER_TEAM) {
         const size_t m = bytes - o < XFER_CHUNK ? bytes - o : XFER_CHUNK;
         if (up) memcpy(slot, host + o, m);
-        e = up ? hipMemcpyAsync(block + o, slot, m, hipMemcpyHostToDevice, c->s)
-               : hipMemcpyAsync(slot, block + o, m, hipMemcpyDeviceToHost, c->s);
-        if (e == hipSuccess) e = hipEventRecord(c->xfer_ev[w], c->s);
-        if (e == hipSuccess) e = hipEventSynchronize(c->xfer_ev[w]);   // the slot is used again
+        e = up ? hipMemcpyAsync(block + o, slot, m, hipMemcpyHostToDevice, s)
+               : hipMemcpyAsync(slot, block + o, m, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(x.ev[w], s);
+        if (e == hipSuccess) e = hipEventSynchronize(x.ev[w]);   // the slot is used again
         if (e == hipSuccess && !up) memcpy(host + o, slot, m);
     }
     return e;
 }
 
-static int xfer(tb_ctx *c, void *host, void *block, size_t bytes, bool up) {
+int tb_xfer(HostXfer &x, hipStream_t s, std::string &err, void *host, void *block, size_t bytes, bool up) {
+    hipError_t e[XFER_TEAM] = {};
     if (bytes < XFER_MIN) {
-        TB_CHECK(c, up ? hipMemcpyAsync(block, host, bytes, hipMemcpyHostToDevice, c->s)
-                       : hipMemcpyAsync(host, block, bytes, hipMemcpyDeviceToHost, c->s));
-        if (!up) TB_CHECK(c, hipStreamSynchronize(c->s));
-        return 0;
-    }
-    if (xfer_slots(c)) return -1;
-    int dev = 0;
-    TB_CHECK(c, hipGetDevice(&dev));
-    hipError_t err[XFER_TEAM];
-    std::thread team[XFER_TEAM];
-    for (int w = 0; w < XFER_TEAM; w++) {
-        auto work = [=, &err] { err[w] = xfer_worker(c, w, dev, (char *)host, (char *)block, bytes, up); };
-        try {
-            if (w + 1 < XFER_TEAM) team[w] = std::thread(work);
-            else work();
-        } catch (const std::exception &) {
-            work();   // no thread to be had: this one moves the chunks
+        e[0] = up ? hipMemcpyAsync(block, host, bytes, hipMemcpyHostToDevice, s)
+                  : hipMemcpyAsync(host, block, bytes, hipMemcpyDeviceToHost, s);
+        if (e[0] == hipSuccess && !up) e[0] = hipStreamSynchronize(s);
+    } else {
+        int dev = 0;
+        for (int w = 0; w < XFER_TEAM && e[0] == hipSuccess; w++)
+            if (!x.ev[w]) e[0] = hipEventCreateWithFlags(&x.ev[w], hipEventDisableTiming);
+        if (e[0] == hipSuccess && !x.pin)
+            e[0] = hipHostMalloc((void **)&x.pin, XFER_CHUNK * XFER_TEAM, hipHostMallocDefault);
+        if (e[0] == hipSuccess) e[0] = hipGetDevice(&dev);
+        std::thread team[XFER_TEAM];
+        const int n = e[0] == hipSuccess ? XFER_TEAM : 0;   // e[0] is worker 0's from here on
+        for (int w = 0; w < n; w++) {
+            auto work = [&x, &e, s, w, dev, host, block, bytes, up] {
+                e[w] = xfer_worker(x, s, w, dev, (char *)host, (char *)block, bytes, up);
+            };
+            try {
+                if (w + 1 < XFER_TEAM) team[w] = std::thread(work);
+                else work();
+            } catch (const std::exception &) {
+                work();   // no thread to be had: this one moves the chunks
+            }
         }
+        for (std::thread &t : team)
+            if (t.joinable()) t.join();
     }
-    for (std::thread &t : team)
-        if (t.joinable()) t.join();
-    for (hipError_t e : err) TB_CHECK(c, e);
+    for (hipError_t v : e)
+        if (v != hipSuccess) {
+            err = std::string("host transfer: ") + hipGetErrorString(v);
+            return -1;
+        }
     return 0;
+}
+
+void tb_xfer_free(HostXfer &x) {
+    if (x.pin) hipHostFree(x.pin);
+    for (hipEvent_t &e : x.ev)
+        if (e) hipEventDestroy(e);
+    x = HostXfer();
+}
+
+static int xfer(tb_ctx *c, void *host, void *block, size_t bytes, bool up) {
+    return tb_xfer(c->xfer, c->s, c->err, host, block, bytes, up);
 }
 
 extern "C" int tb_upload_field(tb_ctx *c, int f, const double *host) {

@@ -825,6 +825,7 @@ struct tb_net {
     double *dscal = nullptr;    // device scalars
     double *hscal = nullptr;    // pinned host mirror
     Acts inf, trn;
+    HostXfer xfer;
     // snapshot store
     int cap = 0, count = 0, sx = 0, sy = 0, sz = 0;
     bf16_t *s_in = nullptr;
@@ -1164,6 +1165,7 @@ extern "C" void tb_net_destroy(tb_net *net) {
     if (net->s) hipStreamSynchronize(net->s);
     acts_free(net->inf);
     acts_free(net->trn);
+    tb_xfer_free(net->xfer);
     hipFree(net->w); hipFree(net->g); hipFree(net->m); hipFree(net->v);
     hipFree(net->red); hipFree(net->dscal);
     if (net->hscal) hipHostFree(net->hscal);
@@ -1198,17 +1200,11 @@ extern "C" int tb_net_forward(tb_net *net, const float *in3, int nx, int ny, int
     if (!net || !in3 || !out) return -1;
     if (acts_ensure(net, net->trn, nx, ny, nz, true)) return -1;
     Acts &A = net->trn;
-    float *d3 = nullptr;
-    NET_CHECK(net, hipMalloc((void **)&d3, sizeof(float) * 3 * A.v0));
-    int rc = 0;
-    if (hipMemcpyAsync(d3, in3, sizeof(float) * 3 * A.v0, hipMemcpyHostToDevice, net->s) != hipSuccess) rc = -1;
-    if (!rc) hipLaunchKernelGGL(k_expand3, grid1d(A.v0), dim3(256), 0, net->s, (const float *)d3, A.v0, A.in16);
-    if (!rc) rc = forward(net, net->s, A);
-    if (!rc && hipMemcpyAsync(out, A.out, sizeof(float) * A.v0, hipMemcpyDeviceToHost, net->s) != hipSuccess) rc = -1;
-    if (hipStreamSynchronize(net->s) != hipSuccess) rc = -1;
-    hipFree(d3);
-    if (rc && net->err.empty()) net->err = "tb_net_forward failed";
-    return rc;
+    float *d3 = (float *)A.plx;   // at least 16 BF16 channels per voxel, free until a backward pass
+    if (tb_xfer(net->xfer, net->s, net->err, const_cast<float *>(in3), d3, sizeof(float) * 3 * A.v0, true)) return -1;
+    hipLaunchKernelGGL(k_expand3, grid1d(A.v0), dim3(256), 0, net->s, (const float *)d3, A.v0, A.in16);
+    if (forward(net, net->s, A)) return -1;
+    return tb_xfer(net->xfer, net->s, net->err, out, A.out, sizeof(float) * A.v0, false);
 }
 
 // loss and full parameter gradient for host input / target (tests)
@@ -1217,22 +1213,14 @@ extern "C" int tb_net_gradient(tb_net *net, const float *in3, const float *targe
     if (!net || !in3 || !target || !grad) return -1;
     if (acts_ensure(net, net->trn, nx, ny, nz, true)) return -1;
     Acts &A = net->trn;
-    float *d3 = nullptr;
-    NET_CHECK(net, hipMalloc((void **)&d3, sizeof(float) * 3 * A.v0));
-    int rc = 0;
-    if (hipMemcpyAsync(d3, in3, sizeof(float) * 3 * A.v0, hipMemcpyHostToDevice, net->s) != hipSuccess ||
-        hipMemcpyAsync(A.tgt, target, sizeof(float) * A.v0, hipMemcpyHostToDevice, net->s) != hipSuccess ||
-        hipMemsetAsync(net->g, 0, sizeof(float) * net->np, net->s) != hipSuccess)
-        rc = -1;
-    if (!rc) hipLaunchKernelGGL(k_expand3, grid1d(A.v0), dim3(256), 0, net->s, (const float *)d3, A.v0, A.in16);
-    if (!rc) rc = forward(net, net->s, A);
-    if (!rc) rc = loss_eval(net, net->s, A, true, loss);
-    if (!rc) rc = backward(net, net->s, A);
-    if (!rc && hipMemcpyAsync(grad, net->g, sizeof(float) * net->np, hipMemcpyDeviceToHost, net->s) != hipSuccess) rc = -1;
-    if (hipStreamSynchronize(net->s) != hipSuccess) rc = -1;
-    hipFree(d3);
-    if (rc && net->err.empty()) net->err = "tb_net_gradient failed";
-    return rc;
+    float *d3 = (float *)A.plx;
+    if (tb_xfer(net->xfer, net->s, net->err, const_cast<float *>(in3), d3, sizeof(float) * 3 * A.v0, true) ||
+        tb_xfer(net->xfer, net->s, net->err, const_cast<float *>(target), A.tgt, sizeof(float) * A.v0, true))
+        return -1;
+    NET_CHECK(net, hipMemsetAsync(net->g, 0, sizeof(float) * net->np, net->s));
+    hipLaunchKernelGGL(k_expand3, grid1d(A.v0), dim3(256), 0, net->s, (const float *)d3, A.v0, A.in16);
+    if (forward(net, net->s, A) || loss_eval(net, net->s, A, true, loss) || backward(net, net->s, A)) return -1;
+    return tb_xfer(net->xfer, net->s, net->err, grad, net->g, sizeof(float) * net->np, false);
 }
 
 // snapshot store ------------------------------------------------------------
