@@ -458,6 +458,7 @@ enum {
 int tb_geometry_run(tb_ctx *c, const double *h_xz);
 int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0);
 int tb_read_scalars(tb_ctx *c, int first, int count);
+int tb_wait_published(tb_ctx *c, unsigned long long want);
 int tb_sync(tb_ctx *c);
 int tb_dot(tb_ctx *c, const double *a, const double *b, int slot);
 int tb_mg_build(tb_ctx *c);

@@ -482,16 +482,13 @@ __global__ void k_publish(const double *__restrict__ scal, int first, int count,
     *(volatile unsigned long long *)hseq = seq;
 }
 
-int tb_read_scalars(tb_ctx *c, int first, int count) {
-    const unsigned long long want = ++c->pub_seq;
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, c->s, (const double *)c->scal, first, count, c->hscal, c->hseq,
-                       want);
-    TB_LAUNCH_CHECK(c);
+// spin until the device has published sequence number want (or a later one)
+int tb_wait_published(tb_ctx *c, unsigned long long want) {
     const auto t0 = std::chrono::steady_clock::now();
-    for (unsigned n = 1; __atomic_load_n(c->hseq, __ATOMIC_ACQUIRE) != want; n++) {
+    for (unsigned n = 1; __atomic_load_n(c->hseq, __ATOMIC_ACQUIRE) < want; n++) {
         if ((n & 4095) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1)) {
             TB_CHECK(c, hipStreamSynchronize(c->s));
-            if (__atomic_load_n(c->hseq, __ATOMIC_ACQUIRE) != want) {
+            if (__atomic_load_n(c->hseq, __ATOMIC_ACQUIRE) < want) {
                 c->err = "scalar read-back: the device did not publish";
                 return -1;
             }
@@ -500,6 +497,14 @@ int tb_read_scalars(tb_ctx *c, int first, int count) {
         __builtin_ia32_pause();
     }
     return 0;
+}
+
+int tb_read_scalars(tb_ctx *c, int first, int count) {
+    const unsigned long long want = ++c->pub_seq;
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, c->s, (const double *)c->scal, first, count, c->hscal, c->hseq,
+                       want);
+    TB_LAUNCH_CHECK(c);
+    return tb_wait_published(c, want);
 }
 
 // wait until the context's stream has drained (spin, as tb_read_scalars)
