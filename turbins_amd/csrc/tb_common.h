@@ -338,6 +338,7 @@ struct tb_ctx {
 
     // immersed boundary: node tables and the scaled matrix rows
     int nib[4] = {0, 0, 0, 0};
+    int ib_cap[4] = {0, 0, 0, 0};   // nodes the tables hold
     tb_ib_node *ib[4] = {};
     long *ib_row[4] = {};
     int *ib_cnt[4] = {};

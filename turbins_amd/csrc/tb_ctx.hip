@@ -161,7 +161,7 @@ extern "C" tb_ctx *tb_create(const tb_config *cfg) {
 static void free_ib(tb_ctx *c, int q) {
     hipFree(c->ib[q]); hipFree(c->ib_row[q]); hipFree(c->ib_cnt[q]); hipFree(c->ib_col[q]); hipFree(c->ib_val[q]);
     c->ib[q] = nullptr; c->ib_row[q] = nullptr; c->ib_cnt[q] = nullptr; c->ib_col[q] = nullptr; c->ib_val[q] = nullptr;
-    c->nib[q] = 0;
+    c->nib[q] = c->ib_cap[q] = 0;
 }
 
 extern "C" void tb_destroy(tb_ctx *c) {

@@ -15,6 +15,11 @@ __device__ inline double dmin(double a, double b) { return a > b ? b : a; }
 __device__ inline int imax(int a, int b) { return a < b ? b : a; }
 __device__ inline int imin(int a, int b) { return a > b ? b : a; }
 
+__global__ void k_fill(double *p, double v, long n) {
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i < n) p[i] = v;
+}
+
 // Surface_initialize (Surface.c:96-192): sdf guess y - interface(x, z)
 __global__ void k_sdf_guess(Dims d, GridDev g, const double *__restrict__ h, double offset,
                             double *__restrict__ p0, double *__restrict__ p, Tiles t) {
@@ -26,15 +31,69 @@ __global__ void k_sdf_guess(Dims d, GridDev g, const double *__restrict__ h, dou
     p[id] = v;
 }
 
-__device__ inline double ls_godunov(const Dims &d, const GridDev &g, const double *__restrict__ p0,
-                                    const double *__restrict__ p, double a_dEta, double a_dXi, double a_dPhi, double dt,
-                                    int scaled_guard, int i, int j, int k) {
-    int NI = d.NX - 1, NJ = d.NY - 1, NK = d.NZ - 1;   // the node lies in [0,NI) x [0,NJ) x [0,NK)
+// What the pseudo-time steps need of the initial field p0, formed once: the
+// smoothed sign pp0 / sqrt(pp0^2 + dx^2) (Levelset.c:267-494), or next to the
+// interface -1, 0 or 1 moved up by LS_NEAR, and there the Russo-Smereka distance
+constexpr double LS_NEAR = 4.0;
+
+__global__ void __launch_bounds__(256) k_ls_setup(Dims d, GridDev g, const double *__restrict__ p0, int scaled_guard,
+                                                  double *__restrict__ sgn, double *__restrict__ dist, Tiles t) {
+    int i, j, k;
+    if (!tile_point(t, i, j, k)) return;
+    int NI = d.NX - 1, NJ = d.NY - 1, NK = d.NZ - 1;
+    if (i >= NI || j >= NJ || k >= NK) return;
     long id = gidx(d, i, j, k);
     double dx = g.dxc[i];
     double pp0 = p0[id];
     double sign_0 = pp0 / sqrt(pp0 * pp0 + dx * dx);
+    int ix;
+    ix = imin(i + 1, NI - 1); double p_e = p0[gidx(d, ix, j, k)]; double DeltaX = g.xc[ix];
+    ix = imin(j + 1, NJ - 1); double p_n = p0[gidx(d, i, ix, k)]; double DeltaY = g.yc[ix];
+    ix = imin(k + 1, NK - 1); double p_f = p0[gidx(d, i, j, ix)]; double DeltaZ = g.zc[ix];
+    ix = imax(i - 1, 0); double p_w = p0[gidx(d, ix, j, k)]; DeltaX -= g.xc[ix];
+    ix = imax(j - 1, 0); double p_s = p0[gidx(d, i, ix, k)]; DeltaY -= g.yc[ix];
+    ix = imax(k - 1, 0); double p_b = p0[gidx(d, i, j, ix)]; DeltaZ -= g.zc[ix];
+    double p_p = pp0, D = 0.0;
+    bool near = false;
+    if (((p_p * p_w) < 0.0) || ((p_p * p_e) < 0.0) || ((p_p * p_n) < 0.0) || ((p_p * p_s) < 0.0) ||
+        ((p_p * p_b) < 0.0) || ((p_p * p_f) < 0.0)) {
+        const double tol = 0.01;
+        // scaled guard: min(tol, 1.5 d_c) keeps interior central differences
+        // on fine grids; equal to the absolute tol when every d_c >= tol/1.5
+        double gx = tol, gy = tol, gz = tol;
+        if (scaled_guard) {
+            gx = dmin(tol, 1.5 * g.dxc[i]);
+            gy = dmin(tol, 1.5 * g.dyc[j]);
+            gz = dmin(tol, 1.5 * g.dzc[k]);
+        }
+        double Dphi_dx = (fabs(DeltaX) > gx) ? (p_e - p_w) / DeltaX : 0.0;
+        double Dphi_dy = (fabs(DeltaY) > gy) ? (p_n - p_s) / DeltaY : 0.0;
+        double Dphi_dz = (fabs(DeltaZ) > gz) ? (p_f - p_b) / DeltaZ : 0.0;
+        double Dt = sqrt(Dphi_dx * Dphi_dx + Dphi_dy * Dphi_dy + Dphi_dz * Dphi_dz);
+        if (Dt < tol) Dt = tol;
+        near = true;
+        D = p_p / Dt;
+        if (fabs(sign_0) < 1.0e-8) sign_0 = 0.0;
+        else if (sign_0 > 0.0) sign_0 = 1.0;
+        else sign_0 = -1.0;
+    }
+    sgn[id] = near ? sign_0 + LS_NEAR : sign_0;
+    dist[id] = D;
+}
+
+__device__ inline double ls_godunov(const Dims &d, const GridDev &g, const double *__restrict__ sgn,
+                                    const double *__restrict__ dist, const double *__restrict__ p, double a_dEta, double a_dXi, double a_dPhi,
+                                    double dt, int i, int j, int k) {
+    int NI = d.NX - 1, NJ = d.NY - 1, NK = d.NZ - 1;   // the node lies in [0,NI) x [0,NJ) x [0,NK)
+    long id = gidx(d, i, j, k);
+    double sign_0 = sgn[id];
     const double pc = p[id];
+    if (sign_0 > LS_NEAR - 2.0) {   // next to the interface
+        double ddx = g.dxc[i], ddy = g.dyc[j], ddz = g.dzc[k];
+        double Ds = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
+        const double H = ((sign_0 - LS_NEAR) * fabs(pc) - dist[id]) / Ds;
+        return pc + -H * dt;
+    }
     const double pe = p[id + 1], pn = p[id + d.px], pf = p[id + d.plane];
     const double pw = p[id - (i > 0 ? 1 : 0)], ps = p[id - (j > 0 ? d.px : 0)], pb = p[id - (k > 0 ? d.plane : 0)];
     // differences towards i - 1 (at i = 0 the one towards i + 1) and i + 1
@@ -58,38 +117,6 @@ __device__ inline double ls_godunov(const Dims &d, const GridDev &g, const doubl
         tx = dmax(am * am, bp * bp); ty = dmax(cm * cm, dp * dp); tz = dmax(em * em, fp * fp);
     }
     double H = sign_0 * (sqrt(tx + ty + tz) - 1.0);
-    int ix;
-    ix = imin(i + 1, NI - 1); double p_e = p0[gidx(d, ix, j, k)]; double DeltaX = g.xc[ix];
-    ix = imin(j + 1, NJ - 1); double p_n = p0[gidx(d, i, ix, k)]; double DeltaY = g.yc[ix];
-    ix = imin(k + 1, NK - 1); double p_f = p0[gidx(d, i, j, ix)]; double DeltaZ = g.zc[ix];
-    ix = imax(i - 1, 0); double p_w = p0[gidx(d, ix, j, k)]; DeltaX -= g.xc[ix];
-    ix = imax(j - 1, 0); double p_s = p0[gidx(d, i, ix, k)]; DeltaY -= g.yc[ix];
-    ix = imax(k - 1, 0); double p_b = p0[gidx(d, i, j, ix)]; DeltaZ -= g.zc[ix];
-    double p_p = pp0;
-    if (((p_p * p_w) < 0.0) || ((p_p * p_e) < 0.0) || ((p_p * p_n) < 0.0) || ((p_p * p_s) < 0.0) ||
-        ((p_p * p_b) < 0.0) || ((p_p * p_f) < 0.0)) {
-        const double tol = 0.01;
-        // scaled guard: min(tol, 1.5 d_c) keeps interior central differences
-        // on fine grids; equal to the absolute tol when every d_c >= tol/1.5
-        double gx = tol, gy = tol, gz = tol;
-        if (scaled_guard) {
-            gx = dmin(tol, 1.5 * g.dxc[i]);
-            gy = dmin(tol, 1.5 * g.dyc[j]);
-            gz = dmin(tol, 1.5 * g.dzc[k]);
-        }
-        double Dphi_dx = (fabs(DeltaX) > gx) ? (p_e - p_w) / DeltaX : 0.0;
-        double Dphi_dy = (fabs(DeltaY) > gy) ? (p_n - p_s) / DeltaY : 0.0;
-        double Dphi_dz = (fabs(DeltaZ) > gz) ? (p_f - p_b) / DeltaZ : 0.0;
-        double Dt = sqrt(Dphi_dx * Dphi_dx + Dphi_dy * Dphi_dy + Dphi_dz * Dphi_dz);
-        if (Dt < tol) Dt = tol;
-        double D = p_p / Dt;
-        if (fabs(sign_0) < 1.0e-8) sign_0 = 0.0;
-        else if (sign_0 > 0.0) sign_0 = 1.0;
-        else sign_0 = -1.0;
-        double ddx = g.dxc[i], ddy = g.dyc[j], ddz = g.dzc[k];
-        double Ds = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-        H = (sign_0 * fabs(pc) - D) / Ds;
-    }
     return pc + -H * dt;
 }
 
@@ -101,12 +128,12 @@ __device__ inline double ls_godunov(const Dims &d, const GridDev &g, const doubl
 // last plane per axis keeps its value.  The one-sided differences are formed
 // where they are used, with their own expressions, so the values are those of
 // stored derivative arrays; those arrays, the old copy and the three
-// launches they took are gone.  Bound by memory: p, p0 and q once (24 B per
-// point) against 112 B; 470 -> 99 us a step at 512x256x128.
-__global__ void __launch_bounds__(256) k_ls_step(Dims d, GridDev g, const double *__restrict__ p0,
-                                                 const double *__restrict__ p, double *__restrict__ q, double a_dEta,
-                                                 double a_dXi, double a_dPhi, double dt, int scaled_guard, int first,
-                                                 double *part, Tiles t) {
+// launches they took are gone.  Bound by memory: p, the sign and q once (24 B per
+// point) against 112 B.
+__global__ void __launch_bounds__(256) k_ls_step(Dims d, GridDev g, const double *__restrict__ sgn,
+                                                 const double *__restrict__ dist, const double *__restrict__ p,
+                                                 double *__restrict__ q, double a_dEta, double a_dXi, double a_dPhi,
+                                                 double dt, int first, double *part, Tiles t) {
     __shared__ double sh[16];
     double v[1] = {0.0};
     int i, j, k;
@@ -115,7 +142,7 @@ __global__ void __launch_bounds__(256) k_ls_step(Dims d, GridDev g, const double
         const double old = p[id];
         double now = old;
         if (i < d.NX - 1 && j < d.NY - 1 && k < d.NZ - 1)
-            now = ls_godunov(d, g, p0, p, a_dEta, a_dXi, a_dPhi, dt, scaled_guard, i, j, k);
+            now = ls_godunov(d, g, sgn, dist, p, a_dEta, a_dXi, a_dPhi, dt, i, j, k);
         q[id] = now;
         const double error = fabs(now - (first ? 0.0 : old));
         v[0] = error * error * g.dxc[i] * g.dyc[j] * g.dzc[k];
@@ -472,6 +499,35 @@ __global__ void k_ib_nodes(Dims d, GridDev g, int q, QCoords qc, const double *_
     nodes[a] = nd;
 }
 
+// IMMERSED nodes per (j, k) row, one wave per row
+__global__ void __launch_bounds__(256) k_ib_count(Dims d, const uint8_t *__restrict__ st, int *__restrict__ cnt) {
+    const long r = blockIdx.x * 4L + threadIdx.y;
+    if (r >= (long)d.NY * d.NZ) return;
+    int n = 0;
+    for (int i = threadIdx.x; i < d.NX; i += 64) n += st[r * d.px + i] == TB_IMMERSED;
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_down(n, o, 64);
+    if (threadIdx.x == 0) cnt[r] = n;
+}
+
+// their indices, a row's nodes from its first entry on
+__global__ void __launch_bounds__(256) k_ib_list(Dims d, const uint8_t *__restrict__ st, const int *__restrict__ first,
+                                                 tb_ib_node *__restrict__ nodes) {
+    const long r = blockIdx.x * 4L + threadIdx.y;
+    if (r >= (long)d.NY * d.NZ) return;
+    int at = first[r];
+    const int j = (int)(r % d.NY), k = (int)(r / d.NY);
+    for (int i0 = 0; i0 < d.NX; i0 += 64) {
+        const int i = i0 + threadIdx.x;
+        const bool im = i < d.NX && st[r * d.px + i] == TB_IMMERSED;
+        const unsigned long long m = __ballot(im);
+        if (im) {
+            tb_ib_node &nd = nodes[at + __popcll(m & ((1ull << threadIdx.x) - 1))];
+            nd.i = i; nd.j = j; nd.k = k;
+        }
+        at += __popcll(m);
+    }
+}
+
 // Matrix row of an IMMERSED node (Velocity.c:718-762, Conc.c:668-708):
 // self coefficient 1 + sum of self weights, other weights with
 // |coef| >= LSYS_DROP_TOLERANCE, all scaled by ap_solid; columns sorted.
@@ -530,8 +586,12 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
     c->reinit_its = 0;
     double *sdf_c = c->f[TB_F_SDF_C];
     if (c->has_geometry) {
-        double *dh = nullptr, *p0 = c->kv[0], *alt = c->kv[4];
-        TB_CHECK(c, hipMalloc((void **)&dh, sizeof(double) * (size_t)d.NX * d.NZ));
+        // the Krylov vectors are free here; kv[4] alone may be written outside
+        // the box points (the others' row padding stays 0): it holds the
+        // heights first, then the second iterate
+        double *p0 = c->kv[0], *dh = c->kv[4], *sgn = c->kv[2], *dist = c->kv[3], *alt = c->kv[4], *part = c->red;
+        const bool own_part = all.per_xcd * NXCD > (long)RED_SLOTS * RED_MAX_BLOCKS;
+        if (own_part) TB_CHECK(c, hipMalloc((void **)&part, sizeof(double) * (size_t)(all.per_xcd * NXCD)));
         TB_CHECK(c, hipMemcpyAsync(dh, h_xz, sizeof(double) * (size_t)d.NX * d.NZ, hipMemcpyHostToDevice, c->s));
         double offset = c->cfg.bottom_offset ? c->hgrid[13][0] * 2.001 : 0.0;   // Grid.c:913
         hipLaunchKernelGGL(k_sdf_guess, tiles_grid(all), tiles_block(), 0, c->s, d, c->g, dh, offset, p0, sdf_c, all);
@@ -544,8 +604,9 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
         double dm = dmin_[0] > dmin_[1] ? dmin_[1] : dmin_[0];
         dm = dm > dmin_[2] ? dmin_[2] : dm;
         double dt = 0.5 * dm;
-        double *part = nullptr;
-        TB_CHECK(c, hipMalloc((void **)&part, sizeof(double) * (size_t)(all.per_xcd * NXCD)));
+        hipLaunchKernelGGL(k_ls_setup, tiles_grid(all), tiles_block(), 0, c->s, d, c->g, (const double *)p0,
+                           c->cfg.reinit_guard == TB_REINIT_SCALED ? 1 : 0, sgn, dist, all);
+        TB_LAUNCH_CHECK(c);
         const int max_iterations = 500;   // Surface.c:199
         // step n goes from cur[n & 1] to the other buffer; step n + 1 is
         // queued before step n's norm is read, so the GPU does not wait for
@@ -553,10 +614,9 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
         double *cur[2] = {sdf_c, alt};
         const unsigned long long seq0 = c->pub_seq;
         auto queue = [&](int n) -> int {
-            hipLaunchKernelGGL(k_ls_step, tiles_grid(all), tiles_block(), 0, c->s, d, c->g, (const double *)p0,
-                               (const double *)cur[n & 1], cur[(n + 1) & 1], 1.0 / c->dEta, 1.0 / c->dXi,
-                               1.0 / c->dPhi, dt, c->cfg.reinit_guard == TB_REINIT_SCALED ? 1 : 0, n == 0 ? 1 : 0,
-                               part, all);
+            hipLaunchKernelGGL(k_ls_step, tiles_grid(all), tiles_block(), 0, c->s, d, c->g, (const double *)sgn,
+                               (const double *)dist, (const double *)cur[n & 1], cur[(n + 1) & 1], 1.0 / c->dEta,
+                               1.0 / c->dXi, 1.0 / c->dPhi, dt, n == 0 ? 1 : 0, part, all);
             hipLaunchKernelGGL(k_ls_sum, dim3(1), dim3(1024), 0, c->s, (const double *)part, all.per_xcd * NXCD,
                                c->hscal + S_TMP0 + (n & 1), c->hseq, ++c->pub_seq);
             TB_LAUNCH_CHECK(c);
@@ -582,19 +642,18 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
         hipLaunchKernelGGL(k_q_sdf, tiles_grid(all), tiles_block(), 0, c->s, d, c->g, sdf_c, c->f[TB_F_SDF_U],
                            c->f[TB_F_SDF_V], c->f[TB_F_SDF_W], all);
         TB_LAUNCH_CHECK(c);
-        TB_CHECK(c, hipStreamSynchronize(c->s));
-        hipFree(part);
-        hipFree(dh);
+        if (own_part) {
+            TB_CHECK(c, hipStreamSynchronize(c->s));
+            hipFree(part);
+        }
     } else {
-        std::vector<double> ones((size_t)d.ntot, 1.0);
         for (int q = 0; q < 4; q++)
-            TB_CHECK(c, hipMemcpyAsync(c->f[TB_F_SDF_U + q], ones.data(), sizeof(double) * d.ntot,
-                                       hipMemcpyHostToDevice, c->s));
-        TB_CHECK(c, hipStreamSynchronize(c->s));
+            hipLaunchKernelGGL(k_fill, dim3((unsigned)((d.ntot + 255) / 256)), dim3(256), 0, c->s,
+                               c->f[TB_F_SDF_U + q], 1.0, d.ntot);
+        TB_LAUNCH_CHECK(c);
     }
     // classification
-    uint8_t *pre = nullptr;
-    TB_CHECK(c, hipMalloc((void **)&pre, (size_t)d.ntot));
+    uint8_t *pre = (uint8_t *)c->kv[4];
     for (int q = 0; q < 4; q++) {
         TB_CHECK(c, hipMemsetAsync(c->st[q], 0, (size_t)d.ntot, c->s));
         hipLaunchKernelGGL(k_classify, tiles_grid(all), tiles_block(), 0, c->s, d, q, (int)c->has_geometry,
@@ -606,35 +665,47 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
             TB_LAUNCH_CHECK(c);
         }
     }
-    TB_CHECK(c, hipStreamSynchronize(c->s));
-    hipFree(pre);
     // IB tables: the lexicographic (k, j, i) list of IMMERSED nodes
-    // (Immersed_set_q_immersed_indices, Immersed.c:379-445) is compacted on
-    // the host; everything per node runs on the device.
-    std::vector<uint8_t> hf((size_t)d.NX * d.NY * d.NZ);
+    // (Immersed_set_q_immersed_indices, Immersed.c:379-445).  The rows are counted
+    // on the device, their offsets summed on the host and the list filled on the
+    // device; everything per node runs there too.
+    const long rows = (long)d.NY * d.NZ;
+    std::vector<int> first[4];
+    int *cnt = (int *)c->kv[4];   // [4][rows]; ntot doubles hold them
+    if (c->has_geometry) {
+        for (int q = 0; q < 4; q++)
+            hipLaunchKernelGGL(k_ib_count, dim3((unsigned)((rows + 3) / 4)), dim3(64, 4), 0, c->s, d,
+                               (const uint8_t *)c->st[q], cnt + q * rows);
+        TB_LAUNCH_CHECK(c);
+        for (int q = 0; q < 4; q++) {
+            first[q].resize((size_t)rows + 1);
+            TB_CHECK(c, hipMemcpyAsync(first[q].data() + 1, cnt + q * rows, sizeof(int) * rows, hipMemcpyDeviceToHost,
+                                       c->s));
+        }
+        TB_CHECK(c, hipStreamSynchronize(c->s));
+    }
     for (int q = 0; q < 4; q++) {
-        tb_free_ib(c, q);
+        c->nib[q] = 0;
         if (!c->has_geometry) continue;
-        if (tb_download_flags(c, q, hf.data())) return -1;
-        std::vector<tb_ib_node> nodes;
-        for (int k = 0; k < d.NZ; k++)
-            for (int j = 0; j < d.NY; j++)
-                for (int i = 0; i < d.NX; i++)
-                    if (hf[((size_t)k * d.NY + j) * d.NX + i] == TB_IMMERSED) {
-                        tb_ib_node nd;
-                        memset(&nd, 0, sizeof(nd));
-                        nd.i = i; nd.j = j; nd.k = k;
-                        nodes.push_back(nd);
-                    }
-        int n = (int)nodes.size();
+        first[q][0] = 0;
+        for (long r = 0; r < rows; r++) first[q][r + 1] += first[q][r];
+        const int n = first[q][rows];
         c->nib[q] = n;
         if (n == 0) continue;
-        TB_CHECK(c, hipMalloc((void **)&c->ib[q], sizeof(tb_ib_node) * n));
-        TB_CHECK(c, hipMalloc((void **)&c->ib_row[q], sizeof(long) * n));
-        TB_CHECK(c, hipMalloc((void **)&c->ib_cnt[q], sizeof(int) * n));
-        TB_CHECK(c, hipMalloc((void **)&c->ib_col[q], sizeof(long) * 9 * (size_t)n));
-        TB_CHECK(c, hipMalloc((void **)&c->ib_val[q], sizeof(double) * 9 * (size_t)n));
-        TB_CHECK(c, hipMemcpyAsync(c->ib[q], nodes.data(), sizeof(tb_ib_node) * n, hipMemcpyHostToDevice, c->s));
+        if (n > c->ib_cap[q]) {
+            tb_free_ib(c, q);
+            TB_CHECK(c, hipMalloc((void **)&c->ib[q], sizeof(tb_ib_node) * n));
+            TB_CHECK(c, hipMalloc((void **)&c->ib_row[q], sizeof(long) * n));
+            TB_CHECK(c, hipMalloc((void **)&c->ib_cnt[q], sizeof(int) * n));
+            TB_CHECK(c, hipMalloc((void **)&c->ib_col[q], sizeof(long) * 9 * (size_t)n));
+            TB_CHECK(c, hipMalloc((void **)&c->ib_val[q], sizeof(double) * 9 * (size_t)n));
+            c->ib_cap[q] = n;
+            c->nib[q] = n;
+        }
+        TB_CHECK(c, hipMemcpyAsync(cnt + q * rows, first[q].data(), sizeof(int) * rows, hipMemcpyHostToDevice, c->s));
+        TB_CHECK(c, hipMemsetAsync(c->ib[q], 0, sizeof(tb_ib_node) * n, c->s));
+        hipLaunchKernelGGL(k_ib_list, dim3((unsigned)((rows + 3) / 4)), dim3(64, 4), 0, c->s, d,
+                           (const uint8_t *)c->st[q], (const int *)(cnt + q * rows), c->ib[q]);
         QCoords qc;
         if (q == TB_Q_U) { qc.x = c->g.xu; qc.y = c->g.yu; qc.z = c->g.zu; }
         else if (q == TB_Q_V) { qc.x = c->g.xv; qc.y = c->g.yv; qc.z = c->g.zv; }
@@ -644,8 +715,8 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
                            c->f[TB_F_SDF_U + q], c->st[q], c->ib[q], n);
         TB_LAUNCH_CHECK(c);
         if (tb_ib_rows(c, q)) return -1;
-        TB_CHECK(c, hipStreamSynchronize(c->s));
     }
+    TB_CHECK(c, hipStreamSynchronize(c->s));   // the offsets' host copies end here
     return 0;
 }
 
