@@ -278,6 +278,7 @@ struct HelmHistory {
     double rate[2] = {0.0, 0.0};
     unsigned nsolve = 0;
     double *buf = nullptr;       // second iterate buffer of the solves (allocated on first use, with inc)
+    double *spare = nullptr;     // third one, on the grids whose quantities are solved as one set
     float *inc = nullptr;        // the last solve's increment x_new - x_start, in FP32
     bool inc_ok = false;         // inc belongs to this field's current trajectory
 };
@@ -342,7 +343,7 @@ struct tb_ctx {
     tb_ib_node *ib[4] = {};
     long *ib_row[4] = {};
     int *ib_cnt[4] = {};
-    long *ib_col[4] = {};        // 9 per row, sorted
+    long *ib_col[4] = {};        // 9 per row, sorted; other IMMERSED nodes as complements
     double *ib_val[4] = {};      // 9 per row
     int reinit_its = 0;
     bool has_geometry = false;
@@ -458,6 +459,7 @@ enum {
 // internal entry points shared between translation units
 int tb_geometry_run(tb_ctx *c, const double *h_xz);
 int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0);
+int tb_reduce_read(tb_ctx *c, int nblocks, int nslots, int slot0, int groups = 1, long gstride = 0);
 int tb_read_scalars(tb_ctx *c, int first, int count);
 int tb_wait_published(tb_ctx *c, unsigned long long want);
 int tb_sync(tb_ctx *c);
@@ -484,7 +486,7 @@ int tb_open_store_old(tb_ctx *c);
 int tb_open_rk_average(tb_ctx *c, double old_frac, double new_frac);
 int tb_outflow_async(tb_ctx *c, double dt);   // tb_outflow_convective without the final sync
 void tb_open_free(tb_ctx *c);
-int tb_helm_inc_alloc(tb_ctx *c, int q);   // the increment buffer of quantity q (once)
+int tb_helm_inc_alloc(tb_ctx *c, int q, bool spare);   // the iterate and increment buffers of quantity q (once)
 void tb_free_deposits(tb_ctx *c, int first);
 int tb_ib_rows(tb_ctx *c, int q);
 

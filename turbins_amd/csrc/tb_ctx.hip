@@ -68,10 +68,11 @@ static int dev_alloc(tb_ctx *c, void **p, size_t bytes) {
     return 0;
 }
 
-int tb_helm_inc_alloc(tb_ctx *c, int q) {
+int tb_helm_inc_alloc(tb_ctx *c, int q, bool spare) {
     HelmHistory &h = c->helm[q];
-    if (h.buf && h.inc) return 0;
+    if (h.buf && h.inc && (h.spare || !spare)) return 0;
     h.inc_ok = false;
+    if (spare && !h.spare && dev_alloc(c, (void **)&h.spare, sizeof(double) * (size_t)c->d.ntot)) return -1;
     if (!h.buf && dev_alloc(c, (void **)&h.buf, sizeof(double) * (size_t)c->d.ntot)) return -1;
     if (!h.inc && dev_alloc(c, (void **)&h.inc, sizeof(float) * (size_t)c->d.ntot)) return -1;
     return 0;
@@ -179,9 +180,9 @@ extern "C" void tb_destroy(tb_ctx *c) {
         hipFree(c->cs[n].c); hipFree(c->cs[n].conv); hipFree(c->cs[n].rhs); hipFree(c->cs[n].old);
     }
     tb_open_free(c);
-    for (int q = 0; q < 3; q++) { hipFree(c->helm[q].buf); hipFree(c->helm[q].inc); }
+    for (int q = 0; q < 3; q++) { hipFree(c->helm[q].buf); hipFree(c->helm[q].spare); hipFree(c->helm[q].inc); }
     // slot conc_sel's buffers are helm[3]'s (synced)
-    for (int n = 0; n < TB_NCONC_MAX; n++) { hipFree(c->cs[n].h.buf); hipFree(c->cs[n].h.inc); }
+    for (int n = 0; n < TB_NCONC_MAX; n++) { hipFree(c->cs[n].h.buf); hipFree(c->cs[n].h.spare); hipFree(c->cs[n].h.inc); }
     hipFree(c->ctot);
     tb_free_deposits(c, 0);
     for (int f = 0; f < TB_F_COUNT; f++) hipFree(c->f[f]);
@@ -449,20 +450,38 @@ extern "C" int tb_set_helmholtz_rtol(tb_ctx *c, double rtol) {
 // ---------------------------------------------------------------------------
 // reductions
 
+// the word that tells the host that hscal is written (see k_publish)
+__device__ inline void publish(unsigned long long *hseq, unsigned long long seq) {
+    __threadfence_system();
+    *(volatile unsigned long long *)hseq = seq;
+}
+
+// sums of `groups` sets of nslots partial-sum arrays, gstride apart, into
+// out[slot0 ...], set by set; with hscal given also published to the host
 __global__ void k_reduce_finish(const double *__restrict__ part, double *__restrict__ out, int nblocks,
-                                int nslots, int slot0) {
+                                int nslots, int slot0, int groups, long gstride, double *hscal,
+                                unsigned long long *hseq, unsigned long long seq) {
     __shared__ double sh[RED_SLOTS * 16];
-    double v[RED_SLOTS];
+    for (int g = 0; g < groups; g++) {
+        double v[RED_SLOTS];
 #pragma unroll
-    for (int a = 0; a < RED_SLOTS; a++) {
-        double s = 0.0;
-        if (a < nslots)
-            for (int b = threadIdx.x; b < nblocks; b += blockDim.x) s += part[a * RED_MAX_BLOCKS + b];
-        v[a] = s;
+        for (int a = 0; a < RED_SLOTS; a++) {
+            double s = 0.0;
+            if (a < nslots)
+                for (int b = threadIdx.x; b < nblocks; b += blockDim.x) s += part[a * (long)RED_MAX_BLOCKS + b];
+            v[a] = s;
+        }
+        block_sum<RED_SLOTS>(v, sh);
+        if (threadIdx.x == 0)
+            for (int a = 0; a < nslots; a++) {
+                out[slot0 + a] = v[a];
+                if (hscal) hscal[slot0 + a] = v[a];
+            }
+        __syncthreads();   // the next set's sums reuse sh
+        part += gstride;
+        slot0 += nslots;
     }
-    block_sum<RED_SLOTS>(v, sh);
-    if (threadIdx.x == 0)
-        for (int a = 0; a < nslots; a++) out[slot0 + a] = v[a];
+    if (hscal && threadIdx.x == 0) publish(hseq, seq);
 }
 
 // Scalar read-back without a blocking stream synchronisation: one thread
@@ -478,8 +497,7 @@ __global__ void k_publish(const double *__restrict__ scal, int first, int count,
                           unsigned long long *hseq, unsigned long long seq) {
     if (threadIdx.x != 0) return;
     for (int a = 0; a < count; a++) hscal[first + a] = scal[first + a];
-    __threadfence_system();
-    *(volatile unsigned long long *)hseq = seq;
+    publish(hseq, seq);
 }
 
 // spin until the device has published sequence number want (or a later one)
@@ -511,9 +529,20 @@ int tb_read_scalars(tb_ctx *c, int first, int count) {
 int tb_sync(tb_ctx *c) { return tb_read_scalars(c, 0, 0); }
 
 int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0) {
-    hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, c->s, c->red, c->scal, nblocks, nslots, slot0);
+    hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, c->s, c->red, c->scal, nblocks, nslots, slot0, 1, 0L,
+                       (double *)nullptr, (unsigned long long *)nullptr, 0ull);
     TB_LAUNCH_CHECK(c);
     return 0;
+}
+
+// tb_reduce_finish and the read-back of its sums in one launch (each launch
+// and its gap cost 3 us or more): hscal[slot0 ...] holds them on return
+int tb_reduce_read(tb_ctx *c, int nblocks, int nslots, int slot0, int groups, long gstride) {
+    const unsigned long long want = ++c->pub_seq;
+    hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, c->s, c->red, c->scal, nblocks, nslots, slot0, groups,
+                       gstride, c->hscal, c->hseq, want);
+    TB_LAUNCH_CHECK(c);
+    return tb_wait_published(c, want);
 }
 
 constexpr int DOT_BLOCKS = 1024;
@@ -635,6 +664,7 @@ extern "C" int tb_set_conc_fields(tb_ctx *c, int nconc, const tb_conc_field *fie
         } else {
             dev_release(c, s.c); dev_release(c, s.conv); dev_release(c, s.rhs); dev_release(c, s.old);
             dev_release(c, s.h.buf);
+            dev_release(c, s.h.spare);
             dev_release(c, s.h.inc);
         }
     }
@@ -646,10 +676,11 @@ extern "C" int tb_set_conc_fields(tb_ctx *c, int nconc, const tb_conc_field *fie
     }
     for (int n = 0; n < nconc; n++) {
         c->cs[n].p = fields[n];
-        double *buf = c->cs[n].h.buf;   // kept, the increment's content no longer a guess
+        double *buf = c->cs[n].h.buf, *spare = c->cs[n].h.spare;   // kept, the increment's content no longer a guess
         float *inc = c->cs[n].h.inc;
         c->cs[n].h = HelmHistory();
         c->cs[n].h.buf = buf;
+        c->cs[n].h.spare = spare;
         c->cs[n].h.inc = inc;
     }
     c->helm[TB_Q_C] = c->cs[0].h;

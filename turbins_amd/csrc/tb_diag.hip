@@ -449,8 +449,7 @@ int cell_sums(tb_ctx *c, bool visc, int nslots, double *out, const char *who) {
                            c->red, t);
     }
     TB_LAUNCH_CHECK(c);
-    if (tb_reduce_finish(c, (int)grid.x, nslots, S_TMP0)) return -1;
-    if (tb_read_scalars(c, S_TMP0, nslots)) return -1;
+    if (tb_reduce_read(c, (int)grid.x, nslots, S_TMP0)) return -1;
     for (int a = 0; a < nslots; a++) out[a] = c->hscal[S_TMP0 + a];
     return 0;
 }

@@ -1113,8 +1113,7 @@ static int diag_sums(tb_ctx *c, double out[3]) {
                        (const double *)c->f[TB_F_V], (const double *)c->f[TB_F_W], (const double *)c->f[TB_F_C],
                        (const uint8_t *)c->st[3], c->red, t, tb_in_plane(c, TB_Q_U), tb_out_plane(c, TB_Q_U));
     TB_LAUNCH_CHECK(c);
-    if (tb_reduce_finish(c, (int)grid.x, 3, S_TMP0)) return -1;
-    if (tb_read_scalars(c, S_TMP0, 3)) return -1;
+    if (tb_reduce_read(c, (int)grid.x, 3, S_TMP0)) return -1;
     for (int a = 0; a < 3; a++) out[a] = c->hscal[S_TMP0 + a];
     return 0;
 }

@@ -530,9 +530,10 @@ __global__ void __launch_bounds__(256) k_ib_list(Dims d, const uint8_t *__restri
 
 // Matrix row of an IMMERSED node (Velocity.c:718-762, Conc.c:668-708):
 // self coefficient 1 + sum of self weights, other weights with
-// |coef| >= LSYS_DROP_TOLERANCE, all scaled by ap_solid; columns sorted.
-__global__ void k_ib_rows(Dims d, const tb_ib_node *nodes, int n, double ap_solid, long *row, int *cnt, long *col,
-                          double *val) {
+// |coef| >= LSYS_DROP_TOLERANCE, all scaled by ap_solid; columns sorted.  The
+// column of another IMMERSED node is stored as its complement.
+__global__ void k_ib_rows(Dims d, const uint8_t *__restrict__ st, const tb_ib_node *nodes, int n, double ap_solid,
+                          long *row, int *cnt, long *col, double *val) {
     int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= n) return;
     const tb_ib_node &nd = nodes[a];
@@ -554,7 +555,8 @@ __global__ void k_ib_rows(Dims d, const tb_ib_node *nodes, int n, double ap_soli
     row[a] = self;
     cnt[a] = m;
     for (int s = 0; s < 9; s++) {
-        col[(long)a * 9 + s] = (s < m) ? cc[s] : self;
+        const long ce = (s < m) ? cc[s] : self;
+        col[(long)a * 9 + s] = (ce != self && st[ce] == TB_IMMERSED) ? ~ce : ce;
         val[(long)a * 9 + s] = (s < m) ? vv[s] : 0.0;
     }
 }
@@ -573,7 +575,8 @@ static double ap_solid_for(tb_ctx *c, int q) {
 int tb_ib_rows(tb_ctx *c, int q) {
     const int n = c->nib[q];
     if (n == 0) return 0;
-    hipLaunchKernelGGL(k_ib_rows, dim3((n + 63) / 64), dim3(64), 0, c->s, c->d, (const tb_ib_node *)c->ib[q], n,
+    hipLaunchKernelGGL(k_ib_rows, dim3((n + 63) / 64), dim3(64), 0, c->s, c->d,
+                       (const uint8_t *)c->st[q], (const tb_ib_node *)c->ib[q], n,
                        ap_solid_for(c, q), c->ib_row[q], c->ib_cnt[q], c->ib_col[q], c->ib_val[q]);
     TB_LAUNCH_CHECK(c);
     return 0;

@@ -14,6 +14,7 @@
 // registers.  The neighbour-status tests of the reference reduce to index
 // tests, because BOUNDARY nodes are exactly the box planes.
 #include <cmath>
+#include <utility>
 
 #include "tb_common.h"
 
@@ -32,6 +33,33 @@ struct HelmOp {
     int open_w, open_e;
 };
 
+// What the Gauss-Seidel kernels need of one quantity's solve.  On small grids
+// u, v, w and the concentration fields are solved side by side, one grid row
+// (blockIdx.y) each: their systems are independent, and one quantity's launches
+// leave most of the chip idle there.
+struct GsView {
+    HelmOp H;
+    const double *b, *x0;          // right-hand side; the field the solve started from
+    const double *from;            // iterate read and iterate written by a pair
+    double *to;
+    const float *inc;              // increment added to `from` (none: null)
+    float *dn;                     // increment to - x0, written by the residual check
+    const long *row, *col;         // IMMERSED rows (ib_row, ...)
+    const int *cnt;
+    const double *val;
+    int nib;
+};
+
+constexpr int HELM_SET = 3 + TB_NCONC_MAX;
+
+template <int N>
+struct GsSet {   // a kernel argument: at most 4 KB
+    GsView v[N];
+    __device__ const GsView &mine() const { return v[N == 1 ? 0 : blockIdx.y]; }
+};
+
+static_assert(sizeof(GsSet<HELM_SET>) <= 4096 - 64, "kernel arguments");
+
 // wall rule applied to ap when a neighbour is absent:
 // 0 nothing (normal component on the wall), 1 no-slip (ap -= a),
 // 2 free-slip / Neumann (ap += a)
@@ -43,15 +71,15 @@ __device__ inline double wallmod(double ap, double a, int rule) {
 
 // MODE 0: y = A x ; MODE 1: also partial w.y ; MODE 2: also partials x.y, y.y
 // MODE 3: residual only: partials |w - A x|^2 and |w|^2 with w = b, nothing
-// stored except that IMMERSED rows must hold (A x) from k_ib_apply in y.
-// MODE 4: MODE 3 and the increment dn = x - x0 over the box (the Gauss-Seidel
-// solve's change to the field it started from).
+// stored (IMMERSED rows must hold (A x) from k_ib_apply in y), and the
+// increment dn = x - x0 over the box (the Gauss-Seidel solve's change to the
+// field it started from).
 // IMMERSED rows are produced by k_ib_apply, which runs first; here their y is
 // only read for the dot products.
 template <int MODE>
-__global__ void __launch_bounds__(256) k_helm_km(HelmOp H, const double *__restrict__ x, double *__restrict__ y,
-                                                 const double *__restrict__ w, double *part, KTiles t,
-                                                 const double *__restrict__ x0, float *__restrict__ dn) {
+__device__ __forceinline__ void helm_rows(const HelmOp &H, const double *__restrict__ x, double *__restrict__ y,
+                                          const double *__restrict__ w, double *part, const KTiles &t,
+                                          const double *__restrict__ x0, float *__restrict__ dn) {
     __shared__ double sh[32];
     double acc[2] = {0.0, 0.0};
     int i, j, k0, k1;
@@ -122,8 +150,8 @@ __global__ void __launch_bounds__(256) k_helm_km(HelmOp H, const double *__restr
         for (int k = k0; k < k1; k++) {
             double xp = x[id + ((k + 1 < NZ) ? d.plane : 0)];
             const double xs = x[id - os], xw = x[id - ow], xe = x[id + oe], xn = x[id + on];
-            const double wv = (MODE == 1 || MODE >= 3) ? __builtin_nontemporal_load(&w[id]) : 0.0;
-            const double x0v = (MODE == 4) ? __builtin_nontemporal_load(&x0[id]) : 0.0;
+            const double wv = (MODE == 1 || MODE == 3) ? __builtin_nontemporal_load(&w[id]) : 0.0;
+            const double x0v = (MODE == 3) ? __builtin_nontemporal_load(&x0[id]) : 0.0;
             const int s = H.st[id];
             // the fluid row is formed for every node and selected afterwards:
             // no status-dependent branch sits between the loads and the math
@@ -159,9 +187,9 @@ __global__ void __launch_bounds__(256) k_helm_km(HelmOp H, const double *__restr
             } else if (MODE < 3) {
                 st_stream(&y[id], yv);
             }
-            if (MODE == 4) st_stream(&dn[id], (float)(xc - x0v));
+            if (MODE == 3) st_stream(&dn[id], (float)(xc - x0v));
             if (MODE == 1) acc[0] += wv * yv;
-            if (MODE >= 3) { acc[0] += (wv - yv) * (wv - yv); acc[1] += wv * wv; }
+            if (MODE == 3) { acc[0] += (wv - yv) * (wv - yv); acc[1] += wv * wv; }
             if (MODE == 2) { acc[0] += xc * yv; acc[1] += yv * yv; }
             xm = xc;
             xc = xp;
@@ -177,16 +205,28 @@ __global__ void __launch_bounds__(256) k_helm_km(HelmOp H, const double *__restr
     }
 }
 
+template <int MODE>
+__global__ void __launch_bounds__(256) k_helm_km(HelmOp H, const double *__restrict__ x, double *__restrict__ y,
+                                                 const double *__restrict__ w, double *part, KTiles t) {
+    helm_rows<MODE>(H, x, y, w, part, t, nullptr, nullptr);
+}
+
+// residual check of each solve of the set: x = from, A x of the IMMERSED rows
+// in `to`; partial sums pstride apart
+template <int N>
+__global__ void __launch_bounds__(256) k_helm_check(GsSet<N> S, double *part, long pstride, KTiles t) {
+    const GsView &V = S.mine();
+    helm_rows<3>(V.H, V.from, V.to, V.b, part + (N == 1 ? 0 : blockIdx.y) * pstride, t, V.x0, V.dn);
+}
+
 // IMMERSED rows from the sorted IB row table.  With target > 0 each row is
 // multiplied by target / (its diagonal): inside the Krylov solve this
 // rescales the IB equations (right-hand side 0) to the size of the fluid
 // rows, which takes BiCGStab from ~15-20 to 3-4 iterations; any scaled
 // residual >= the true one, so the stopping test stays conservative.
-__global__ void k_ib_apply(const long *__restrict__ row, const int *__restrict__ cnt, const long *__restrict__ col,
-                           const double *__restrict__ val, int n, const double *__restrict__ x,
-                           double *__restrict__ y, double target) {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n) return;
+__device__ __forceinline__ void ib_apply_row(int a, const long *__restrict__ row, const int *__restrict__ cnt,
+                                             const long *__restrict__ col, const double *__restrict__ val,
+                                             const double *__restrict__ x, double *__restrict__ y, double target) {
     double s = 0.0, dg = 1.0;
     const long r = row[a];
     const int m = cnt[a];
@@ -195,7 +235,8 @@ __global__ void k_ib_apply(const long *__restrict__ row, const int *__restrict__
     double cv[9], xv[9];
 #pragma unroll
     for (int e = 0; e < 9; e++) {
-        ci[e] = e < m ? col[(long)a * 9 + e] : r;
+        const long ce = e < m ? col[(long)a * 9 + e] : r;
+        ci[e] = ce < 0 ? ~ce : ce;
         cv[e] = e < m ? val[(long)a * 9 + e] : 0.0;
     }
 #pragma unroll
@@ -208,6 +249,21 @@ __global__ void k_ib_apply(const long *__restrict__ row, const int *__restrict__
     }
     double f = (target > 0.0) ? target / dg : 1.0;
     y[r] = (f > 1.0) ? f * s : s;
+}
+
+__global__ void k_ib_apply(const long *__restrict__ row, const int *__restrict__ cnt, const long *__restrict__ col,
+                           const double *__restrict__ val, int n, const double *__restrict__ x,
+                           double *__restrict__ y, double target) {
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a < n) ib_apply_row(a, row, cnt, col, val, x, y, target);
+}
+
+// (A x) of each solve's IMMERSED rows for k_helm_check
+template <int N>
+__global__ void k_ib_check(GsSet<N> S) {
+    const GsView &V = S.mine();
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a < V.nib) ib_apply_row(a, V.row, V.cnt, V.col, V.val, V.from, V.to, 0.0);
 }
 
 static HelmOp make_op(tb_ctx *c, int q, double dt) {
@@ -228,10 +284,10 @@ static HelmOp make_op(tb_ctx *c, int q, double dt) {
     return H;
 }
 
-// y = A x (scaled: IB rows rescaled for the Krylov solve); mode 1/2/3 leave
+// y = A x (scaled: IB rows rescaled for the Krylov solve); mode 1/2 leave
 // partial sums in c->red.  Returns the number of partials, or -1.
 static int helm_apply(tb_ctx *c, const HelmOp &H, const double *x, double *y, bool scaled, int mode,
-                      const double *w = nullptr, const double *x0 = nullptr, float *dn = nullptr) {
+                      const double *w = nullptr) {
     int q = H.q;
     if (c->nib[q] > 0)
         hipLaunchKernelGGL(k_ib_apply, dim3((c->nib[q] + 255) / 256), dim3(256), 0, c->s, c->ib_row[q], c->ib_cnt[q],
@@ -239,15 +295,11 @@ static int helm_apply(tb_ctx *c, const HelmOp &H, const double *x, double *y, bo
     KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ);
     if (c->prof_on) tb_prof_begin(c, TB_K_HELM_OP);
     if (mode == 0)
-        hipLaunchKernelGGL(k_helm_km<0>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t, x0, dn);
+        hipLaunchKernelGGL(k_helm_km<0>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t);
     else if (mode == 1)
-        hipLaunchKernelGGL(k_helm_km<1>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t, x0, dn);
-    else if (mode == 2)
-        hipLaunchKernelGGL(k_helm_km<2>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t, x0, dn);
-    else if (mode == 3)
-        hipLaunchKernelGGL(k_helm_km<3>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t, x0, dn);
+        hipLaunchKernelGGL(k_helm_km<1>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t);
     else
-        hipLaunchKernelGGL(k_helm_km<4>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t, x0, dn);
+        hipLaunchKernelGGL(k_helm_km<2>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t);
     if (c->prof_on) tb_prof_end(c, TB_K_HELM_OP);
     TB_LAUNCH_CHECK(c);
     return (int)(t.per_xcd * NXCD);
@@ -406,13 +458,14 @@ constexpr int GS_START = 3;         // plane steps a block's start takes
 // The tiles cover the box without its last plane along each axis (see
 // k_gs_last_planes), so 512 x 256 x 128 cells take exactly 8 x 16 x 4 tiles
 // instead of 9 x 17 x 9 with nearly empty ones walking the full plane chain.
-static GsTiles make_gs_tiles(const Dims &d) {
+// nq: solves in the launch
+static GsTiles make_gs_tiles(const Dims &d, int nq) {
     GsTiles t;
     t.tx = (d.NX - 1 + GS_TX - 1) / GS_TX;
     t.ty = (d.NY - 1 + GS_TY - 1) / GS_TY;
     long best = 0;
     for (int tk = GS_TK_MAX; tk >= 1; tk--) {
-        const long kc = (d.NZ - 1 + tk - 1) / tk, n = t.tx * t.ty * kc;
+        const long kc = (d.NZ - 1 + tk - 1) / tk, n = t.tx * t.ty * kc * nq;
         const long step = n <= GS_RESIDENT / 2 ? 5 : 8 * ((n + GS_RESIDENT - 1) / GS_RESIDENT);
         const long cost = step * (tk + 3 + GS_START);
         if (best == 0 || cost < best) { best = cost; t.tk = tk; t.kc = (int)kc; }
@@ -428,11 +481,11 @@ static GsTiles make_gs_tiles(const Dims &d) {
 // positions outside the box hold zeros or finite values of other planes.
 // Element offsets are 32-bit (the host checks the field size).  ADD: the
 // pair starts from xo + dd (the field plus the last solve's increment, an
-// extrapolated initial guess) without forming it in memory.
+// extrapolated initial guess; dd null: xo) without forming it in memory.
 template <bool ADD>
-__global__ void __launch_bounds__(GS_THREADS) k_helm_gs_pair(HelmOp H, const double *__restrict__ xo,
-                                                             double *__restrict__ xn, const double *__restrict__ b,
-                                                             GsTiles T, const float *__restrict__ dd) {
+__device__ __forceinline__ void gs_pair(const HelmOp &H, const double *__restrict__ xo, double *__restrict__ xn,
+                                        const double *__restrict__ b, const GsTiles &T,
+                                        const float *__restrict__ dd) {
     __shared__ double so[GS_ORING][GS_OY * GS_OX];
     __shared__ double sr[3][GS_HY * GS_HX];
     __shared__ AxisGS cx[GS_OX], cy[GS_OY], cz[GS_OZ];
@@ -483,7 +536,7 @@ __global__ void __launch_bounds__(GS_THREADS) k_helm_gs_pair(HelmOp H, const dou
 #pragma unroll
         for (int u = 0; u < GS_OLD_PER; u++) {
             ro[u] = ooff[u] >= 0 ? xo[m * plane + ooff[u]] : 0.0;
-            if (ADD) rd[u] = ooff[u] >= 0 ? dd[m * plane + ooff[u]] : 0.0f;
+            if (ADD) rd[u] = dd && ooff[u] >= 0 ? dd[m * plane + ooff[u]] : 0.0f;
         }
     };
     auto put_old = [&](int m) {
@@ -608,14 +661,24 @@ __global__ void __launch_bounds__(GS_THREADS) k_helm_gs_pair(HelmOp H, const dou
     write_plane(k1 - 1);
 }
 
+template <bool ADD, int N>
+__global__ void __launch_bounds__(GS_THREADS) k_helm_gs_pair(GsSet<N> S, GsTiles T) {
+    const GsView &V = S.mine();
+    gs_pair<ADD>(V.H, V.from, V.to, V.b, T, V.inc);
+}
+
 // The last plane of each axis, outside the sweep tiles.  Its points are
 // BOUNDARY by classification: their rows read ap_solid q = b and no other
 // row couples to them (zero coefficients), so their Gauss-Seidel value
 // b / (ap_solid + 1/dt), the expression of gs_value, does not depend on x and
-// is written into both iterate buffers once per gs_pairs call.  Points where
-// two planes meet are written twice with the same value.
-__global__ void k_gs_last_planes(HelmOp H, const double *__restrict__ b, double *__restrict__ x1,
-                                 double *__restrict__ x2) {
+// is written into both iterate buffers (from and to) once per solve.  Points
+// where two planes meet are written twice with the same value.
+template <int N>
+__global__ void k_gs_last_planes(GsSet<N> S) {
+    const GsView &V = S.mine();
+    const HelmOp &H = V.H;
+    const double *b = V.b;
+    double *x1 = const_cast<double *>(V.from), *x2 = V.to;
     const Dims &d = H.d;
     const long n1 = (long)d.NY * d.NZ, n2 = (long)d.NX * d.NZ, n3 = (long)d.NX * d.NY;
     long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -636,27 +699,38 @@ __global__ void k_gs_last_planes(HelmOp H, const double *__restrict__ b, double 
     x2[id] = v;
 }
 
-// IMMERSED rows, Jacobi over the IB table: new value of row a into tmp[a]
-// (x_im = (b_im - sum_{g != im} v_g x_g) / v_im), then scattered, so the
-// result does not depend on the order in which rows run
-__global__ void k_ib_gs(const long *__restrict__ row, const int *__restrict__ cnt, const long *__restrict__ col,
-                        const double *__restrict__ val, int n, const double *__restrict__ x,
-                        const double *__restrict__ b, double *__restrict__ tmp) {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    const long r = row[a];
-    const int m = cnt[a];
+// IMMERSED rows, Jacobi over the IB table (x_im = (b_im - sum_{g != im} v_g
+// x_g) / v_im): the row's new value is written over the old one that the pair
+// left in `to`; other IMMERSED nodes (complemented columns) are read where the
+// pair read them, in `from` (+ inc), so the result does not depend on the
+// order in which rows run and takes one launch (with a buffer between and a
+// second one it was 4 + 3 us and a gap at 200x72x36, 8 + 5 at 512x256x128).
+template <int N>
+__global__ void k_ib_gs(GsSet<N> S) {
+    const GsView &V = S.mine();
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a >= V.nib) return;
+    const double *from = V.from, *b = V.b;
+    double *x = V.to;
+    const float *inc = V.inc;
+    const long r = V.row[a];
+    const int m = V.cnt[a];
     // every column and value, then every gather, issued before the first
     // is used; the sum runs in column order as a loop over them would
     long ci[9];
     double cv[9], xv[9];
 #pragma unroll
     for (int e = 0; e < 9; e++) {
-        ci[e] = e < m ? col[(long)a * 9 + e] : r;
-        cv[e] = e < m ? val[(long)a * 9 + e] : 0.0;
+        ci[e] = e < m ? V.col[(long)a * 9 + e] : r;
+        cv[e] = e < m ? V.val[(long)a * 9 + e] : 0.0;
     }
 #pragma unroll
-    for (int e = 0; e < 9; e++) xv[e] = (e < m && ci[e] != r) ? x[ci[e]] : 0.0;
+    for (int e = 0; e < 9; e++) {
+        xv[e] = 0.0;
+        if (e >= m || ci[e] == r) continue;
+        if (ci[e] >= 0) xv[e] = x[ci[e]];
+        else xv[e] = inc ? from[~ci[e]] + (double)inc[~ci[e]] : from[~ci[e]];
+    }
     double s = 0.0, dg = 1.0;
 #pragma unroll
     for (int e = 0; e < 9; e++) {
@@ -664,74 +738,108 @@ __global__ void k_ib_gs(const long *__restrict__ row, const int *__restrict__ cn
         if (ci[e] == r) dg = cv[e];
         else s += cv[e] * xv[e];
     }
-    tmp[a] = (b[r] - s) / dg;
+    x[r] = (b[r] - s) / dg;
 }
 
-__global__ void k_ib_scatter(const long *__restrict__ row, int n, const double *__restrict__ tmp,
-                             double *__restrict__ x) {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a < n) x[row[a]] = tmp[a];
+// One quantity's Gauss-Seidel solve
+struct GsRun {
+    int q = 0;
+    int field = 0;                 // concentration field (q = TB_Q_C)
+    HelmOp H;
+    double *x = nullptr;           // the field; kept while the solve runs
+    const double *b = nullptr;
+    double *cur = nullptr, *alt = nullptr;   // iterate buffers
+    bool spare = false;            // alt comes from the history's third buffer, else kv[6]
+    const double *src = nullptr;   // start of the first pair (else cur)
+    const float *inc = nullptr;    // and the increment added to it
+    bool planes = false;           // last planes written
+    HelmHistory h;
+    int nib = 0;
+    const long *row = nullptr, *col = nullptr;
+    const int *cnt = nullptr;
+    const double *val = nullptr;
+    int par = 0, chunk = 0, todo = 0, its = 0;
+    double prev = NAN, rate = 0.0, res = NAN;
+    bool done = false, ok = false;
+};
+
+static void gs_ib(tb_ctx *c, GsRun &r) {
+    const int q = r.q;
+    r.nib = c->nib[q];
+    r.row = c->ib_row[q]; r.col = c->ib_col[q]; r.cnt = c->ib_cnt[q]; r.val = c->ib_val[q];
 }
 
-// ||b - A x||^2 and ||b||^2 into S_TMP1, S_TMP2 (host mirror)
-// |b - A x|^2 and |b|^2; with x0 given also the increment x - x0 into dn
-static int helm_residual(tb_ctx *c, const HelmOp &H, const double *x, const double *b, double *ibuf, double &rr,
-                         double &bb, const double *x0 = nullptr, float *dn = nullptr) {
-    int nb = helm_apply(c, H, x, ibuf, false, x0 ? 4 : 3, b, x0, dn);
-    if (nb < 0 || tb_reduce_finish(c, nb, 2, S_TMP1)) return -1;
-    if (tb_read_scalars(c, S_TMP1, 2)) return -1;
-    rr = c->hscal[S_TMP1];
-    bb = c->hscal[S_TMP2];
-    return 0;
+static GsView view(const GsRun &r, const double *from, double *to, const float *inc) {
+    return {r.H, r.b, r.x, from, to, inc, r.h.inc, r.row, r.col, r.cnt, r.val, r.nib};
 }
 
-// n sweep pairs, each followed by the Jacobi update of the IMMERSED rows,
-// alternating between the buffers cur and alt (the same size and pitch);
-// cur is swapped to the buffer that holds the result.  With src given the
-// first pair starts from src (plus inc, when given) instead of cur; inc may
-// be cur itself: the last planes written into cur first are read there only
-// with zero coefficients (no row couples to them).
-static int gs_pairs(tb_ctx *c, const HelmOp &H, double *&cur, double *&alt, const double *b, int n,
-                    const double *src = nullptr, const float *inc = nullptr) {
-    const int q = H.q;
-    double *tmp = c->kv[4];
-    const GsTiles T = make_gs_tiles(c->d);
+// up to todo sweep pairs of each run, each followed by the Jacobi update of
+// the IMMERSED rows, alternating between the buffers cur and alt (the same
+// size and pitch); cur is swapped to the buffer that holds the result
+template <int N>
+static int gs_pairs(tb_ctx *c, GsRun *const *run, int n) {
     if (c->d.ntot >= (1L << 31)) {
         c->err = "Helmholtz sweeps: field exceeds 2^31 elements";
         return -1;
     }
-    if (n > 0) {
-        const Dims &d = c->d;
+    const Dims &d = c->d;
+    GsSet<N> S;
+    int m = 0, most = 0;
+    for (int a = 0; a < n; a++) {
+        most = run[a]->todo > most ? run[a]->todo : most;
+        if (run[a]->planes || run[a]->todo < 1) continue;
+        run[a]->planes = true;
+        S.v[m++] = view(*run[a], run[a]->cur, run[a]->alt, nullptr);
+    }
+    if (m > 0) {
         const long np = (long)d.NY * d.NZ + (long)d.NX * d.NZ + (long)d.NX * d.NY;
-        hipLaunchKernelGGL(k_gs_last_planes, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->s, H, b, cur, alt);
+        hipLaunchKernelGGL(k_gs_last_planes<N>, dim3((unsigned)((np + 255) / 256), m), dim3(256), 0, c->s, S);
         TB_LAUNCH_CHECK(c);
     }
-    for (int sw = 0; sw < n; sw++) {
-        const double *from = (sw == 0 && src) ? src : cur;
-        if (sw == 0 && src && inc) {
-            TB_PROF(c, TB_K_HELM_GS,
-                    hipLaunchKernelGGL(k_helm_gs_pair<true>, dim3(T.per_xcd * NXCD), dim3(GS_THREADS), 0, c->s, H,
-                                       from, alt, b, T, inc));
-        } else {
-            TB_PROF(c, TB_K_HELM_GS,
-                    hipLaunchKernelGGL(k_helm_gs_pair<false>, dim3(T.per_xcd * NXCD), dim3(GS_THREADS), 0, c->s, H,
-                                       from, alt, b, T, (const float *)nullptr));
+    for (int sw = 0; sw < most; sw++) {
+        int nib = 0;
+        bool add = false;
+        m = 0;
+        for (int a = 0; a < n; a++) {
+            GsRun &r = *run[a];
+            if (sw >= r.todo) continue;
+            S.v[m++] = view(r, r.src ? r.src : r.cur, r.alt, r.src ? r.inc : nullptr);
+            add |= r.src && r.inc;
+            nib = r.nib > nib ? r.nib : nib;
+            r.src = nullptr;
+            std::swap(r.cur, r.alt);
         }
-        double *w = cur;
-        cur = alt;
-        alt = w;
-        if (c->nib[q] > 0) {
-            const dim3 gi((c->nib[q] + 255) / 256);
-            if (c->prof_on) tb_prof_begin(c, TB_K_IB);
-            hipLaunchKernelGGL(k_ib_gs, gi, dim3(256), 0, c->s, c->ib_row[q], c->ib_cnt[q], c->ib_col[q],
-                               c->ib_val[q], c->nib[q], (const double *)cur, b, tmp);
-            hipLaunchKernelGGL(k_ib_scatter, gi, dim3(256), 0, c->s, c->ib_row[q], c->nib[q], (const double *)tmp,
-                               cur);
-            if (c->prof_on) tb_prof_end(c, TB_K_IB);
-        }
+        const GsTiles T = make_gs_tiles(d, m);
+        const dim3 grid(T.per_xcd * NXCD, m);
+        if (add) TB_PROF(c, TB_K_HELM_GS, hipLaunchKernelGGL((k_helm_gs_pair<true, N>), grid, dim3(GS_THREADS), 0, c->s, S, T));
+        else TB_PROF(c, TB_K_HELM_GS, hipLaunchKernelGGL((k_helm_gs_pair<false, N>), grid, dim3(GS_THREADS), 0, c->s, S, T));
+        if (nib > 0)
+            TB_PROF(c, TB_K_IB, hipLaunchKernelGGL(k_ib_gs<N>, dim3((nib + 255) / 256, m), dim3(256), 0, c->s, S));
         TB_LAUNCH_CHECK(c);
     }
     return 0;
+}
+
+// |b - A x|^2 and |b|^2 of each run's iterate into hscal[S_SUB + 2 a ...], its
+// increment over the field into h.inc; the other iterate's IMMERSED rows,
+// which no pair reads, hold A x in between
+template <int N>
+static int gs_check(tb_ctx *c, GsRun *const *run, int n) {
+    constexpr long PART = RED_MAX_BLOCKS / HELM_SET;
+    GsSet<N> S;
+    int nib = 0;
+    for (int a = 0; a < n; a++) {
+        S.v[a] = view(*run[a], run[a]->cur, run[a]->alt, nullptr);
+        nib = run[a]->nib > nib ? run[a]->nib : nib;
+    }
+    if (nib > 0) hipLaunchKernelGGL(k_ib_check<N>, dim3((nib + 255) / 256, n), dim3(256), 0, c->s, S);
+    const KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ);
+    dim3 grid = ktiles_grid(t);
+    grid.y = n;
+    TB_PROF(c, TB_K_HELM_OP, hipLaunchKernelGGL(k_helm_check<N>, grid, tiles_block(), 0, c->s, S, c->red, PART, t));
+    TB_LAUNCH_CHECK(c);
+    TB_CHECK(c, hipEventRecord(c->ev1, c->s));   // the sums below end after it
+    return tb_reduce_read(c, (int)(t.per_xcd * NXCD), 2, S_SUB, n, PART);
 }
 
 // copy the box points of src into dst (row padding untouched)
@@ -742,21 +850,43 @@ static int copy_box(tb_ctx *c, double *dst, const double *src) {
     return 0;
 }
 
-// returns 0 and sets ok when converged (the field of quantity q then holds
-// the solution); ok = false when the sweeps stall (contraction per pair worse
-// than 0.5) or run out of sweeps, x then holds the last iterate.  The initial
-// guess is the field plus the increment of the quantity's last solve, when
-// that solve converged on the same trajectory (the reference starts from the
-// field alone; both stop at the same residual test).  Three FP64 buffers
-// take part: the field x, read by the first pair and kept so that each
-// residual check also writes the increment, and the two iterate buffers,
-// kv[6] and the quantity's own second buffer.  On convergence the field
-// takes the result's buffer, the second buffer the other iterate's and
-// kv[6] the old field's (no kernel or graph keeps any of these pointers
-// between calls).  The increment is kept in FP32: it only moves the start
-// of the next solve, which converges to the same residual test, and the
-// check that writes it and the first pair that reads it stream half the
-// bytes for it.
+// Grids up to this size have all their quantities solved as one set, each with
+// a third iterate buffer of its own.
+constexpr long HELM_SET_POINTS = 1L << 20;
+
+// the run of quantity q (the selected concentration field's for TB_Q_C)
+static int gs_begin(tb_ctx *c, int q, const HelmOp &H, GsRun &r) {
+    r.spare = c->d.ntot <= HELM_SET_POINTS;
+    if (tb_helm_inc_alloc(c, q, r.spare)) return -1;
+    r.q = q;
+    r.field = c->conc_sel;
+    r.H = H;
+    r.x = c->f[TB_F_U + q];
+    r.b = c->f[TB_F_RHS_U + q];
+    r.h = c->helm[q];
+    gs_ib(c, r);
+    r.src = r.x;
+    r.inc = r.h.inc_ok ? r.h.inc : nullptr;
+    c->helm[q].inc_ok = r.h.inc_ok = false;   // the increment is overwritten by the first residual check
+    r.cur = r.h.buf;
+    r.alt = r.spare ? r.h.spare : c->kv[6];
+    r.par = (int)(r.h.nsolve++ & 1u);
+    r.chunk = r.h.sweeps[r.par] > 0 ? r.h.sweeps[r.par] : 2;
+    r.rate = r.h.rate[r.par];
+    return 0;
+}
+
+// sets ok of the runs that converged; the others stalled (contraction per
+// pair worse than 0.5) or ran out of sweeps, cur then holds the last iterate.
+// The initial guess is the field plus the increment of the quantity's last
+// solve, when that solve converged on the same trajectory (the reference
+// starts from the field alone; both stop at the same residual test).  Three
+// FP64 buffers take part: the field x, read by the first pair and kept so
+// that each residual check also writes the increment, and the two iterate
+// buffers, the quantity's second buffer and its third or (large grids) kv[6].
+// The increment is kept in FP32: it only moves the start of the next solve,
+// which converges to the same residual test, and the check that writes it
+// and the first pair that reads it stream half the bytes for it.
 // The true residual costs about two thirds of a sweep pair, so it is
 // evaluated only where the solve may have converged: first after as many
 // pairs as the last solve of the same quantity and RK stage parity needed
@@ -764,64 +894,74 @@ static int copy_box(tb_ctx *c, double *dst, const double *src) {
 // from the observed contraction (at most 3 at a time: the contraction
 // improves as the sweeps go, a longer prediction overshoots).  The initial
 // residual is not evaluated (res0 = NaN).
-static int helm_gs_solve(tb_ctx *c, const HelmOp &H, double *x, const double *b, double rtol, int maxit, int &its,
-                         double &res0, double &res, double &bn, bool &ok) {
-    const int q = H.q;
-    double *ibuf = c->kv[5];
-    double rr, bb;
-    res0 = NAN;
-    res = NAN;
-    its = 0;
-    ok = false;
-    if (maxit < 1) return 0;
-    if (tb_helm_inc_alloc(c, q)) return -1;
-    HelmHistory &h = c->helm[q];
-    const bool field = x == c->f[TB_F_U + q];
-    const float *inc = (field && h.inc_ok) ? h.inc : nullptr;
-    h.inc_ok = false;   // the increment is overwritten by the first residual check
-    double *cur = h.buf, *alt = c->kv[6];
-    const int par = (int)(h.nsolve++ & 1u);
-    int chunk = h.sweeps[par] > 0 ? h.sweeps[par] : 2;
-    double prev = NAN, rate = h.rate[par];
-    const double *src = x;
-    while (!ok && its < maxit) {
-        const int m = chunk < maxit - its ? chunk : maxit - its;
-        if (gs_pairs(c, H, cur, alt, b, m, src, inc)) return -1;
-        src = nullptr;
-        inc = nullptr;
-        its += m;
-        if (helm_residual(c, H, cur, b, ibuf, rr, bb, field ? x : nullptr, field ? h.inc : nullptr)) return -1;
-        bn = sqrt(bb);
-        if (bn == 0.0) bn = 1.0;
-        res = sqrt(rr) / bn;
-        if (!(res == res)) break;
-        ok = res <= rtol;
-        if (ok) break;
-        if (prev == prev) rate = pow(res / prev, 1.0 / m);
-        prev = res;
-        if (!(rate > 0.0)) rate = 0.05;   // no estimate yet
-        if (!(rate < 0.5)) break;
-        const int need = (int)ceil(log(rtol / res) / log(rate));
-        chunk = need < 1 ? 1 : (need > 3 ? 3 : need);
+template <int N>
+static int gs_solve(tb_ctx *c, GsRun *run, int n, double rtol, int maxit) {
+    for (;;) {
+        GsRun *act[N];
+        int m = 0;
+        for (int a = 0; a < n; a++) {
+            GsRun &r = run[a];
+            if (r.done || r.its >= maxit) continue;
+            r.todo = r.chunk < maxit - r.its ? r.chunk : maxit - r.its;
+            act[m++] = &r;
+        }
+        if (m == 0) break;
+        if (gs_pairs<N>(c, act, m) || gs_check<N>(c, act, m)) return -1;
+        for (int a = 0; a < m; a++) {
+            GsRun &r = *act[a];
+            const double rr = c->hscal[S_SUB + 2 * a], bb = c->hscal[S_SUB + 2 * a + 1];
+            double bn = sqrt(bb);
+            if (bn == 0.0) bn = 1.0;
+            r.its += r.todo;
+            r.res = sqrt(rr) / bn;
+            r.ok = r.res <= rtol;
+            r.done = r.ok || !(r.res == r.res);
+            if (r.done) continue;
+            if (r.prev == r.prev) r.rate = pow(r.res / r.prev, 1.0 / r.todo);
+            r.prev = r.res;
+            if (!(r.rate > 0.0)) r.rate = 0.05;   // no estimate yet
+            if (!(r.rate < 0.5)) { r.done = true; continue; }
+            const int need = (int)ceil(log(rtol / r.res) / log(r.rate));
+            r.chunk = need < 1 ? 1 : (need > 3 ? 3 : need);
+        }
     }
-    if (ok) {
+    for (int a = 0; a < n; a++) {
+        GsRun &r = run[a];
+        if (!r.ok) continue;
         // one pair fewer next time when this residual shows it would have
         // sufficed at the last contraction
-        const double r1 = (rate > 0.0 && rate < 0.5) ? rate : 0.05;
-        h.sweeps[par] = (its > 1 && res / r1 <= rtol) ? its - 1 : its;
-        if (prev == prev) h.rate[par] = rate;
-    }
-    if (ok && field) {
-        // cur: the solution, h.inc: its increment over x (the iterates never
-        // write x, which is now free)
-        c->f[TB_F_U + q] = cur;
-        h.buf = alt;
-        c->kv[6] = x;
-        h.inc_ok = true;
-    } else if (copy_box(c, x, cur)) {
-        return -1;   // BiCGStab continues from x
+        const double r1 = (r.rate > 0.0 && r.rate < 0.5) ? r.rate : 0.05;
+        r.h.sweeps[r.par] = (r.its > 1 && r.res / r1 <= rtol) ? r.its - 1 : r.its;
+        if (r.prev == r.prev) r.h.rate[r.par] = r.rate;
     }
     return 0;
+}
+
+// The run's result into the context (with its concentration field selected):
+// the field takes the result's buffer, the second buffer the other
+// iterate's and the third one (or kv[6]) the old field's (no kernel or graph
+// keeps any of these pointers between calls).
+static int gs_end(tb_ctx *c, GsRun &r) {
+    const int q = r.q;
+    c->helm[q] = r.h;
+    if (!r.ok) return copy_box(c, r.x, r.cur);   // BiCGStab continues from x
+    c->f[TB_F_U + q] = r.cur;
+    c->helm[q].buf = r.alt;
+    if (r.spare) c->helm[q].spare = r.x;
+    else c->kv[6] = r.x;
+    c->helm[q].inc_ok = true;
+    return 0;
+}
+
+static void gs_stats(const GsRun &r, double ms, tb_solve_stats *st) {
+    if (!st) return;
+    st->iterations = r.its;
+    st->converged = 1;
+    st->fallback = 0;
+    st->vcycles = 0;
+    st->res0 = NAN;
+    st->res = r.res;
+    st->ms = ms;
 }
 
 // The smoother of tb_helmholtz_solve by itself: f_x <- `pairs` red-black
@@ -834,10 +974,16 @@ extern "C" int tb_helmholtz_gs_sweeps(tb_ctx *c, int q, double dt, int f_b, int 
         return -1;
     }
     tb_field_written(c, f_x);
-    HelmOp H = make_op(c, q, dt);
-    double *cur = c->f[f_x], *alt = c->kv[6];
-    if (gs_pairs(c, H, cur, alt, c->f[f_b], pairs)) return -1;
-    if (cur != c->f[f_x] && copy_box(c, c->f[f_x], cur)) return -1;
+    GsRun r, *one = &r;
+    r.q = q;
+    r.H = make_op(c, q, dt);
+    r.b = c->f[f_b];
+    gs_ib(c, r);
+    r.cur = c->f[f_x];
+    r.alt = c->kv[6];
+    r.todo = pairs;
+    if (gs_pairs<1>(c, &one, 1)) return -1;
+    if (r.cur != c->f[f_x] && copy_box(c, c->f[f_x], r.cur)) return -1;
     TB_CHECK(c, hipStreamSynchronize(c->s));
     return 0;
 }
@@ -956,40 +1102,14 @@ static int read_scalars(tb_ctx *c, int first, int count) { return tb_read_scalar
 // guess = the current field; stops at ||b - A x|| <= rtol ||b|| (PETSc's
 // default test relative to the right-hand side), checked on the true
 // residual at the end.
-extern "C" int tb_helmholtz_solve(tb_ctx *c, int q, double dt, tb_solve_stats *st) {
-    if (!c || q < 0 || q > 3) { if (c) c->err = "tb_helmholtz_solve: bad quantity"; return -1; }
-    HelmOp H = make_op(c, q, dt);
+// handover: 1 when the Gauss-Seidel sweeps stopped contracting (or ran out of
+// pairs) and this finishes the solve.
+static int bicgstab(tb_ctx *c, int q, const HelmOp &H, int handover, tb_solve_stats *st) {
     long n = c->d.ntot;
     double *x = c->f[TB_F_U + q], *b = c->f[TB_F_RHS_U + q];
     double *r = c->kv[0], *rh = c->kv[1], *p = c->kv[2], *v = c->kv[3], *sv = c->kv[4], *t = c->kv[5];
-    double rtol = c->cfg.helm_rtol;
-    int maxit = c->cfg.helm_maxit;
-    TB_CHECK(c, hipEventRecord(c->ev0, c->s));
-    // 1 when the Gauss-Seidel sweeps stopped contracting (or ran out of
-    // pairs) and BiCGStab finished the solve
-    int handover = 0;
-    if (c->helm_method == TB_HELM_GS) {
-        int gits = 0;
-        double g0 = 0.0, gres = 0.0, gbn = 1.0;
-        bool ok = false;
-        if (helm_gs_solve(c, H, x, b, rtol, maxit, gits, g0, gres, gbn, ok)) return -1;
-        if (ok) {
-            TB_CHECK(c, hipEventRecord(c->ev1, c->s));
-            if (tb_sync(c)) return -1;
-            if (st) {
-                st->iterations = gits;
-                st->converged = 1;
-                st->fallback = 0;
-                st->vcycles = 0;
-                st->res0 = g0;
-                st->res = gres;
-                st->ms = tb_elapsed_ms(c);
-            }
-            return 0;
-        }
-        // sweeps stalled: BiCGStab continues from the current x
-        handover = 1;
-    }
+    const double rtol = c->cfg.helm_rtol;
+    const int maxit = c->cfg.helm_maxit;
     c->helm[q].inc_ok = false;   // the increment is recorded by the Gauss-Seidel solve only
     if (helm_apply(c, H, x, t, true, 0) < 0) return -1;
     hipLaunchKernelGGL(k_bicg_init, dim3(VB), dim3(VT), 0, c->s, n, b, t, r, rh, p, v, c->red);
@@ -1042,4 +1162,72 @@ extern "C" int tb_helmholtz_solve(tb_ctx *c, int q, double dt, tb_solve_stats *s
         st->ms = tb_elapsed_ms(c);
     }
     return (tres <= rtol) ? 0 : 1;
+}
+
+extern "C" int tb_helmholtz_solve(tb_ctx *c, int q, double dt, tb_solve_stats *st) {
+    if (!c || q < 0 || q > 3) { if (c) c->err = "tb_helmholtz_solve: bad quantity"; return -1; }
+    const HelmOp H = make_op(c, q, dt);
+    TB_CHECK(c, hipEventRecord(c->ev0, c->s));
+    if (c->helm_method != TB_HELM_GS) return bicgstab(c, q, H, 0, st);
+    GsRun r;
+    if (gs_begin(c, q, H, r) || gs_solve<1>(c, &r, 1, c->cfg.helm_rtol, c->cfg.helm_maxit) || gs_end(c, r)) return -1;
+    if (!r.ok) return bicgstab(c, q, H, 1, st);
+    gs_stats(r, tb_elapsed_ms(c), st);
+    return 0;
+}
+
+// The predictor solves of a stage: u, v, w and every concentration field.
+// st[q]: their stats, field 0's for the concentration (a set's time is shared
+// out evenly).  Returns the worst of the solves' codes.
+int tb_helmholtz_all(tb_ctx *c, double dt, tb_solve_stats *st) {
+    const int sel = c->conc_sel;
+    const bool set = c->helm_method == TB_HELM_GS && c->d.ntot <= HELM_SET_POINTS;
+    int worst = 0, first = 0;   // concentration fields from `first` on are solved one by one
+    if (set) {
+        GsRun run[HELM_SET];
+        int n = 0;
+        TB_CHECK(c, hipEventRecord(c->ev0, c->s));
+        for (int q = 0; q < 3; q++, n++)
+            if (gs_begin(c, q, make_op(c, q, dt), run[n])) return -1;
+        // the IMMERSED rows of the concentration grid are those of one Pe at a time
+        tb_conc_sync(c);
+        bool same = true;
+        for (int f = 1; f < c->nconc; f++) same &= c->cs[f].p.pe == c->cs[0].p.pe;
+        if (c->nconc == 1 || same || c->nib[TB_Q_C] == 0)
+            for (; first < c->nconc; first++, n++) {
+                if (c->nconc > 1 && tb_conc_use(c, first)) return -1;
+                if (gs_begin(c, TB_Q_C, make_op(c, TB_Q_C, dt), run[n])) return -1;
+            }
+        if (gs_solve<HELM_SET>(c, run, n, c->cfg.helm_rtol, c->cfg.helm_maxit)) return -1;
+        const double ms = tb_elapsed_ms(c) / n;
+        for (int a = 0; a < n; a++) {
+            GsRun &r = run[a];
+            if (a >= 3 && c->nconc > 1 && tb_conc_use(c, r.field)) return -1;
+            tb_solve_stats s;
+            if (gs_end(c, r)) return -1;
+            if (r.ok) {
+                gs_stats(r, ms, &s);
+            } else {
+                const int rc = bicgstab(c, r.q, r.H, 1, &s);
+                if (rc < 0) return -1;
+                if (rc > worst) worst = rc;
+            }
+            if (a < 3 || r.field == 0) st[r.q] = s;
+        }
+    }
+    for (int q = 0; q < 3 && !set; q++) {
+        const int rc = tb_helmholtz_solve(c, q, dt, &st[q]);
+        if (rc < 0) return -1;
+        if (rc > worst) worst = rc;
+    }
+    for (int f = first; f < c->nconc; f++) {
+        if (c->nconc > 1 && tb_conc_use(c, f)) return -1;
+        tb_solve_stats s;
+        const int rc = tb_helmholtz_solve(c, TB_Q_C, dt, &s);
+        if (rc < 0) return -1;
+        if (rc > worst) worst = rc;
+        if (f == 0) st[TB_Q_C] = s;
+    }
+    if (c->nconc > 1 && tb_conc_use(c, sel)) return -1;
+    return worst;
 }

@@ -1520,8 +1520,7 @@ static int residual(tb_ctx *c, const PoisCtx &P, bool neumann, const double *x, 
     hipLaunchKernelGGL(k_pois_km<1>, ktiles_grid(P.kt), tiles_block(), 0, c->s, neumann ? P.Pn : P.Pp, x, b, r, r32,
                        c->red, P.kt);
     TB_LAUNCH_CHECK(c);
-    if (tb_reduce_finish(c, (int)P.nblk, 3, S_RES)) return -1;
-    if (read_s(c, S_RES, 3)) return -1;
+    if (tb_reduce_read(c, (int)P.nblk, 3, S_RES)) return -1;
     rr = c->hscal[S_RES];
     bb = c->hscal[S_RES + 1];   // x.b in S_RES + 2
     return 0;
@@ -1596,8 +1595,7 @@ static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double
             inner++;
             if (inner >= 200) break;
             if (its - its0 > skip && its < maxit) {
-                if (tb_reduce_finish(c, PB, 1, S_RR)) return -1;
-                if (read_s(c, S_RR, 1)) return -1;
+                if (tb_reduce_read(c, PB, 1, S_RR)) return -1;
                 double rrel = sqrt(c->hscal[S_RR]) / bn;
                 if (!(rrel == rrel)) { c->err = "Poisson CG produced NaN"; return -1; }
                 if (rrel <= 0.5 * rtol) break;

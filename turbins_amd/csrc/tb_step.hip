@@ -9,6 +9,7 @@
 #include "tb_common.h"
 
 int tb_eno_rhs_async(tb_ctx *c, double dt, bool store_conv);
+int tb_helmholtz_all(tb_ctx *c, double dt, tb_solve_stats *st);
 
 extern "C" int tb_step(tb_ctx *c, double dt, tb_step_stats *st) {
     if (!c || !(dt > 0.0)) { if (c) c->err = "tb_step: bad argument"; return -1; }
@@ -18,7 +19,6 @@ extern "C" int tb_step(tb_ctx *c, double dt, tb_step_stats *st) {
     TB_CHECK(c, hipEventRecord(e0, c->s));
     int worst = 0;
     if (tb_store_old(c)) return -1;
-    const int sel = c->conc_sel;
     for (int stage = 0; stage < 2; stage++) {
         // the convective outflow condition from the stage-start fields
         // (Outflow_impose_convective_boundary; its place in the unpublished
@@ -30,23 +30,12 @@ extern "C" int tb_step(tb_ctx *c, double dt, tb_step_stats *st) {
         // ENO and the right-hand sides (tb_eno_conv + tb_set_rhs) in one
         // pass; the convective terms stay in registers
         if (tb_eno_rhs_async(c, dt, false)) return -1;
-        for (int q = 0; q < 3; q++) {
-            int rc = tb_helmholtz_solve(c, q, dt, &loc.helm[stage][q]);
-            if (rc < 0) return -1;
-            if (rc > worst) worst = rc;
-        }
-        // every concentration field; the stats report field 0
-        for (int n = 0; n < c->nconc; n++) {
-            if (c->nconc > 1 && tb_conc_use(c, n)) return -1;
-            tb_solve_stats cst;
-            int rc = tb_helmholtz_solve(c, TB_Q_C, dt, &cst);
-            if (rc < 0) return -1;
-            if (rc > worst) worst = rc;
-            if (n == 0) loc.helm[stage][TB_Q_C] = cst;
-        }
-        if (c->nconc > 1 && tb_conc_use(c, sel)) return -1;
+        // u, v, w and every concentration field; the stats report field 0
+        int rc = tb_helmholtz_all(c, dt, loc.helm[stage]);
+        if (rc < 0) return -1;
+        if (rc > worst) worst = rc;
         if (tb_poisson_rhs(c, dt)) return -1;
-        int rc = tb_poisson_solve(c, &loc.pois[stage]);
+        rc = tb_poisson_solve(c, &loc.pois[stage]);
         if (rc < 0) return -1;
         if (rc > worst) worst = rc;
         if (tb_project(c, dt)) return -1;
