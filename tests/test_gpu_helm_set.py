@@ -1,4 +1,4 @@
-"""On small grids a step solves the predictor systems of all quantities as one
+"""A step solves the predictor systems of all quantities as one
 set of Gauss-Seidel solves.  The same steps with BiCGStab, which solves them
 one by one, stop at the same residual test (1e-13 of the right-hand side, rows
 dominated by 1/dt, so the solutions agree to a few 1e-13 per solve); the

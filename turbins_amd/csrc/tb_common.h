@@ -278,7 +278,7 @@ struct HelmHistory {
     double rate[2] = {0.0, 0.0};
     unsigned nsolve = 0;
     double *buf = nullptr;       // second iterate buffer of the solves (allocated on first use, with inc)
-    double *spare = nullptr;     // third one, on the grids whose quantities are solved as one set
+    double *spare = nullptr;     // third one, where the quantities are solved as one set
     float *inc = nullptr;        // the last solve's increment x_new - x_start, in FP32
     bool inc_ok = false;         // inc belongs to this field's current trajectory
 };
@@ -371,6 +371,7 @@ struct tb_ctx {
     hipGraphExec_t vc_exec = nullptr;
     int helm_method = TB_HELM_GS;    // Helmholtz solver
     HelmHistory helm[4];         // Gauss-Seidel history of u, v, w and the selected concentration field
+    bool helm_sets = true;       // cleared when there is no memory for the sets' third buffers
     double ir_floor = 1e-5;      // tb_set_mixed_inner: kept for callers, the direct inner solve has no target
     int ir_maxit = 40;           // FP32 solves per refinement pass (0: none)
     int pcg_its = 0;             // iterations of the last FP64 solve
@@ -486,7 +487,8 @@ int tb_open_store_old(tb_ctx *c);
 int tb_open_rk_average(tb_ctx *c, double old_frac, double new_frac);
 int tb_outflow_async(tb_ctx *c, double dt);   // tb_outflow_convective without the final sync
 void tb_open_free(tb_ctx *c);
-int tb_helm_inc_alloc(tb_ctx *c, int q, bool spare);   // the iterate and increment buffers of quantity q (once)
+int tb_helm_inc_alloc(tb_ctx *c, int q);   // the increment buffer of quantity q (once)
+bool tb_helm_spares(tb_ctx *c);            // third iterate buffers of all quantities; false: no memory for them
 void tb_free_deposits(tb_ctx *c, int first);
 int tb_ib_rows(tb_ctx *c, int q);
 

@@ -68,14 +68,33 @@ static int dev_alloc(tb_ctx *c, void **p, size_t bytes) {
     return 0;
 }
 
-int tb_helm_inc_alloc(tb_ctx *c, int q, bool spare) {
+int tb_helm_inc_alloc(tb_ctx *c, int q) {
     HelmHistory &h = c->helm[q];
-    if (h.buf && h.inc && (h.spare || !spare)) return 0;
+    if (h.buf && h.inc) return 0;
     h.inc_ok = false;
-    if (spare && !h.spare && dev_alloc(c, (void **)&h.spare, sizeof(double) * (size_t)c->d.ntot)) return -1;
     if (!h.buf && dev_alloc(c, (void **)&h.buf, sizeof(double) * (size_t)c->d.ntot)) return -1;
     if (!h.inc && dev_alloc(c, (void **)&h.inc, sizeof(float) * (size_t)c->d.ntot)) return -1;
     return 0;
+}
+
+bool tb_helm_spares(tb_ctx *c) {
+    tb_conc_sync(c);
+    double **p[3 + TB_NCONC_MAX];
+    int n = 0;
+    for (int q = 0; q < 3; q++) p[n++] = &c->helm[q].spare;
+    for (int f = 0; f < c->nconc; f++) p[n++] = &c->cs[f].h.spare;
+    for (int a = 0; a < n && c->helm_sets; a++)
+        if (!*p[a] && dev_alloc(c, (void **)p[a], sizeof(double) * (size_t)c->d.ntot)) {
+            (void)hipGetLastError();
+            for (int b = 0; b < n; b++) {
+                if (*p[b]) c->bytes -= (int64_t)(sizeof(double) * (size_t)c->d.ntot);
+                hipFree(*p[b]);
+                *p[b] = nullptr;
+            }
+            c->helm_sets = false;
+        }
+    c->helm[TB_Q_C] = c->cs[c->conc_sel].h;
+    return c->helm_sets;
 }
 
 double tb_elapsed_ms(tb_ctx *c) {

@@ -33,10 +33,10 @@ struct HelmOp {
     int open_w, open_e;
 };
 
-// What the Gauss-Seidel kernels need of one quantity's solve.  On small grids
-// u, v, w and the concentration fields are solved side by side, one grid row
-// (blockIdx.y) each: their systems are independent, and one quantity's launches
-// leave most of the chip idle there.
+// What the Gauss-Seidel kernels need of one quantity's solve.  u, v, w and
+// the concentration fields are solved side by side, one grid row (blockIdx.y)
+// each: their systems are independent, and one quantity's launches leave much
+// of the chip idle.
 struct GsView {
     HelmOp H;
     const double *b, *x0;          // right-hand side; the field the solve started from
@@ -851,13 +851,17 @@ static int copy_box(tb_ctx *c, double *dst, const double *src) {
 }
 
 // Grids up to this size have all their quantities solved as one set, each with
-// a third iterate buffer of its own.
-constexpr long HELM_SET_POINTS = 1L << 20;
+// a third iterate buffer of its own.  Four quantities' solves of a step, one by
+// one and as a set: 0.59 and 0.24 ms at 64x16x16, 1.00 / 0.58 at 192x64x64,
+// 1.59 / 0.86 at 256x128x64, 3.37 / 2.93 at 512x128x128 and 6.87 / 6.58 at
+// 512x256x128, where a launch's last round of blocks is what is left to share;
+// beyond, that is not worth the memory.
+constexpr long HELM_SET_POINTS = 1L << 25;
 
 // the run of quantity q (the selected concentration field's for TB_Q_C)
-static int gs_begin(tb_ctx *c, int q, const HelmOp &H, GsRun &r) {
-    r.spare = c->d.ntot <= HELM_SET_POINTS;
-    if (tb_helm_inc_alloc(c, q, r.spare)) return -1;
+static int gs_begin(tb_ctx *c, int q, const HelmOp &H, bool spare, GsRun &r) {
+    if (tb_helm_inc_alloc(c, q)) return -1;
+    r.spare = spare;
     r.q = q;
     r.field = c->conc_sel;
     r.H = H;
@@ -883,7 +887,7 @@ static int gs_begin(tb_ctx *c, int q, const HelmOp &H, GsRun &r) {
 // starts from the field alone; both stop at the same residual test).  Three
 // FP64 buffers take part: the field x, read by the first pair and kept so
 // that each residual check also writes the increment, and the two iterate
-// buffers, the quantity's second buffer and its third or (large grids) kv[6].
+// buffers, the quantity's second buffer and its third (in a set) or kv[6].
 // The increment is kept in FP32: it only moves the start of the next solve,
 // which converges to the same residual test, and the check that writes it
 // and the first pair that reads it stream half the bytes for it.
@@ -1170,7 +1174,7 @@ extern "C" int tb_helmholtz_solve(tb_ctx *c, int q, double dt, tb_solve_stats *s
     TB_CHECK(c, hipEventRecord(c->ev0, c->s));
     if (c->helm_method != TB_HELM_GS) return bicgstab(c, q, H, 0, st);
     GsRun r;
-    if (gs_begin(c, q, H, r) || gs_solve<1>(c, &r, 1, c->cfg.helm_rtol, c->cfg.helm_maxit) || gs_end(c, r)) return -1;
+    if (gs_begin(c, q, H, false, r) || gs_solve<1>(c, &r, 1, c->cfg.helm_rtol, c->cfg.helm_maxit) || gs_end(c, r)) return -1;
     if (!r.ok) return bicgstab(c, q, H, 1, st);
     gs_stats(r, tb_elapsed_ms(c), st);
     return 0;
@@ -1181,14 +1185,14 @@ extern "C" int tb_helmholtz_solve(tb_ctx *c, int q, double dt, tb_solve_stats *s
 // out evenly).  Returns the worst of the solves' codes.
 int tb_helmholtz_all(tb_ctx *c, double dt, tb_solve_stats *st) {
     const int sel = c->conc_sel;
-    const bool set = c->helm_method == TB_HELM_GS && c->d.ntot <= HELM_SET_POINTS;
+    const bool set = c->helm_method == TB_HELM_GS && c->d.ntot <= HELM_SET_POINTS && tb_helm_spares(c);
     int worst = 0, first = 0;   // concentration fields from `first` on are solved one by one
     if (set) {
         GsRun run[HELM_SET];
         int n = 0;
         TB_CHECK(c, hipEventRecord(c->ev0, c->s));
         for (int q = 0; q < 3; q++, n++)
-            if (gs_begin(c, q, make_op(c, q, dt), run[n])) return -1;
+            if (gs_begin(c, q, make_op(c, q, dt), true, run[n])) return -1;
         // the IMMERSED rows of the concentration grid are those of one Pe at a time
         tb_conc_sync(c);
         bool same = true;
@@ -1196,7 +1200,7 @@ int tb_helmholtz_all(tb_ctx *c, double dt, tb_solve_stats *st) {
         if (c->nconc == 1 || same || c->nib[TB_Q_C] == 0)
             for (; first < c->nconc; first++, n++) {
                 if (c->nconc > 1 && tb_conc_use(c, first)) return -1;
-                if (gs_begin(c, TB_Q_C, make_op(c, TB_Q_C, dt), run[n])) return -1;
+                if (gs_begin(c, TB_Q_C, make_op(c, TB_Q_C, dt), true, run[n])) return -1;
             }
         if (gs_solve<HELM_SET>(c, run, n, c->cfg.helm_rtol, c->cfg.helm_maxit)) return -1;
         const double ms = tb_elapsed_ms(c) / n;
