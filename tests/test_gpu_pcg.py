@@ -1,0 +1,47 @@
+"""The FP64 conjugate gradient iteration where its launches differ: boxes of
+the blocked smoother with every sum added up by its consumers, more partial
+sums than that (the sweeps of a finest level without boxes), two passes for
+the direction and the operator above a million cells, and a single block.
+
+A random right-hand side of zero mean is solved from zero; the oracle's
+residual of the result is the tolerance up to its summation order.  A
+tolerance out of FP64's reach ends with status 1 and the best iterate: the
+residual's own rounding is about 1e-16 times the row sum times the solution
+over the right-hand side, below 1e-11 here."""
+import numpy as np
+import pytest
+
+from turbins_amd import Solver, abi, workload as W
+
+pytestmark = pytest.mark.gpu
+
+import oracle  # noqa: E402  (checker only)
+
+RTOL = 1e-10
+
+
+@pytest.mark.parametrize("nx,ny,nz,lx", [(8, 8, 8, 1.0), (66, 18, 16, 8.0), (96, 64, 66, 2.0), (128, 96, 100, 2.0)])
+def test_plain_poisson(nx, ny, nz, lx):
+    print("pcg", nx, ny, nz, flush=True)
+    c = W.case("lock64", nx=nx, ny=ny, nz=nz, lx=lx, ly=1.0, lz=1.0)
+    cfg = W.config_for(c, pois_rtol=RTOL, pois_mode=abi.POIS_FP64_PCG)
+    g, o = Solver(cfg), oracle.Oracle(cfg)
+    b = np.zeros((nz + 1, ny + 1, nx + 1))
+    r = np.random.default_rng(nx + ny + nz).standard_normal((nz, ny, nx))
+    b[:nz, :ny, :nx] = r - r.mean()
+    nb = np.linalg.norm(b)
+    for rtol in (RTOL, RTOL, 1e-18):   # the second solve reads back its residual later
+        g.set_poisson_mode(abi.POIS_FP64_PCG, rtol)
+        g.upload("PHI", np.zeros(g.NT))
+        g.upload("PRHS", b)
+        st = g.poisson_solve()
+        x = g.download("PHI")
+        res = np.linalg.norm(b.ravel() - o.poisson_apply(x)) / nb
+        print("rtol", rtol, "its", st.iterations, "res", st.res, "oracle", res, flush=True)
+        if rtol == RTOL:
+            assert st.converged and res <= RTOL * (1 + 1e-6) and st.iterations <= 30
+        else:
+            assert not st.converged and res <= 1e-11 and np.isfinite(x).all()
+        assert x.reshape(b.shape)[nz - 1, ny - 1, nx - 1] == 0.0
+    g.close()
+    o.close()

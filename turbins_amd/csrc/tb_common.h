@@ -376,7 +376,7 @@ struct tb_ctx {
     int ir_maxit = 40;           // FP32 solves per refinement pass (0: none)
     int pcg_its = 0;             // iterations of the last FP64 solve
     // partial sums r . z, sum z, sum r left in red by the V-cycle's last
-    // finest-level pair; 0: that level has no pairs
+    // smoothing launch of the finest level; 0: it left none
     int vc_dot_blocks = 0;
     int mg_pre0 = 0, mg_post0 = 0;   // FP64 sweeps on the finest level per V-cycle side; 0: cfg.mg_pre / cfg.mg_post
     bool mg_blocked = true;      // small finest levels smoothed by one blocked launch per V-cycle side
@@ -459,7 +459,7 @@ enum {
 
 // internal entry points shared between translation units
 int tb_geometry_run(tb_ctx *c, const double *h_xz);
-int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0);
+int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0, int first_array = 0);
 int tb_reduce_read(tb_ctx *c, int nblocks, int nslots, int slot0, int groups = 1, long gstride = 0);
 int tb_read_scalars(tb_ctx *c, int first, int count);
 int tb_wait_published(tb_ctx *c, unsigned long long want);

@@ -160,8 +160,10 @@ __global__ void __launch_bounds__(256) k_pois_km(PoisOp P, const double *__restr
     block_sum<3>(acc, sh);
     if (threadIdx.x == 0 && threadIdx.y == 0) {
         part[blockIdx.x] = acc[0];
-        part[RED_MAX_BLOCKS + blockIdx.x] = acc[1];
-        part[2 * RED_MAX_BLOCKS + blockIdx.x] = acc[2];
+        if (RESID) {
+            part[RED_MAX_BLOCKS + blockIdx.x] = acc[1];
+            part[2 * RED_MAX_BLOCKS + blockIdx.x] = acc[2];
+        }
     }
 }
 
@@ -839,7 +841,9 @@ __device__ inline void block_cells(int nx, int ny, int nz, F f) {
 // box grown by 2*NP - m cells, which is every cell a later half sweep of the
 // box reads.  ZERO: the sweeps start from x = 0 and read only b (the
 // pre-smoother).  PROL: the starting iterate is src + P xc, the coarse
-// level's correction prolonged on the fly (the post-smoother).  Every cell
+// level's correction prolonged on the fly (the post-smoother), and the box's
+// partial sums of b . x, x and b go to part (r . z, sum z and sum r of the
+// Krylov method around the cycle).  Every cell
 // value is formed by the expressions of rb_value and prolong_sum, so the
 // result equals the launch-per-half-sweep sequence bit for bit.
 constexpr int BLK_THREADS = 1024;
@@ -862,7 +866,7 @@ struct BlkShape {
 template <typename T, int NP, bool ZERO, bool PROL, int FIRST>
 __global__ void __launch_bounds__(BLK_THREADS) k_rbgs_blk(LV<T> L, const T *__restrict__ src, const T *__restrict__ b,
                                                           T *__restrict__ dst, BlkShape S, LV<T> C, int cx, int cy,
-                                                          int cz, const T *__restrict__ xc) {
+                                                          int cz, const T *__restrict__ xc, double *part) {
     extern __shared__ double smem_blk[];
     constexpr int H = 2 * NP;
     const int rx = S.bx + 2 * H, ry = S.by + 2 * H, rz = S.bz + 2 * H;
@@ -933,10 +937,24 @@ __global__ void __launch_bounds__(BLK_THREADS) k_rbgs_blk(LV<T> L, const T *__re
         });
         __syncthreads();
     }
+    double acc[3] = {0.0, 0.0, 0.0};
     block_cells(min(S.bx, L.nx - ox), min(S.by, L.ny - oy), min(S.bz, L.nz - oz), [&](int a, int e, int f) {
         const int i = ox + a, j = oy + e, k = oz + f;
-        dst[lidx(L, i, j, k)] = xs[((k - gz) * ry + (j - gy)) * rx + (i - gx)];
+        const int q = ((k - gz) * ry + (j - gy)) * rx + (i - gx);
+        const T v = xs[q];
+        dst[lidx(L, i, j, k)] = v;
+        if (PROL) {
+            acc[0] += (double)bs[q] * (double)v;
+            acc[1] += (double)v;
+            acc[2] += (double)bs[q];
+        }
     });
+    if (PROL) {
+        __syncthreads();   // the box is read; its LDS takes the wave sums
+        block_sum<3>(acc, smem_blk);
+        if (threadIdx.x == 0)
+            for (int a = 0; a < 3; a++) part[a * RED_MAX_BLOCKS + lt] = acc[a];
+    }
 }
 
 // LDS bytes of k_rbgs_blk for box (bx, by, bz) on level L (coarsened by its
@@ -1198,13 +1216,14 @@ static void launch_blk_np(tb_ctx *c, const dim3 &grid, int lds, int kind, const 
     const dim3 blk(BLK_THREADS);
     if (kind == BLK_ZERO)
         hipLaunchKernelGGL((k_rbgs_blk<double, NP, true, false, 0>), grid, blk, lds, c->s, lv, src, b, dst, S, cv,
-                           L.cx, L.cy, L.cz, xc);
+                           L.cx, L.cy, L.cz, xc, nullptr);
     else
         hipLaunchKernelGGL((k_rbgs_blk<double, NP, false, true, 1>), grid, blk, lds, c->s, lv, src, b, dst, S, cv,
-                           L.cx, L.cy, L.cz, xc);
+                           L.cx, L.cy, L.cz, xc, c->red);
 }
 
-static void launch_blk(tb_ctx *c, int l, int np, int kind, const double *src, double *dst, const double *xc) {
+// returns the number of boxes
+static int launch_blk(tb_ctx *c, int l, int np, int kind, const double *src, double *dst, const double *xc) {
     const Level &L = c->lev[l];
     const LV<double> lv = lv_of<double>(L), cv = lv_of<double>(c->lev[l + 1]);
     const double *b = L.b64;
@@ -1214,6 +1233,7 @@ static void launch_blk(tb_ctx *c, int l, int np, int kind, const double *src, do
     const dim3 grid((unsigned)(S.per_xcd * NXCD));
     if (np == 1) launch_blk_np<1>(c, grid, lds, kind, lv, src, b, dst, S, cv, L, xc);
     else launch_blk_np<2>(c, grid, lds, kind, lv, src, b, dst, S, cv, L, xc);
+    return S.nb;
 }
 
 // the blocked smoother serves a finest level of at most BLK_MAX_CELLS cells,
@@ -1304,7 +1324,7 @@ static int vcycle_level(tb_ctx *c, int l) {
         TB_PROF(c, TB_K_MG_TRANSFER, resid_restrict(c, l, B.r, c->kv[5]));
         TB_LAUNCH_CHECK(c);
         if (vcycle_level(c, l + 1)) return -1;
-        TB_PROF(c, kid, launch_blk(c, l, post, BLK_PROL, B.r, B.x, xc));
+        TB_PROF(c, kid, c->vc_dot_blocks = launch_blk(c, l, post, BLK_PROL, B.r, B.x, xc));
         TB_LAUNCH_CHECK(c);
         return 0;
     }
@@ -1406,13 +1426,180 @@ extern "C" int tb_set_graphs(tb_ctx *c, int on) {
 constexpr int PB = 1024;
 constexpr int PT = 256;
 
+// Up to this many partial sums are added up by every block that needs the
+// total instead of a launch of its own (5 us and a gap against about 1 us of
+// loads from L2 at 512).
+constexpr int SUM_INLINE = 512;
+
+// the totals of nb partial sums of NV of red's arrays in every thread
+// (a 256-thread block; sh: NV * 16 doubles)
+template <int NV>
+__device__ inline void inline_sum(const double *red, int nb, double (&v)[NV], double *sh) {
+#pragma unroll
+    for (int a = 0; a < NV; a++) {
+        v[a] = 0.0;
+        for (int b = threadIdx.y * blockDim.x + threadIdx.x; b < nb; b += 256) v[a] += red[a * (long)RED_MAX_BLOCKS + b];
+    }
+    block_sum<NV>(v, sh);
+    if (threadIdx.x == 0 && threadIdx.y == 0)
+#pragma unroll
+        for (int a = 0; a < NV; a++) sh[a * 16] = v[a];
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < NV; a++) v[a] = sh[a * 16];
+    __syncthreads();   // sh is free again
+}
+
+// red's array of the partial sums of p . q: blocks of the kernel that writes
+// it may still read the first three
+constexpr int PQ_ARRAY = 3;
+
+// beta of the direction update p = (z - mean z) + beta p from the sums of
+// r . z, z and r: rz_new / rz_old with rz_new = r . (z - mean z), stored in the
+// scalar slot rz_new (another one than rz_old, which every block reads).  The
+// V-cycle's output has an arbitrary mean and the operator does not see it:
+// left in, it lets the rounding of r's own mean into beta, and solves whose
+// right-hand side is small stagnated (200 iterations instead of 11 at
+// 64x16x16).
+__device__ inline void pcg_beta(const double (&sums)[3], double *s, int rz_old, int rz_new, bool first, double ncell,
+                                bool store, double &mean, double &beta) {
+    mean = sums[1] / ncell;
+    const double rzn = sums[0] - mean * sums[2];
+    beta = first || s[rz_old] == 0.0 ? 0.0 : rzn / s[rz_old];
+    if (store) s[rz_new] = rzn;
+}
+
+// the same by one block into the slots S_MEAN and S_BETA, for more than
+// SUM_INLINE partial sums; the many blocks of a large grid then start from two
+// loads (with the totals' loads and the divisions in each block the update
+// below took 107 us at 512x128x128)
+__global__ void __launch_bounds__(1024) k_pcg_beta(const double *__restrict__ part, int nb, double *s, int rz_old,
+                                                   int rz_new, int first, double ncell) {
+    __shared__ double sh[48];
+    double v[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+        for (int b = threadIdx.x; b < nb; b += 1024) v[a] += part[a * (long)RED_MAX_BLOCKS + b];
+    block_sum<3>(v, sh);
+    if (threadIdx.x != 0) return;
+    double mean, beta;
+    pcg_beta(v, s, rz_old, rz_new, first != 0, ncell, true, mean, beta);
+    s[S_MEAN] = mean;
+    s[S_BETA] = beta;
+}
+
+// The direction update on the cells, in place (no p term when first), from
+// S_MEAN and S_BETA
+__global__ void __launch_bounds__(256) k_pcg_p(Dims d, const double *__restrict__ z, double *__restrict__ p,
+                                               const double *__restrict__ s, int first, Tiles t) {
+    const double mean = s[S_MEAN], beta = s[S_BETA];
+    int i, j, k;
+    if (!tile_point(t, i, j, k)) return;
+    const long id = gidx(d, i, j, k);
+    const double v = z[id] - mean;
+    p[id] = first ? v : v + beta * p[id];
+}
+
+// Cells up to which the direction update and the operator are one pass: it
+// forms each neighbour's p again, twice the operator's loads, for a launch
+// fewer.  Steps with the sums added up in place, fused and in two passes: 1.34
+// and 1.49 ms at 64x16x16, 2.28 / 2.36 at 128x64x32, 2.85 / 2.87 at 192x64x64,
+// 8.20 / 8.05 at 512x128x64, 13.08 / 12.94 at 512x128x128.
+constexpr long PCG_FUSED_CELLS = 1L << 20;
+
+// The direction update and the operator in one pass:
+// p = (z - mean z) + beta po on the cells (0 on the half-cell planes; no po
+// term when FIRST), q = A p, partial p . q.  A neighbour's p is formed from z
+// and po by the same expression; po and p are two buffers.
+template <bool FIRST, bool INLINE>
+__global__ void __launch_bounds__(256) k_pcg_pa(PoisOp P, const double *__restrict__ z, const double *__restrict__ po,
+                                                double *__restrict__ p, double *__restrict__ q, int nsum, double *s,
+                                                int rz_old, int rz_new, double ncell, double *red, KTiles t) {
+    __shared__ double sh[48];
+    double mean, beta;
+    if (INLINE) {
+        double sums[3];
+        inline_sum<3>(red, nsum, sums, sh);
+        pcg_beta(sums, s, rz_old, rz_new, FIRST, ncell, blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0, mean,
+                 beta);
+    } else {
+        mean = s[S_MEAN];
+        beta = s[S_BETA];
+    }
+    double acc[1] = {0.0};
+    int i, j, k0, k1;
+    bool act;
+    ktile_column(t, i, j, k0, k1, act);
+    if (act) {
+        const Dims &d = P.d;
+        const GridDev &g = P.g;
+        const int NI = d.NX - 1, NJ = d.NY - 1, NK = d.NZ - 1;
+        const bool bnd_col = (i == NI) || (j == NJ);
+        const double Cx = P.Cx, Cy = P.Cy, Cz = P.Cz;
+        const int ip1 = i + 1 <= NI ? i + 1 : NI, jp1 = j + 1 <= NJ ? j + 1 : NJ;
+        const double mpx = g.mxc[i], mex = g.mxu[ip1], mwx = g.mxu[i];
+        const double mpy = g.myc[j], mny = g.myv[jp1], msy = g.myv[j];
+        const double axy = -Cx * mpx * (mex + mwx) - Cy * mpy * (mny + msy);
+        const double aw = Cx * mpx * mwx, ae = Cx * mpx * mex, an = Cy * mpy * mny, as = Cy * mpy * msy;
+        const bool hs = j > 0, hw = i > 0, he = i < NI - 1, hn = j < NJ - 1;
+        // absent neighbours are clamped to the point itself (zero coefficient
+        // below), so all loads are issued unconditionally
+        const long os = hs ? d.px : 0, on = hn ? d.px : 0, ow = hw ? 1 : 0, oe = he ? 1 : 0;
+        auto dir = [&](long e) {
+            const double v = z[e] - mean;
+            return FIRST ? v : v + beta * po[e];
+        };
+        long id = gidx(d, i, j, k0);
+        double xm = dir(id - ((k0 > 0) ? d.plane : 0)), xc = dir(id);
+        for (int k = k0; k < k1; k++) {
+            const double xp = dir(id + ((k + 1 < NK) ? d.plane : 0));
+            const double xs = dir(id - os), xw = dir(id - ow), xe = dir(id + oe), xn = dir(id + on);
+            if (bnd_col || k == NK) {
+                p[id] = 0.0;
+                st_stream(&q[id], 0.0);
+            } else {
+                const double mpz = g.mzc[k], mfz = g.mzw[k + 1], mbz = g.mzw[k];
+                double ap = axy - Cz * mpz * (mbz + mfz);
+                const double ab = Cz * mpz * mbz, af = Cz * mpz * mfz;
+                const bool hb = k > 0, hf = k < NK - 1;
+                if (!hb) ap += ab;
+                if (!hs) ap += as;
+                if (!hw) ap += aw;
+                if (!he) ap += ae;
+                if (!hn) ap += an;
+                if (!hf) ap += af;
+                double r = 0.0;
+                r = hb ? r + ab * xm : r;
+                r = hs ? r + as * xs : r;
+                r = hw ? r + aw * xw : r;
+                r += ap * xc;
+                r = he ? r + ae * xe : r;
+                r = hn ? r + an * xn : r;
+                r = hf ? r + af * xp : r;
+                p[id] = xc;
+                st_stream(&q[id], r);
+                acc[0] += xc * r;
+            }
+            xm = xc;
+            xc = xp;
+            id += d.plane;
+        }
+    }
+    block_sum<1>(acc, sh);
+    if (threadIdx.x == 0 && threadIdx.y == 0) red[PQ_ARRAY * (long)RED_MAX_BLOCKS + blockIdx.x] = acc[0];
+}
+
 // x += alpha p ; r -= alpha q ; partial r.r      (alpha = rz / pq; 0 where the
 // direction vanishes, r then being a constant the operator cannot reduce)
-__global__ void k_pcg_xr(long n, double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
-                         const double *__restrict__ q, const double *__restrict__ s, int rz, double *part) {
+template <bool INLINE>
+__global__ void __launch_bounds__(PT) k_pcg_xr(long n, double *__restrict__ x, double *__restrict__ r,
+                                               const double *__restrict__ p, const double *__restrict__ q, int nsum,
+                                               const double *__restrict__ s, int rz, double *red) {
     __shared__ double sh[16];
-    const double pq = s[S_PQ], alpha = pq == 0.0 ? 0.0 : s[rz] / pq;
-    double acc[1] = {0.0};
+    double acc[1];
+    if (INLINE) inline_sum<1>(red + PQ_ARRAY * (long)RED_MAX_BLOCKS, nsum, acc, sh);
+    const double pq = INLINE ? acc[0] : s[S_PQ], alpha = pq == 0.0 ? 0.0 : s[rz] / pq;
+    acc[0] = 0.0;
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         x[i] += alpha * p[i];
         double ri = r[i] - alpha * q[i];
@@ -1420,7 +1607,7 @@ __global__ void k_pcg_xr(long n, double *__restrict__ x, double *__restrict__ r,
         acc[0] += ri * ri;
     }
     block_sum<1>(acc, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
+    if (threadIdx.x == 0) red[blockIdx.x] = acc[0];
 }
 
 // partial sums of r . z, z and r
@@ -1436,26 +1623,6 @@ __global__ void k_pcg_rz(long n, const double *__restrict__ r, const double *__r
     block_sum<3>(acc, sh);
     if (threadIdx.x == 0)
         for (int a = 0; a < 3; a++) part[a * RED_MAX_BLOCKS + blockIdx.x] = acc[a];
-}
-
-// p = (z - mean z) + beta p on the cells, beta = rz_new / rz_old (no p term
-// when first), rz_new = r . (z - mean z) from the sums in S_TMP0..2 (r . z,
-// sum z, sum r), stored in the scalar slot rz_new (another one than rz_old,
-// which every block reads).  The V-cycle's output has an arbitrary mean and
-// the operator does not see it: left in, it lets the rounding of r's own mean
-// into beta, and solves whose right-hand side is small stagnated (200
-// iterations instead of 11 at 64x16x16).
-__global__ void __launch_bounds__(256) k_pcg_p(Dims d, const double *__restrict__ z, double *__restrict__ p, double *s,
-                                               int rz_old, int rz_new, int first, double ncell, Tiles t) {
-    const double mean = s[S_TMP0 + 1] / ncell;
-    const double rzn = s[S_TMP0] - mean * s[S_TMP0 + 2];
-    const double beta = first || s[rz_old] == 0.0 ? 0.0 : rzn / s[rz_old];
-    if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) s[rz_new] = rzn;
-    int i, j, k;
-    if (!tile_point(t, i, j, k)) return;
-    const long id = gidx(d, i, j, k);
-    const double v = z[id] - mean;
-    p[id] = first ? v : v + beta * p[id];
 }
 
 // x -= x[corner] on non-boundary cells ; boundary entries set to 0
@@ -1537,13 +1704,14 @@ constexpr int PCG_SKIP_MAX = 16;
 static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double bn, double rtol, int maxit,
                  int &its, int &vcy, double &res, const double *rr_known) {
     long n = c->d.ntot;
-    double *r = c->kv[0], *z = c->kv[1], *p = c->kv[2], *q = c->kv[3];
+    double *r = c->kv[0], *z = c->kv[1], *p = c->kv[2], *q = c->kv[3], *po = c->kv[6];
     const double ncell = (double)c->ncx * c->ncy * c->ncz;
+    const bool fused = (long)c->ncx * c->ncy * c->ncz <= PCG_FUSED_CELLS;
     double rr, bb;
-    // the V-cycle and the direction update write interior cells only; keep
-    // the half-cell planes of z and p at 0
+    // the V-cycle and k_pcg_p write interior cells only; keep the half-cell
+    // planes of z and p at 0
     TB_CHECK(c, hipMemsetAsync(z, 0, sizeof(double) * n, c->s));
-    TB_CHECK(c, hipMemsetAsync(p, 0, sizeof(double) * n, c->s));
+    if (!fused) TB_CHECK(c, hipMemsetAsync(p, 0, sizeof(double) * n, c->s));
     if (rr_known) {
         rr = *rr_known;
     } else {
@@ -1552,28 +1720,49 @@ static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double
     }
     res = sqrt(rr) / bn;
     int slot = 0;
-    // z = V(r), then p = z + beta p
+    const int nvb = (int)std::min<long>(PB, (n + PT - 1) / PT);   // blocks of the vector kernels
+    // z = V(r), then p = z + beta p, q = A p and the partial sums of p . q
     auto direction = [&](bool first) -> int {
         if (tb_vcycle64(c, r, z)) return -1;
         vcy++;
-        // the sums of r . z, z and r: the V-cycle's last pair's, or a
-        // separate pass when the finest level has no pairs
+        // the sums of r . z, z and r: the V-cycle's last smoothing launch's,
+        // or a separate pass when the finest level has no such
         int nb = c->vc_dot_blocks;
         if (nb == 0) {
-            nb = PB;
-            hipLaunchKernelGGL(k_pcg_rz, dim3(PB), dim3(PT), 0, c->s, n, (const double *)r, (const double *)z, c->red);
+            nb = nvb;
+            hipLaunchKernelGGL(k_pcg_rz, dim3(nvb), dim3(PT), 0, c->s, n, (const double *)r, (const double *)z, c->red);
             TB_LAUNCH_CHECK(c);
         }
-        if (tb_reduce_finish(c, nb, 3, S_TMP0)) return -1;
         const int old = S_RZ + slot;
         slot ^= 1;
-        hipLaunchKernelGGL(k_pcg_p, tiles_grid(P.cells), tiles_block(), 0, c->s, c->d, (const double *)z, p, c->scal,
-                           old, S_RZ + slot, first ? 1 : 0, ncell, P.cells);
+        const bool in = fused && nb <= SUM_INLINE;
+        if (!in)
+            hipLaunchKernelGGL(k_pcg_beta, dim3(1), dim3(1024), 0, c->s, (const double *)c->red, nb, c->scal, old,
+                               S_RZ + slot, first ? 1 : 0, ncell);
+        if (fused) {
+            std::swap(p, po);
+            const auto k = first ? (in ? k_pcg_pa<true, true> : k_pcg_pa<true, false>)
+                                 : (in ? k_pcg_pa<false, true> : k_pcg_pa<false, false>);
+            TB_PROF(c, TB_K_POIS_OP,
+                    hipLaunchKernelGGL(k, ktiles_grid(P.kt), tiles_block(), 0, c->s, P.Pn, (const double *)z,
+                                       (const double *)po, p, q, nb, c->scal, old, S_RZ + slot, ncell, c->red, P.kt));
+        } else {
+            hipLaunchKernelGGL(k_pcg_p, tiles_grid(P.cells), tiles_block(), 0, c->s, c->d, (const double *)z, p,
+                               (const double *)c->scal, first ? 1 : 0, P.cells);
+            TB_PROF(c, TB_K_POIS_OP,
+                    hipLaunchKernelGGL(k_pois_km<0>, ktiles_grid(P.kt), tiles_block(), 0, c->s, P.Pn,
+                                       (const double *)p, (const double *)nullptr, q, (float *)nullptr,
+                                       c->red + PQ_ARRAY * (long)RED_MAX_BLOCKS, P.kt));
+        }
         TB_LAUNCH_CHECK(c);
         return 0;
     };
     const int skip = c->pcg_its > 2 ? std::min(c->pcg_its, PCG_SKIP_MAX) - 2 : 0;
     const int its0 = its;
+    // the recursive residual is followed no further than FP64's reach: beyond,
+    // the iteration only adds rounding to x (a residual of 6e-10 after 200
+    // iterations, from 2e-11 after 10, at 128x96x100 with a tolerance of 1e-18)
+    const double stop = std::max(0.5 * rtol, 1e-15);
     // the passes that may leave the true residual above half of what it was
     // before the tolerance counts as out of reach of FP64
     int stalls = 3;
@@ -1582,23 +1771,21 @@ static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double
         if (direction(true)) return -1;
         int inner = 0;
         while (its < maxit) {
-            TB_PROF(c, TB_K_POIS_OP,
-                    hipLaunchKernelGGL(k_pois_km<0>, ktiles_grid(P.kt), tiles_block(), 0, c->s, P.Pn,
-                                       (const double *)p, (const double *)nullptr, q, (float *)nullptr, c->red, P.kt));
-            TB_LAUNCH_CHECK(c);
-            if (tb_reduce_finish(c, (int)P.nblk, 1, S_PQ)) return -1;
+            const bool in = P.nblk <= SUM_INLINE;
+            if (!in && tb_reduce_finish(c, (int)P.nblk, 1, S_PQ, PQ_ARRAY)) return -1;
             TB_PROF(c, TB_K_PCG_UPD,
-                    hipLaunchKernelGGL(k_pcg_xr, dim3(PB), dim3(PT), 0, c->s, n, x, r, (const double *)p,
-                                       (const double *)q, (const double *)c->scal, S_RZ + slot, c->red));
+                    hipLaunchKernelGGL(in ? k_pcg_xr<true> : k_pcg_xr<false>, dim3(nvb), dim3(PT), 0, c->s, n, x, r,
+                                       (const double *)p, (const double *)q, (int)P.nblk, (const double *)c->scal,
+                                       S_RZ + slot, c->red));
             TB_LAUNCH_CHECK(c);
             its++;
             inner++;
             if (inner >= 200) break;
             if (its - its0 > skip && its < maxit) {
-                if (tb_reduce_read(c, PB, 1, S_RR)) return -1;
+                if (tb_reduce_read(c, nvb, 1, S_RR)) return -1;
                 double rrel = sqrt(c->hscal[S_RR]) / bn;
                 if (!(rrel == rrel)) { c->err = "Poisson CG produced NaN"; return -1; }
-                if (rrel <= 0.5 * rtol) break;
+                if (rrel <= stop) break;
             }
             if (its < maxit && direction(false)) return -1;
         }
