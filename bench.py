@@ -10,8 +10,9 @@ Helmholtz solve to 1e-12.  Two device paths are timed on the same state:
   headline -- learned mode: Galerkin guess on the last eight solutions and
               the trained network's direction (the network is dropped at
               run time if its saved iterations cost more than its
-              inference), then FP32 CG with FP32 V-cycles inside FP64
-              iterative refinement (FP64 GMG-PCG takes over if it stalls)
+              inference), then a direct FP32 solve in cosine modes inside
+              FP64 iterative refinement (FP64 GMG-PCG takes over if it
+              stalls)
 The JSON line's `value` is the headline path's timesteps/s.  Inputs are
 resident in HBM before the timed region; each library step ends with a
 device synchronisation, so the wall clock brackets exactly K steps.
@@ -53,7 +54,6 @@ BYTES_PER_POINT = {
     # momentum u, v, w, three flags, three pressure gradients and c in, three
     # right-hand sides out; concentration c, u, v, w and a flag in, one out
     "ENO_MOM": 83, "ENO_CONC": 41, "PROJECT": 115, "BICG_UPD": 56, "PCG_UPD": 48, "POIS_OP": 16,
-    "CG32_OP": 8, "CG32_UPD": 24,
 }
 WEIGHTS = os.path.join(ROOT, "turbins_amd", "weights", "poisson_guess.f32")
 # HBM bytes per instrumented launch measured with rocprofv3 FETCH_SIZE /
@@ -146,18 +146,18 @@ def roofline(prof, stats, c):
         if name in BYTES_PER_POINT:
             total = BYTES_PER_POINT[name] * NT * n
         elif name == "HELM_OP":
-            # 17 B/point (x, status, y) per launch; the rhat.v launch of each
-            # BiCGStab iteration also reads rhat (8 B/point)
-            total = 17 * NT * n + 8 * NT * helm_its
+            # the Gauss-Seidel solves' residual checks, at least one each: x,
+            # b, the field it started from and the status in, the FP32
+            # increment out
+            total = 29 * NT * n_first
         elif name == "HELM_GS":
             # one fused red+black sweep pair: x, b and the status byte read
             # once, the new x written once; the first pair of each solve also
             # reads the last solve's increment (FP32, 4 B/point)
-            total = 25 * NT * n + 4 * NT * n_first
+            # (a launch carries the pairs of up to four solves)
+            total = 25 * NT * helm_its + 4 * NT * n_first
         elif name == "RBGS0":
             total = 24 * ncell * n      # FP64 fused pair: x, b read, x written
-        elif name == "RBGS0_F32":
-            total = 12 * ncell * n      # FP32 fused pair: x, b read, x written
         else:
             continue
         if best is None or ms > best[1]:
@@ -170,7 +170,7 @@ def roofline(prof, stats, c):
     achieved = per_launch / avg_s / 1e9
     traffic = MEASURED_TRAFFIC.get(name) if c["nx"] == 512 and c["ny"] == 256 and c["nz"] == 128 else None
     if name == "HELM_GS" and traffic is not None:
-        traffic = ((n - n_first) * traffic + n_first * MEASURED_TRAFFIC["HELM_GS_FIRST"]) / n
+        traffic = ((helm_its - n_first) * traffic + n_first * MEASURED_TRAFFIC["HELM_GS_FIRST"]) / n
     return {"kernel": name, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
             "bytes_per_launch": int(per_launch), "avg_launch_us": round(avg_s * 1e6, 2), "launches": n}
@@ -349,7 +349,7 @@ def main():
             "helmholtz_rtol": 1e-12,
             "headline_path": "Galerkin guess from the last eight solutions"
                              + (" + network direction while its gate is open" if learned else "")
-                             + ", FP32 CG + FP32 V-cycles inside FP64 iterative refinement",
+                             + ", direct FP32 solve inside FP64 iterative refinement",
             "learned_guess_loaded": learned,
             # what the timed headline steps ran: the network's direction
             # only while its run-time gate was open
@@ -368,7 +368,7 @@ def main():
             "solve_ms_per_step_plain": phase_ms(st_plain),
             "headline_vs_fp64_step_rel_l2": mixed_err,
             "solve_ms_per_step_headline": phase_ms(st_head),
-            "precision": "FP64 fields/ENO/Helmholtz/outer Poisson; FP32 multigrid in the headline path",
+            "precision": "FP64 fields/ENO/Helmholtz/outer Poisson; FP32 direct solve in the headline path",
         },
         "roofline": rl,
     }

@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(ConvFwd a) {
 // values, so 27 products (28 with the ones row that sums dY for the bias)
 // follow three 16-byte row loads.  Bound by the matrix cores; the partial sums of a
 // block's four waves meet in LDS, those of the blocks in k_wgrad_sum, in a fixed
-// order.  64^3 voxels, 48 -> 16 channels: 466 -> 24 us (the scalar gathers of
+// order.  64^3 voxels, 48 -> 16 channels: 466 -> 15 us (the scalar gathers of
 // the voxel-major form bound it).
 constexpr int WG_TILES = 28;                 // 27 taps and the bias
 constexpr int WG_ELEMS = WG_TILES * 256;

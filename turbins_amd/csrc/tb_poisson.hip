@@ -410,24 +410,15 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
 #pragma unroll
     for (int r6 = 0; r6 < 6; r6++) roff[r6] = clampi(2 * Jc - 2 + r6, 0, ny - 1) * F.px + i;
     // planes kc-1 .. kc+2 of x and kc, kc+1 of b in registers: the loads of
-    // a plane are issued two steps before its residual needs them.  The
-    // wave's edge lanes also prefetch the x neighbour across the wave edge
-    // (west for lane 0, east for lane 63) of rows 2J-1 .. 2J+2 of planes
-    // kc .. kc+2, so no load waits inside the residual.  FP32 only: the
-    // FP64 form runs faster with the registers left to occupancy and loads
-    // those values where it uses them.
-    constexpr bool PF = sizeof(T) == 4;
-    T xm[6], xc[6], xp[6], xq[6], bc0[4], bc1[4], ec[4], ep[4], eq[4];
-    const int eoff = !PF ? 0 : (lane == 0 && i > 0) ? -1 : ((lane == 63 && i < nx - 1) ? 1 : 0);
+    // a plane are issued two steps before its residual needs them.  (The x
+    // neighbours across the wave's edges are loaded where they are used:
+    // prefetched too, they take registers that occupancy needs more.)
+    T xm[6], xc[6], xp[6], xq[6], bc0[4], bc1[4];
     int kc = 0;   // fine plane held in xc
-    auto load_plane = [&](int kf, T *dst, T *edst) {
+    auto load_plane = [&](int kf, T *dst) {
         if (kf < 0 || kf >= nz) return;
 #pragma unroll
         for (int r6 = 0; r6 < 6; r6++) dst[r6] = x[kf * pl + roff[r6]];
-        if (eoff != 0) {
-#pragma unroll
-            for (int tj = 0; tj < 4; tj++) edst[tj] = x[kf * pl + roff[1 + tj] + eoff];
-        }
     };
     auto load_b = [&](int kf, T *dst) {
         if (kf < 0 || kf >= nz) return;
@@ -438,9 +429,9 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
 #pragma unroll
         for (int r6 = 0; r6 < 6; r6++) { xm[r6] = xc[r6]; xc[r6] = xp[r6]; xp[r6] = xq[r6]; }
 #pragma unroll
-        for (int tj = 0; tj < 4; tj++) { bc0[tj] = bc1[tj]; ec[tj] = ep[tj]; ep[tj] = eq[tj]; }
+        for (int tj = 0; tj < 4; tj++) bc0[tj] = bc1[tj];
         kc++;
-        load_plane(kc + 2, xq, eq);
+        load_plane(kc + 2, xq);
         load_b(kc + 1, bc1);
     };
     // y-restricted residual of fine plane kc (absent planes are not read).
@@ -459,12 +450,11 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
             const bool hs = jr > 0, hn = jr < ny - 1;
             const T xcc = xc[r6];
             // x neighbours from the adjacent lanes (a wave is 64 consecutive
-            // i); the wave's edge lanes take their prefetched values (ec[tj]
-            // is row roff[1 + tj])
+            // i); the wave's edge lanes load theirs
             T xw = __shfl_up(xcc, 1, 64), xe = __shfl_down(xcc, 1, 64);
             const int id = kc * pl + roff[r6];
-            if (lane == 0) xw = hw ? (PF ? ec[tj] : x[id - 1]) : xcc;
-            if (lane == 63) xe = he ? (PF ? ec[tj] : x[id + 1]) : xcc;
+            if (lane == 0) xw = hw ? x[id - 1] : xcc;
+            if (lane == 63) xe = he ? x[id + 1] : xcc;
             xw = hw ? xw : xcc;
             xe = he ? xe : xcc;
             const T xs = hs ? xc[r6 - 1] : xcc, xn = hn ? xc[r6 + 1] : xcc;
@@ -481,11 +471,10 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
         return sum;
     };
     kc = 2 * K0 - 1 < 0 ? 0 : 2 * K0 - 1;
-    T edummy[4];
-    load_plane(kc - 1, xm, edummy);
-    load_plane(kc, xc, ec);
-    load_plane(kc + 1, xp, ep);
-    load_plane(kc + 2, xq, eq);
+    load_plane(kc - 1, xm);
+    load_plane(kc, xc);
+    load_plane(kc + 1, xp);
+    load_plane(kc + 2, xq);
     load_b(kc, bc0);
     load_b(kc + 1, bc1);
     T Rm1 = plane_sum();
@@ -2019,7 +2008,7 @@ static void launch_dots(tb_ctx *c, long n, const Dirs &D, const double *b, const
     else hipLaunchKernelGGL((k_guess_dots<H, false>), dim3(PB), dim3(PT), 0, c->s, n, D, b, d, q, c->red);
 }
 
-// On return with ndir > 0, x is pinned and lev[0].b32 holds the FP32 copy of
+// On return with ndir > 0, x is pinned and r32 holds the FP32 copy of
 // its residual, whose squared norm is rrg (and that of b bbg); with ndir = 0
 // x is untouched.  c->guess_r / guess_nr receive the products phi_k . b for
 // the Galerkin matrix of the next solve.
