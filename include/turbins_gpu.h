@@ -82,7 +82,7 @@ enum {
 
 /* Poisson modes */
 #define TB_POIS_FP64_PCG 0      /* FP64 CG preconditioned by an FP64 V-cycle */
-#define TB_POIS_MIXED_IR 1      /* direct FP32 solves inside FP64 iterative refinement */
+#define TB_POIS_MIXED_IR 1      /* FP32 V-cycles inside FP64 iterative refinement */
 #define TB_POIS_LEARNED_IR 2    /* learned initial guess + mode 1, fallback to mode 0 */
 
 /* Level-set reinitialisation, near-interface gradient (Levelset.c:426-456):
@@ -142,7 +142,7 @@ typedef struct tb_solve_stats {
                                    GMG-PCG then started from.  Helmholtz: 1 if the
                                    Gauss-Seidel sweeps stopped contracting and BiCGStab
                                    finished the solve. */
-    int32_t vcycles;            /* V-cycles or direct FP32 solves applied (Poisson) */
+    int32_t vcycles;            /* V-cycles applied (Poisson) */
     double res0;                /* initial true relative residual (NaN: not evaluated,
                                    the Helmholtz Gauss-Seidel path) */
     double res;                 /* final true relative residual ||b-Ax||/||b|| */
@@ -531,27 +531,29 @@ int tb_set_helmholtz_rtol(tb_ctx *ctx, double rtol);
 #define TB_HELM_GS 0
 #define TB_HELM_BICGSTAB 1
 int tb_set_helmholtz_method(tb_ctx *ctx, int method);
-/* mixed Poisson mode: the smallest residual reduction asked of an iterative
- * FP32 inner solve and its iteration cap.  The inner solve is direct, one
- * iteration per refinement pass: the reduction is checked and has no effect,
- * a cap of 0 leaves the refinement passes without FP32 work, so every mixed
- * solve hands over to FP64 GMG-PCG at once (st->fallback bit 1) */
+/* mixed Poisson mode: smallest residual reduction one FP32 inner solve is
+ * asked for (default 1e-5) and its iteration cap (default 40); a cap of 0
+ * leaves the refinement passes without FP32 work, so every mixed solve
+ * hands over to FP64 GMG-PCG at once (st->fallback bit 1) */
 int tb_set_mixed_inner(tb_ctx *ctx, double reduction_floor, int maxit);
 /* learned mode: number of previous solutions (1..10, default 8) whose
  * A-norm-optimal combination, with the network's direction when one is
  * attached and its gate open, is the initial guess (the reference starts
  * from the previous pressure alone, Solver.c:256) */
 int tb_set_guess_history(tb_ctx *ctx, int h);
-/* sweeps of the finest multigrid level per side of the FP64 V-cycle (0:
- * mg_pre / mg_post of the config; 1..8 otherwise); the FP32 pair is checked
- * and has no effect, the FP32 solve being direct.  No reference counterpart:
- * hypre's BoomerAMG settings (Solver.c:90-265) are fixed there. */
+/* sweeps of the finest multigrid level per V-cycle side, FP32 and FP64
+ * cycles apart (0: mg_pre / mg_post of the config, which the coarser levels
+ * keep; 1..8 otherwise).  No reference counterpart: hypre's BoomerAMG
+ * settings (Solver.c:90-265) are fixed there. */
 int tb_set_mg_finest_sweeps(tb_ctx *ctx, int pre32, int post32, int pre64, int post64);
-/* multigrid launch structure: 1 (default) a finest level of at most 2^18
- * cells runs each V-cycle side as one launch (all sweep pairs and, after the
- * coarse level, the prolongation, per box in LDS); 0 one launch per half
- * sweep and a separate prolongation.  Both give the same bits.  No reference
- * counterpart (hypre's BoomerAMG, Solver.c:90-265). */
+/* multigrid launch structure: 1 (default) the levels of at most 2^18 cells
+ * between the finest and the LDS-resident coarse cycle run each V-cycle
+ * side as one launch (all sweep pairs and, after the coarse levels, the
+ * prolongation, per box in LDS), and the FP32 fused-pair levels coarsened
+ * in y and z form the prolongation inside their first post-smoothing pair;
+ * 0 one launch per half sweep and a separate prolongation.  Both give the
+ * same bits.  No reference counterpart (hypre's BoomerAMG,
+ * Solver.c:90-265). */
 int tb_set_mg_smoother(tb_ctx *ctx, int blocked);
 /* multigrid V-cycles replayed from HIP graphs (default 1) or launched
  * kernel by kernel (0); results are identical */
@@ -606,9 +608,9 @@ enum {
     TB_K_ENO_MOM = 0, TB_K_ENO_CONC, TB_K_HELM_OP, TB_K_BICG_UPD, TB_K_POIS_OP,
     TB_K_RBGS0, TB_K_RBGS0_F32, TB_K_PCG_UPD, TB_K_PROJECT, TB_K_RHS, TB_K_NET,
     TB_K_CG32_OP, TB_K_CG32_UPD, TB_K_HELM_GS,
-    TB_K_MG_LEVELS,      /* sweeps of multigrid levels between the finest and the direct solve */
+    TB_K_MG_LEVELS,      /* sweeps of the multigrid levels below the finest */
     TB_K_MG_TRANSFER,    /* residual + restriction and prolongation, every level */
-    TB_K_MG_SMALL,       /* the direct solves in cosine modes, or the coarse sweeps */
+    TB_K_MG_SMALL,       /* the one-workgroup cycle of the small levels, or the coarse sweeps */
     TB_K_GUESS,          /* the Galerkin guess's dot products and combination */
     TB_K_IB,             /* the immersed rows' Jacobi updates and scaled applications */
     TB_K_COUNT

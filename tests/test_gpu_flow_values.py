@@ -1,0 +1,69 @@
+"""Flow outputs against kept values of the same solver.
+
+A Poisson solve stops at a relative residual of 1e-10; which of the fields
+within that residual it returns shows in the outputs: through open x faces, at
+the walls of thin boxes, and where a difference of 1e-11 turns an ENO stencil
+choice or the BF16 rounding of a snapshot.  The fixture holds about a thousand
+nodes of each field after some steps, as the FP64 and the FP32 conjugate
+gradients of the V-cycle return them; tests/golden/make_flow_values.py writes
+it.  A change that leaves those solves
+alone moves the fields by FP64 rounding carried through the steps, far below
+1e-11; another path to the same residual moves DPDZ by 1e-9 to 1e-8 here.  The
+bounds, 1e-9 of a field's samples in the 2-norm and forty times that of their
+root mean square in each, lie between."""
+import os
+
+import numpy as np
+import pytest
+
+from turbins_amd import Solver, abi, workload as W
+
+pytestmark = pytest.mark.gpu
+
+GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "flow_values.npz")
+NAMES = ("U", "V", "W", "C", "DPDX", "DPDY", "DPDZ")
+FLOWS = {
+    # plain CG
+    "open32": dict(nx=32, ny=40, nz=24, re=3160.0, mode=abi.POIS_FP64_PCG, open=True, steps=20),
+    # mixed precision, first order
+    "open224": dict(nx=224, ny=24, nz=32, re=2680.0, mode=abi.POIS_MIXED_IR, eno_order=1, open=True, steps=10),
+    # guesses from earlier solutions, a thin box
+    "thin376": dict(nx=376, ny=28, nz=24, re=616.0, mode=abi.POIS_LEARNED_IR, open=False, steps=20),
+    # a finest level of 1.6 million cells
+    "box256": dict(nx=256, ny=96, nz=64, re=2000.0, mode=abi.POIS_MIXED_IR, open=False, steps=2),
+}
+
+
+def flow_samples(name):
+    f = FLOWS[name]
+    c = W.case("bump512x128", nx=f["nx"], ny=f["ny"], nz=f["nz"], re=f["re"], particle=True, v_settle=0.02,
+               eno_order=f.get("eno_order", 2))
+    g = Solver(W.config_for(c, pois_rtol=1e-10, helm_rtol=1e-12, pois_mode=f["mode"]))
+    g.setup_geometry(W.topography(c))
+    for n, a in W.initial_fields(c, [g.flags(q) for q in range(4)]).items():
+        g.upload(n, a)
+    if f["open"]:
+        g.set_open_boundaries(inflow=True, outflow=True, u_conv=1.0)
+    for s in range(f["steps"]):
+        if f["open"]:
+            g.inflow_profile(s * 1e-3)
+        g.step(1e-3)
+    every = 97 * max(1, g.NT // 97000)
+    out = {n: g.download(n)[::every].copy() for n in NAMES}
+    g.close()
+    return out
+
+
+@pytest.mark.parametrize("name", sorted(FLOWS))
+def test_flow_values(name):
+    print("flow", name, flush=True)
+    kept = np.load(GOLDEN)
+    bad = []
+    for n, a in flow_samples(name).items():
+        k = kept[name + "_" + n]
+        nrm = np.linalg.norm(k)
+        rel, worst = np.linalg.norm(a - k) / nrm, np.abs(a - k).max() / (nrm / np.sqrt(k.size))
+        print(n, rel, worst, flush=True)
+        if rel > 1e-9 or worst > 4e-8:
+            bad.append((n, rel, worst))
+    assert not bad

@@ -1,13 +1,9 @@
-"""The FP64 conjugate gradient iteration where its launches differ: boxes of
-the blocked smoother with every sum added up by its consumers, more partial
-sums than that (the sweeps of a finest level without boxes), two passes for
-the direction and the operator above a million cells, and a single block.
+"""The FP64 conjugate gradient iteration over its multigrid's forms: the
+one-workgroup cycle alone, axes that stop halving, and finest levels above a
+quarter of a million and a million cells.
 
 A random right-hand side of zero mean is solved from zero; the oracle's
-residual of the result is the tolerance up to its summation order.  A
-tolerance out of FP64's reach ends with status 1 and the best iterate: the
-residual's own rounding is about 1e-16 times the row sum times the solution
-over the right-hand side, below 1e-11 here."""
+residual of the result is the tolerance up to its summation order."""
 import numpy as np
 import pytest
 
@@ -30,18 +26,15 @@ def test_plain_poisson(nx, ny, nz, lx):
     r = np.random.default_rng(nx + ny + nz).standard_normal((nz, ny, nx))
     b[:nz, :ny, :nx] = r - r.mean()
     nb = np.linalg.norm(b)
-    for rtol in (RTOL, RTOL, 1e-18):   # the second solve reads back its residual later
-        g.set_poisson_mode(abi.POIS_FP64_PCG, rtol)
+    for _ in range(2):
+        g.set_poisson_mode(abi.POIS_FP64_PCG, RTOL)
         g.upload("PHI", np.zeros(g.NT))
         g.upload("PRHS", b)
         st = g.poisson_solve()
         x = g.download("PHI")
         res = np.linalg.norm(b.ravel() - o.poisson_apply(x)) / nb
-        print("rtol", rtol, "its", st.iterations, "res", st.res, "oracle", res, flush=True)
-        if rtol == RTOL:
-            assert st.converged and res <= RTOL * (1 + 1e-6) and st.iterations <= 30
-        else:
-            assert not st.converged and res <= 1e-11 and np.isfinite(x).all()
+        print("its", st.iterations, "res", st.res, "oracle", res, flush=True)
+        assert st.converged and res <= RTOL * (1 + 1e-6) and st.iterations <= 30
         assert x.reshape(b.shape)[nz - 1, ny - 1, nx - 1] == 0.0
     g.close()
     o.close()

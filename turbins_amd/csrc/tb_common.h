@@ -120,8 +120,11 @@ __device__ inline bool tile_point_kfast(const Tiles &t, int &i, int &j, int &k) 
 // column 512 and row 256) are listed 256 to a block, and the last k chunk
 // takes up to KCHUNK/2 extra planes (129 planes: 8 chunks, not 9).  Each
 // block is a chain of plane steps, so nearly empty tiles would cost as much
-// time as full ones; for the same reason grids with fewer than
-// KTILES_BLOCKS blocks (four per CU) are walked in shorter chunks.
+// time as full ones; for the same reason the Helmholtz kernels, whose sums
+// only decide when a solve stops, walk grids with fewer than KTILES_BLOCKS
+// blocks (four per CU) in shorter chunks.  The Poisson operator keeps whole
+// chunks: its partial sums enter the conjugate gradient's steps, and their
+// order is part of what a solve to a finite tolerance returns.
 constexpr int KCHUNK = 16;
 constexpr int KTILES_BLOCKS = 1024;
 
@@ -133,7 +136,7 @@ struct KTiles {
     long n, per_xcd;    // blocks: (tx * ty + eb) * kc
 };
 
-inline KTiles make_ktiles(int nx, int ny, int nz) {
+inline KTiles make_ktiles(int nx, int ny, int nz, bool shorten = false) {
     KTiles t;
     t.nx = nx; t.ny = ny; t.nz = nz;
     t.tx = nx / TILE_X;
@@ -145,7 +148,7 @@ inline KTiles make_ktiles(int nx, int ny, int nz) {
     for (t.ch = KCHUNK;; t.ch /= 2) {
         t.kc = (nz + t.ch / 2) / t.ch;
         if (t.kc < 1) t.kc = 1;
-        if (t.ch == 2 || (t.tx * t.ty + t.eb) * t.kc >= KTILES_BLOCKS) break;
+        if (!shorten || t.ch == 2 || (t.tx * t.ty + t.eb) * t.kc >= KTILES_BLOCKS) break;
     }
     t.n = (long)(t.tx * t.ty + t.eb) * t.kc;
     t.per_xcd = (t.n + NXCD - 1) / NXCD;
@@ -243,17 +246,6 @@ constexpr int GUESS_HIST = 10;     // stored solutions (upper bound of tb_set_gu
 constexpr int GUESS_DEFAULT = 8;
 constexpr int GUESS_DIRS = GUESS_HIST + 1;
 
-// the cosine matrices and eigenvalues of one axis (tb_spectral.hip)
-struct SpecAxis {
-    int n = 0;
-    void *tab = nullptr;        // packed matrices: forward even and odd, inverse even and odd
-    size_t off[4] = {};         // their offsets, in elements
-    double *lam = nullptr;      // eigenvalues in the stored mode order
-};
-struct Spectral {
-    SpecAxis y, z;
-};
-
 struct Level {
     int nx, ny, nz;       // cells
     int px;               // row pitch (elements)
@@ -261,9 +253,10 @@ struct Level {
     double hx, hy, hz;
     int cx, cy, cz;       // halved towards the next level
     double *x64, *b64, *r64;
+    float *x32, *b32, *r32;
     double *a64;          // second iterate buffer of levels smoothed by fused pairs, else null
+    float *a32;
     bool pairs;           // smoothed by fused sweep pairs
-    Spectral spec[2];     // of the levels solved directly: FP32, FP64
 };
 
 // ---------------------------------------------------------------------------
@@ -362,24 +355,28 @@ struct tb_ctx {
     // multigrid
     int nlev = 0;
     Level lev[16];
-    float *x32 = nullptr, *r32 = nullptr;   // mixed solve: FP32 correction and residual (level-0 layout)
-    bool spec32 = false;         // level 0 fits the FP32 direct solve
-    bool coarse_direct = true;   // the coarsest level is solved directly, else by sweeps
-    // V-cycle replayed from a HIP graph, tied to the level-0 vectors it was
-    // captured with
+    double *coarse_inv64 = nullptr;
+    float *coarse_inv32 = nullptr;
+    float *cg32[3] = {};         // p, q, e of the FP32 inner CG (level-0 layout)
+    // V-cycles replayed from HIP graphs (0: FP64, 1: FP32); the FP64 graph is
+    // tied to the level-0 vectors it was captured with
     bool use_graphs = true;
-    hipGraphExec_t vc_exec = nullptr;
+    hipGraphExec_t vc_exec[2] = {nullptr, nullptr};
     int helm_method = TB_HELM_GS;    // Helmholtz solver
     HelmHistory helm[4];         // Gauss-Seidel history of u, v, w and the selected concentration field
     bool helm_sets = true;       // cleared when there is no memory for the sets' third buffers
-    double ir_floor = 1e-5;      // tb_set_mixed_inner: kept for callers, the direct inner solve has no target
-    int ir_maxit = 40;           // FP32 solves per refinement pass (0: none)
-    int pcg_its = 0;             // iterations of the last FP64 solve
-    // partial sums r . z, sum z, sum r left in red by the V-cycle's last
-    // smoothing launch of the finest level; 0: it left none
-    int vc_dot_blocks = 0;
-    int mg_pre0 = 0, mg_post0 = 0;   // FP64 sweeps on the finest level per V-cycle side; 0: cfg.mg_pre / cfg.mg_post
-    bool mg_blocked = true;      // small finest levels smoothed by one blocked launch per V-cycle side
+    double ir_floor = 1e-5;      // smallest residual reduction asked of one inner FP32 solve
+    int ir_maxit = 40;           // inner iterations per refinement pass
+    int ir_first_its = 0;        // iterations of the last mixed solve's first pass
+    // V-cycles (FP32, FP64) whose last finest-level pair leaves the partial
+    // sums of r . z in red[0 .. vc_dot_blocks); 0: that level has no pairs
+    int vc_dot_blocks[2] = {0, 0};
+    int mg_pre0[2] = {0, 0};     // sweeps on the finest level per V-cycle side (FP32, FP64);
+    int mg_post0[2] = {0, 0};    // 0: cfg.mg_pre / cfg.mg_post as on the coarser levels
+    bool mg_blocked = true;      // mid levels smoothed by one blocked launch per V-cycle side
+    int coarse_n = 0;
+    bool coarse_dense = true;    // coarsest level solved by its dense inverse (<= 1024 cells), else by sweeps
+    int small_l0[2] = {0, 0};   // first level of the one-workgroup cycle: FP32, FP64
     bool mg_built = false;
 
     // Poisson history for the learned guess
@@ -432,8 +429,8 @@ int tb_prof_flush(tb_ctx *c);
 
 // device scalar slots (ctx->scal)
 enum {
-    S_RHO = 0, S_ALPHA, S_OMEGA, S_BETA, S_RZ, S_RZ_1, S_PQ, S_RR, S_TS, S_TT, S_RHV,
-    S_MEAN, S_CORNER, S_TMP0, S_TMP1, S_TMP2, S_SUB = 16,
+    S_RHO = 0, S_ALPHA, S_OMEGA, S_BETA, S_RZ, S_PQ, S_RR, S_TS, S_TT, S_RHV,
+    S_BB, S_MEAN, S_CORNER, S_TMP0, S_TMP1, S_TMP2, S_SUB = 16,
     S_RES = 16 + GUESS_DIRS * GUESS_DIRS + GUESS_DIRS,   // Poisson residual: r.r, b.b, x.b
     S_COUNT = S_RES + 3
 };
@@ -459,7 +456,7 @@ enum {
 
 // internal entry points shared between translation units
 int tb_geometry_run(tb_ctx *c, const double *h_xz);
-int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0, int first_array = 0);
+int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0);
 int tb_reduce_read(tb_ctx *c, int nblocks, int nslots, int slot0, int groups = 1, long gstride = 0);
 int tb_read_scalars(tb_ctx *c, int first, int count);
 int tb_wait_published(tb_ctx *c, unsigned long long want);
@@ -468,11 +465,7 @@ int tb_dot(tb_ctx *c, const double *a, const double *b, int slot);
 int tb_mg_build(tb_ctx *c);
 void tb_mg_free(tb_ctx *c);
 int tb_vcycle64(tb_ctx *c, const double *r_pad, double *z_pad);
-// direct solve of a level in T (tb_spectral.hip)
-template <typename T> bool tb_spec_usable(const Level &L);
-template <typename T> int tb_spec_build(tb_ctx *c, Level &L);
-template <typename T> int tb_spec_solve(tb_ctx *c, const Level &L, const T *in, T *out);
-void tb_spec_free(Level &L);
+int tb_vcycle32(tb_ctx *c);
 int tb_net_predict(tb_ctx *c, double *out, int correction_only);
 int tb_net_record_one(tb_ctx *c);
 double tb_elapsed_ms(tb_ctx *c);

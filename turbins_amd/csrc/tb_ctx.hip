@@ -547,9 +547,9 @@ int tb_read_scalars(tb_ctx *c, int first, int count) {
 // wait until the context's stream has drained (spin, as tb_read_scalars)
 int tb_sync(tb_ctx *c) { return tb_read_scalars(c, 0, 0); }
 
-int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0, int first_array) {
-    hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, c->s, c->red + (long)first_array * RED_MAX_BLOCKS,
-                       c->scal, nblocks, nslots, slot0, 1, 0L, (double *)nullptr, (unsigned long long *)nullptr, 0ull);
+int tb_reduce_finish(tb_ctx *c, int nblocks, int nslots, int slot0) {
+    hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, c->s, c->red, c->scal, nblocks, nslots, slot0, 1, 0L,
+                       (double *)nullptr, (unsigned long long *)nullptr, 0ull);
     TB_LAUNCH_CHECK(c);
     return 0;
 }

@@ -292,7 +292,7 @@ static int helm_apply(tb_ctx *c, const HelmOp &H, const double *x, double *y, bo
     if (c->nib[q] > 0)
         hipLaunchKernelGGL(k_ib_apply, dim3((c->nib[q] + 255) / 256), dim3(256), 0, c->s, c->ib_row[q], c->ib_cnt[q],
                            c->ib_col[q], c->ib_val[q], c->nib[q], x, y, scaled ? H.mod : 0.0);
-    KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ);
+    KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ, true);
     if (c->prof_on) tb_prof_begin(c, TB_K_HELM_OP);
     if (mode == 0)
         hipLaunchKernelGGL(k_helm_km<0>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t);
@@ -833,7 +833,7 @@ static int gs_check(tb_ctx *c, GsRun *const *run, int n) {
         nib = run[a]->nib > nib ? run[a]->nib : nib;
     }
     if (nib > 0) hipLaunchKernelGGL(k_ib_check<N>, dim3((nib + 255) / 256, n), dim3(256), 0, c->s, S);
-    const KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ);
+    const KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ, true);
     dim3 grid = ktiles_grid(t);
     grid.y = n;
     TB_PROF(c, TB_K_HELM_OP, hipLaunchKernelGGL(k_helm_check<N>, grid, tiles_block(), 0, c->s, S, c->red, PART, t));

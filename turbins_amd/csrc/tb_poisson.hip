@@ -1,14 +1,13 @@
-// tb_poisson.hip -- pressure Poisson right-hand side, operator, the
-// multigrid-preconditioned FP64 CG, mixed-precision iterative refinement,
-// projection and the divergence check.
+// tb_poisson.hip -- pressure Poisson right-hand side, operator, geometric
+// multigrid (FP64 and FP32), GMG-preconditioned CG, mixed-precision
+// iterative refinement, projection and the divergence check.
 //
 // The reference assembles a 7-point -Laplacian over the whole box with
 // Neumann walls and one pinned corner cell (Pressure_form_LHS_matrix,
 // Pressure.c:691-936) and hands it to GMRES + BoomerAMG.  Here the operator
 // is applied matrix-free with the same row values; the solve runs CG on the
 // Neumann operator (the same matrix without the pin) with a symmetric V-cycle
-// preconditioner (FP64), or refines with direct FP32 solves of it (mixed
-// modes, tb_spectral.hip), then shifts the result so the pinned cell holds 0.  For a
+// preconditioner, then shifts the result so the pinned cell holds 0.  For a
 // compatible right-hand side (sum b = 0, which the divergence RHS satisfies
 // up to rounding) that is the unique solution of the pinned system.
 #include <algorithm>
@@ -160,10 +159,8 @@ __global__ void __launch_bounds__(256) k_pois_km(PoisOp P, const double *__restr
     block_sum<3>(acc, sh);
     if (threadIdx.x == 0 && threadIdx.y == 0) {
         part[blockIdx.x] = acc[0];
-        if (RESID) {
-            part[RED_MAX_BLOCKS + blockIdx.x] = acc[1];
-            part[2 * RED_MAX_BLOCKS + blockIdx.x] = acc[2];
-        }
+        part[RED_MAX_BLOCKS + blockIdx.x] = acc[1];
+        part[2 * RED_MAX_BLOCKS + blockIdx.x] = acc[2];
     }
 }
 
@@ -194,15 +191,13 @@ extern "C" int tb_poisson_apply(tb_ctx *c, int f_in, int f_out) {
 
 // ---------------------------------------------------------------------------
 // Geometric multigrid on cell-centred levels.  Level 0 is the interior of
-// the padded field layout; the coarser one is compact.  Coarsening halves the
-// directions whose spacing is at most half the largest one (all directions
-// when the spacings are within a factor 2), and the coarse level is solved
-// directly in cosine modes (tb_spectral.hip): a two-grid cycle.  Recursing
-// instead (smoothing every level down to 1024 cells for one workgroup's LDS)
-// took ~15 launches of 4-10 us and a 31 us one-workgroup cycle per V-cycle,
-// against five launches here, and more CG iterations.  A level whose strongly
-// coupled directions do not all halve (an odd cell count) is solved directly
-// itself.
+// the padded field layout; coarser levels are compact.  Coarsening halves a
+// direction when its spacing is at most half the largest one (semi-coarsening
+// the strongly coupled directions first; all directions when the spacings
+// are within a factor 2), stops at <= COARSEST_CELLS cells,
+// and the coarsest level is solved with a dense pseudo-inverse (A + J/n)^-1.
+
+constexpr long COARSEST_CELLS = 64;
 
 template <typename T>
 struct LV {
@@ -223,8 +218,9 @@ __global__ void __launch_bounds__(256) k_zero(LV<T> L, T *__restrict__ x, Tiles 
     x[lidx(L, i, j, k)] = (T)0;
 }
 
-// Per-cell bodies of the multigrid operations, shared by the smoothers (so
-// they give the same bits).
+// Per-cell bodies of the multigrid operations, shared by the one-launch-per-
+// step kernels of the large levels and the single-workgroup kernel of the
+// small ones (so both give the same bits).
 
 // red-black Gauss-Seidel update of cell (i, j, k); zero_init: the other
 // colour still holds the zero initial guess, so no neighbour is read
@@ -240,7 +236,11 @@ __device__ inline T rb_value(const LV<T> &L, int i, int j, int k, T bv, T xw, T 
     s = hn ? s + L.cy * xn : s; dg = hn ? dg + L.cy : dg;
     s = hb ? s + L.cz * xb : s; dg = hb ? dg + L.cz : dg;
     s = hf ? s + L.cz * xf : s; dg = hf ? dg + L.cz : dg;
-    return s / dg;
+    // the FP32 smoother (inside the FP64 refinement) takes the hardware
+    // reciprocal, within 1 ulp, one instruction instead of a correctly
+    // rounded division's ten; the FP64 one divides exactly
+    if constexpr (sizeof(T) == 4) return s * __builtin_amdgcn_rcpf(dg);
+    else return s / dg;
 }
 
 // the Gauss-Seidel value of cell (i, j, k) from x and b (id: its index)
@@ -295,10 +295,43 @@ __device__ inline void resid_cell(const LV<T> &L, const T *__restrict__ x, const
 
 __device__ inline int clampi(int a, int lo, int hi) { return a < lo ? lo : (a > hi ? hi : a); }
 
-// restriction: adjoint of the prolongation / 2 per halved axis, 1-D weights
-// (1/8, 3/8, 3/8, 1/8) with reflection at the walls.  The halved axes are
-// fixed at compile time: the 4 x 4 x 4 taps unroll, so their loads are issued
-// together
+// restriction: adjoint of the prolongation / 2 per halved axis,
+// 1-D weights (1/8, 3/8, 3/8, 1/8) with reflection at the walls
+template <typename T>
+__device__ inline T restrict_value(const LV<T> &F, int cx, int cy, int cz, const T *rf, int I, int J, int K) {
+    const T W[4] = {(T)0.125, (T)0.375, (T)0.375, (T)0.125};
+    T s = (T)0;
+    int tk0 = cz ? -1 : 0, tk1 = cz ? 2 : 0;
+    int tj0 = cy ? -1 : 0, tj1 = cy ? 2 : 0;
+    int ti0 = cx ? -1 : 0, ti1 = cx ? 2 : 0;
+    for (int tk = tk0; tk <= tk1; tk++) {
+        int kf = cz ? clampi(2 * K + tk, 0, F.nz - 1) : K;
+        T wk = cz ? W[tk + 1] : (T)1;
+        for (int tj = tj0; tj <= tj1; tj++) {
+            int jf = cy ? clampi(2 * J + tj, 0, F.ny - 1) : J;
+            T wj = cy ? W[tj + 1] : (T)1;
+            T sj = (T)0;
+            for (int ti = ti0; ti <= ti1; ti++) {
+                int ifn = cx ? clampi(2 * I + ti, 0, F.nx - 1) : I;
+                T wi = cx ? W[ti + 1] : (T)1;
+                sj += wi * rf[lidx(F, ifn, jf, kf)];
+            }
+            s += wk * wj * sj;
+        }
+    }
+    return s;
+}
+
+template <typename T>
+__device__ inline void restrict_cell(const LV<T> &F, const LV<T> &C, int cx, int cy, int cz, const T *__restrict__ rf,
+                                     T *__restrict__ bc, int I, int J, int K) {
+    const T s = restrict_value(F, cx, cy, cz, rf, I, J, K);
+    bc[lidx(C, I, J, K)] = s;
+}
+
+// restriction with the halved axes fixed at compile time: the 4 x 4 x 4
+// taps unroll, so their loads are issued together; same sums in the same
+// order as restrict_cell, so the same bits
 template <typename T, int CX, int CY, int CZ>
 __device__ inline T restrict_sum(const LV<T> &F, const T *__restrict__ rf, int I, int J, int K) {
     const T W[4] = {(T)0.125, (T)0.375, (T)0.375, (T)0.125};
@@ -349,6 +382,35 @@ __device__ inline void prolong_cell(const LV<T> &F, const LV<T> &C, int cx, int 
     xf[id] = xin[id] + s;
 }
 
+// coarsest level: x = Minv (b - mean b), then x -= mean x (whole block;
+// blockDim.x >= n, n <= 1024); MinvT is the inverse stored transposed
+template <typename T>
+__device__ inline void coarse_solve(const T *__restrict__ Minv, int n, const T *__restrict__ b, T *__restrict__ x,
+                                    double *sh, double *bb, double *mean_s) {
+    double v[1] = {0.0};
+    for (int a = threadIdx.x; a < n; a += blockDim.x) v[0] += (double)b[a];
+    block_sum<1>(v, sh);
+    if (threadIdx.x == 0) *mean_s = v[0] / n;
+    __syncthreads();
+    double mb = *mean_s;
+    for (int a = threadIdx.x; a < n; a += blockDim.x) bb[a] = (double)b[a] - mb;
+    __syncthreads();
+    double xr[1] = {0.0};
+    double mine = 0.0;
+    if ((int)threadIdx.x < n) {
+        double s = 0.0;
+        for (int cc = 0; cc < n; cc++) s += (double)Minv[(long)cc * n + threadIdx.x] * bb[cc];
+        mine = s;
+        xr[0] = s;
+    }
+    __syncthreads();
+    block_sum<1>(xr, sh);
+    if (threadIdx.x == 0) *mean_s = xr[0] / n;
+    __syncthreads();
+    if ((int)threadIdx.x < n) x[threadIdx.x] = (T)(mine - *mean_s);
+    __syncthreads();
+}
+
 // red-black Gauss-Seidel half sweep; threads tile (ceil(nx/2), ny, nz)
 template <typename T>
 __global__ void __launch_bounds__(256) k_rbgs(LV<T> L, T *__restrict__ x, const T *__restrict__ b, int color,
@@ -368,6 +430,14 @@ __global__ void __launch_bounds__(256) k_mg_resid(LV<T> L, const T *__restrict__
     resid_cell(L, x, b, r, i, j, k);
 }
 
+template <typename T>
+__global__ void __launch_bounds__(256) k_restrict(LV<T> F, LV<T> C, int cx, int cy, int cz,
+                                                  const T *__restrict__ rf, T *__restrict__ bc, Tiles t) {
+    int I, J, K;
+    if (!tile_point(t, I, J, K)) return;
+    restrict_cell(F, C, cx, cy, cz, rf, bc, I, J, K);
+}
+
 template <typename T, int CX, int CY, int CZ>
 __global__ void __launch_bounds__(256) k_restrict_t(LV<T> F, LV<T> C, const T *__restrict__ rf, T *__restrict__ bc,
                                                     Tiles t) {
@@ -383,7 +453,7 @@ __global__ void __launch_bounds__(256) k_restrict_t(LV<T> F, LV<T> C, const T *_
 // the four rows, from x planes held in registers (rows 2J-2 .. 2J+3), summed
 // over y with the restriction weights, and the z weights are applied over a
 // window of four such plane sums; the residual array never reaches HBM.  The
-// same weights and wall reflection as restrict_sum, summed y first.
+// same weights and wall reflection as restrict_cell, summed y first.
 constexpr int RR_KC = 8;   // coarse planes per block
 
 template <typename T>
@@ -410,15 +480,24 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
 #pragma unroll
     for (int r6 = 0; r6 < 6; r6++) roff[r6] = clampi(2 * Jc - 2 + r6, 0, ny - 1) * F.px + i;
     // planes kc-1 .. kc+2 of x and kc, kc+1 of b in registers: the loads of
-    // a plane are issued two steps before its residual needs them.  (The x
-    // neighbours across the wave's edges are loaded where they are used:
-    // prefetched too, they take registers that occupancy needs more.)
-    T xm[6], xc[6], xp[6], xq[6], bc0[4], bc1[4];
+    // a plane are issued two steps before its residual needs them.  The
+    // wave's edge lanes also prefetch the x neighbour across the wave edge
+    // (west for lane 0, east for lane 63) of rows 2J-1 .. 2J+2 of planes
+    // kc .. kc+2, so no load waits inside the residual.  FP32 only: the
+    // FP64 form runs faster with the registers left to occupancy and loads
+    // those values where it uses them.
+    constexpr bool PF = sizeof(T) == 4;
+    T xm[6], xc[6], xp[6], xq[6], bc0[4], bc1[4], ec[4], ep[4], eq[4];
+    const int eoff = !PF ? 0 : (lane == 0 && i > 0) ? -1 : ((lane == 63 && i < nx - 1) ? 1 : 0);
     int kc = 0;   // fine plane held in xc
-    auto load_plane = [&](int kf, T *dst) {
+    auto load_plane = [&](int kf, T *dst, T *edst) {
         if (kf < 0 || kf >= nz) return;
 #pragma unroll
         for (int r6 = 0; r6 < 6; r6++) dst[r6] = x[kf * pl + roff[r6]];
+        if (eoff != 0) {
+#pragma unroll
+            for (int tj = 0; tj < 4; tj++) edst[tj] = x[kf * pl + roff[1 + tj] + eoff];
+        }
     };
     auto load_b = [&](int kf, T *dst) {
         if (kf < 0 || kf >= nz) return;
@@ -429,9 +508,9 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
 #pragma unroll
         for (int r6 = 0; r6 < 6; r6++) { xm[r6] = xc[r6]; xc[r6] = xp[r6]; xp[r6] = xq[r6]; }
 #pragma unroll
-        for (int tj = 0; tj < 4; tj++) bc0[tj] = bc1[tj];
+        for (int tj = 0; tj < 4; tj++) { bc0[tj] = bc1[tj]; ec[tj] = ep[tj]; ep[tj] = eq[tj]; }
         kc++;
-        load_plane(kc + 2, xq);
+        load_plane(kc + 2, xq, eq);
         load_b(kc + 1, bc1);
     };
     // y-restricted residual of fine plane kc (absent planes are not read).
@@ -450,11 +529,12 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
             const bool hs = jr > 0, hn = jr < ny - 1;
             const T xcc = xc[r6];
             // x neighbours from the adjacent lanes (a wave is 64 consecutive
-            // i); the wave's edge lanes load theirs
+            // i); the wave's edge lanes take their prefetched values (ec[tj]
+            // is row roff[1 + tj])
             T xw = __shfl_up(xcc, 1, 64), xe = __shfl_down(xcc, 1, 64);
             const int id = kc * pl + roff[r6];
-            if (lane == 0) xw = hw ? x[id - 1] : xcc;
-            if (lane == 63) xe = he ? x[id + 1] : xcc;
+            if (lane == 0) xw = hw ? (PF ? ec[tj] : x[id - 1]) : xcc;
+            if (lane == 63) xe = he ? (PF ? ec[tj] : x[id + 1]) : xcc;
             xw = hw ? xw : xcc;
             xe = he ? xe : xcc;
             const T xs = hs ? xc[r6 - 1] : xcc, xn = hn ? xc[r6 + 1] : xcc;
@@ -471,10 +551,11 @@ __global__ void __launch_bounds__(256) k_resid_restrict_011(LV<T> F, LV<T> C, co
         return sum;
     };
     kc = 2 * K0 - 1 < 0 ? 0 : 2 * K0 - 1;
-    load_plane(kc - 1, xm);
-    load_plane(kc, xc);
-    load_plane(kc + 1, xp);
-    load_plane(kc + 2, xq);
+    T edummy[4];
+    load_plane(kc - 1, xm, edummy);
+    load_plane(kc, xc, ec);
+    load_plane(kc + 1, xp, ep);
+    load_plane(kc + 2, xq, eq);
     load_b(kc, bc0);
     load_b(kc + 1, bc1);
     T Rm1 = plane_sum();
@@ -599,13 +680,16 @@ static PairTiles make_pair_tiles(int nx, int ny, int nz, int tk) {
     return t;
 }
 
-// DOT: the block's partial sums of b . xn, xn and b over its own cells (the
-// final values of both colours) go to part -- r . z, sum z and sum r of a
-// V-cycle whose last sweep pair this is.
-template <typename T, int F, bool ZERO, bool DOT>
-__global__ void __launch_bounds__(PAIR_THREADS, 2)
+// DOT: the block's partial sum of b . xn over its own cells (the final
+// values of both colours) goes to part[blockIdx.x] -- r . z of a V-cycle
+// whose last sweep pair this is.  PROL (levels coarsened by (0, 1, 1)): the
+// pair starts from xo + P xc, the coarse correction prolonged as
+// k_prolong_011 does it (same expression, so the same bits), formed as each
+// plane is staged instead of in a pass of its own.
+template <typename T, int F, bool ZERO, bool DOT, bool PROL = false>
+__global__ void __launch_bounds__(PAIR_THREADS, sizeof(T) == 4 ? ((PROL && !DOT) ? 8 : 4) : 2)
     k_rbgs_pair(LV<T> L, const T *__restrict__ xo, T *__restrict__ xn, const T *__restrict__ b, PairTiles P,
-                double *__restrict__ part) {
+                double *__restrict__ part, LV<T> C = LV<T>(), const T *__restrict__ xc = nullptr) {
     __shared__ T so[PAIR_ORING][PAIR_OY * PAIR_OX];
     __shared__ T sr[3][PAIR_HY * PAIR_HX];
     const int nx = L.nx, ny = L.ny, nz = L.nz, px = L.px;
@@ -613,10 +697,10 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
     const int bid = blockIdx.x;
     const int lt = (bid % NXCD) * P.per_xcd + bid / NXCD;
     if (lt >= P.n) {                                        // whole block
-        if (DOT && threadIdx.x < 3) part[threadIdx.x * RED_MAX_BLOCKS + bid] = 0.0;
+        if (DOT && threadIdx.x == 0) part[bid] = 0.0;
         return;
     }
-    double dacc[3] = {0.0, 0.0, 0.0};
+    double dacc[1] = {0.0};
     const int tx = lt % P.tx, rest = lt / P.tx;
     const int i0 = tx * PAIR_TX, j0 = (rest % P.ty) * PAIR_TY;
     const int k0 = (rest / P.ty) * P.tk;
@@ -636,11 +720,30 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
         ooff[u] = (e < PAIR_OY * PAIR_OX && i >= 0 && i < nx && j >= 0 && j < ny) ? j * px + i : -1;
     }
     T ro[PAIR_OLD_PER], ro2[PAIR_OLD_PER];   // xo of the next two planes to stage
+    // PROL: the coarse values of each staged point, rows J0 (a) and J1 (b)
+    // of coarse planes K0 = m / 2 (0) and its neighbour K1 (1), fetched one
+    // plane ahead of their use (the xo values two)
+    T ca0[PAIR_OLD_PER], cb0[PAIR_OLD_PER], ca1[PAIR_OLD_PER], cb1[PAIR_OLD_PER];
+    int coff0[PAIR_OLD_PER], coff1[PAIR_OLD_PER];
+    const int cpl = C.px * C.py;
 #pragma unroll
-    for (int u = 0; u < PAIR_OLD_PER; u++) ro2[u] = (T)0;
+    for (int u = 0; u < PAIR_OLD_PER; u++) {
+        ro2[u] = (T)0;
+        ca0[u] = cb0[u] = ca1[u] = cb1[u] = (T)0;
+        coff0[u] = coff1[u] = 0;
+        if (PROL && ooff[u] >= 0) {
+            const int e = t + u * PAIR_THREADS;
+            const int r = e / PAIR_OX, cc = e - r * PAIR_OX;
+            const int i = i0 - 2 + cc, j = j0 - 2 + r;
+            const int J0 = j >> 1, J1 = clampi((j & 1) ? J0 + 1 : J0 - 1, 0, C.ny - 1);
+            coff0[u] = J0 * C.px + i;
+            coff1[u] = J1 * C.px + i;
+        }
+    }
     // staging on named register arrays (the compiler keeps them in
     // registers only while no pointer to them is taken): fetch the xo plane
-    // after next into ro2, shift it to ro, store ro's plane into its LDS slot
+    // after next into ro2, shift it to ro, fetch its coarse values, store
+    // ro's plane into its LDS slot
     auto fetch_next = [&](int m) {
 #pragma unroll
         for (int u = 0; u < PAIR_OLD_PER; u++) ro2[u] = ooff[u] >= 0 ? xo[m * plane + ooff[u]] : (T)0;
@@ -649,12 +752,32 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
 #pragma unroll
         for (int u = 0; u < PAIR_OLD_PER; u++) ro[u] = ro2[u];
     };
+    auto fetch_coarse = [&](int m) {
+        if (!PROL) return;
+        const int K0 = m >> 1;
+        const int K1 = (m & 1) ? (K0 + 1 < C.nz ? K0 + 1 : C.nz - 1) : (K0 > 0 ? K0 - 1 : 0);
+#pragma unroll
+        for (int u = 0; u < PAIR_OLD_PER; u++) {   // offset 0 outside the box: no branch around the loads
+            ca0[u] = xc[K0 * cpl + coff0[u]];
+            cb0[u] = xc[K0 * cpl + coff1[u]];
+            ca1[u] = xc[K1 * cpl + coff0[u]];
+            cb1[u] = xc[K1 * cpl + coff1[u]];
+        }
+    };
     auto put_cur = [&](int m) {
         T *S = so[m % PAIR_ORING];
+        const T wj1 = (T)0.25, wj0 = (T)1 - wj1, wk1 = (T)0.25, wk0 = (T)1 - wk1;
 #pragma unroll
         for (int u = 0; u < PAIR_OLD_PER; u++) {
             const int e = t + u * PAIR_THREADS;
-            if (e < PAIR_OY * PAIR_OX) S[e] = ro[u];
+            if (e < PAIR_OY * PAIR_OX) {
+                T v = ro[u];
+                if (PROL) {
+                    const T s = wk0 * (wj0 * ca0[u] + wj1 * cb0[u]) + wk1 * (wj0 * ca1[u] + wj1 * cb1[u]);
+                    v = ooff[u] >= 0 ? v + s : (T)0;
+                }
+                S[e] = v;
+            }
         }
     };
     int rrow[PAIR_RED_PER], rc2[PAIR_RED_PER];
@@ -705,10 +828,11 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
     for (int u = 0; u < PAIR_RED_PER; u++) { rb_n[u] = (T)0; rv_n[u] = false; }
     T bb_n = (T)0;
     if (!ZERO) {
-        if (k0 >= 2) { fetch_next(k0 - 2); shift(); put_cur(k0 - 2); }
-        if (k0 >= 1) { fetch_next(k0 - 1); shift(); put_cur(k0 - 1); }
+        if (k0 >= 2) { fetch_next(k0 - 2); shift(); fetch_coarse(k0 - 2); put_cur(k0 - 2); }
+        if (k0 >= 1) { fetch_next(k0 - 1); shift(); fetch_coarse(k0 - 1); put_cur(k0 - 1); }
         fetch_next(k0);
         shift();
+        fetch_coarse(k0);
         if (k0 + 1 < nz) fetch_next(k0 + 1);
     }
     if (k0 >= 1) fetch_red(k0 - 1, rb, rv);
@@ -717,6 +841,7 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
         if (!ZERO) {
             if (m + 1 < nz) put_cur(m + 1);
             shift();
+            if (m + 2 < nz) fetch_coarse(m + 2);
             if (m + 3 < nz) fetch_next(m + 3);
         }
         T rb_nn[PAIR_RED_PER];
@@ -742,11 +867,8 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
                 const T v = rb_value(L, i, j, m, rb[u], S[o - 1], S[o + 1], S[o - PAIR_OX], S[o + PAIR_OX], Sb[o],
                                      Sf[o]);
                 R[r * PAIR_HX + cc] = v;
-                if (DOT && m >= k0 && m < k1 && i >= i0 && i < i0 + PAIR_TX && j >= j0 && j < j0 + PAIR_TY) {
+                if (DOT && m >= k0 && m < k1 && i >= i0 && i < i0 + PAIR_TX && j >= j0 && j < j0 + PAIR_TY)
                     dacc[0] += (double)v * (double)rb[u];
-                    dacc[1] += (double)v;
-                    dacc[2] += (double)rb[u];
-                }
             }
         }
         __syncthreads();
@@ -759,11 +881,7 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
             const int h = (br + 1) * PAIR_HX + cc + 1;
             const T v = rb_value(L, i, bj, k, bb, R[h - 1], R[h + 1], R[h - PAIR_HX], R[h + PAIR_HX], Rb[h], Rf[h]);
             R[h] = v;
-            if (DOT) {
-                dacc[0] += (double)v * (double)bb;
-                dacc[1] += (double)v;
-                dacc[2] += (double)bb;
-            }
+            if (DOT) dacc[0] += (double)v * (double)bb;
         }
         // no barrier: the next staging writes the xo slot of plane m - 1,
         // which the second-colour pass does not read
@@ -778,11 +896,54 @@ __global__ void __launch_bounds__(PAIR_THREADS, 2)
     __syncthreads();
     write_plane(k1 - 1);
     if (DOT) {
-        __shared__ double dsh[48];
-        block_sum<3>(dacc, dsh);
-        if (threadIdx.x == 0)
-            for (int a = 0; a < 3; a++) part[a * RED_MAX_BLOCKS + bid] = dacc[a];
+        __shared__ double dsh[16];
+        block_sum<1>(dacc, dsh);
+        if (threadIdx.x == 0) part[bid] = dacc[0];
     }
+}
+
+template <typename T>
+__global__ void k_coarse(const T *__restrict__ Minv, int n, const T *__restrict__ b, T *__restrict__ x) {
+    __shared__ double sh[16];
+    __shared__ double bb[1024];
+    __shared__ double mean_s;
+    coarse_solve(Minv, n, b, x, sh, bb, &mean_s);
+}
+
+// The small levels of a V-cycle run in one workgroup of 1024 threads with
+// every level resident in LDS (compact layouts), one barrier between phases:
+// their launches (~3-5 us each, 11 per level) and L2 round trips would
+// otherwise cost far more than their work.  Level l0 is read from (b) and
+// written to (x) global memory once; one residual buffer serves all levels.
+// The first level run this way is the largest one that has at most
+// SMALL_LEVEL_CELLS cells and whose levels fit SMALL_LDS_BYTES.  One CU is
+// the limit: an 8192-cell level costs ~40 us there against ~22 us as blocked
+// launches over the chip (measured at 512x256x128), so the cycle starts at
+// 1024 cells.
+constexpr long SMALL_LEVEL_CELLS = 1024;
+constexpr int SMALL_LDS_BYTES = 156 * 1024;
+constexpr int MAXLEV = 16;
+
+template <typename T>
+struct SmallCycle {
+    int l0, nl, pre, post, coarse_n;
+    LV<T> lv[MAXLEV];          // compact layouts of the LDS copies
+    LV<T> g0;                  // layout of level l0 in global memory
+    T *gx0;                    // level l0 in global memory: x out
+    const T *gb0;              //                            b in
+    int xo[MAXLEV], bo[MAXLEV], ro;   // LDS offsets in elements of T
+    int cx[MAXLEV], cy[MAXLEV], cz[MAXLEV];
+    const T *Minv;
+};
+
+// LDS bytes of a small cycle starting at level l0: coarse-solve scratch
+// (1024 + 32 doubles), then x and b of every level and one residual buffer
+template <typename T>
+static int small_lds_bytes(const tb_ctx *c, int l0) {
+    long e = 0;
+    for (int m = l0; m < c->nlev; m++) e += 2L * c->lev[m].nx * c->lev[m].ny * c->lev[m].nz;
+    e += (long)c->lev[l0].nx * c->lev[l0].ny * c->lev[l0].nz;
+    return (int)(sizeof(double) * (1024 + 32) + sizeof(T) * e);
 }
 
 // a / d and a % d for 0 <= a < 2^22, d >= 1, from the float reciprocal inv
@@ -822,7 +983,80 @@ __device__ inline void block_cells(int nx, int ny, int nz, F f) {
     }
 }
 
-// Smoothing of a small finest level in one launch per V-cycle side.  Each block owns an output box of the
+template <typename T>
+__device__ inline void block_sweep(const LV<T> &L, T *x, const T *b, int color, bool zero_init) {
+    block_cells((L.nx + 1) / 2, L.ny, L.nz, [&](int ih, int j, int k) {
+        const int i = 2 * ih + ((j + k + color) & 1);
+        if (i < L.nx) rbgs_cell(L, x, b, i, j, k, zero_init);
+    });
+    __syncthreads();
+}
+
+template <typename T>
+__global__ void __launch_bounds__(1024) k_small_cycle(SmallCycle<T> A) {
+    extern __shared__ double smem[];
+    double *bb = smem, *sh = smem + 1024, *mean_s = smem + 1024 + 16;
+    T *S = reinterpret_cast<T *>(smem + 1024 + 32);
+    const int last = A.nl - 1;
+    {
+        const LV<T> &L = A.lv[A.l0];
+        T *b0 = S + A.bo[A.l0];
+        block_cells(L.nx, L.ny, L.nz, [&](int i, int j, int k) {
+            b0[(k * L.ny + j) * L.nx + i] = A.gb0[lidx(A.g0, i, j, k)];
+        });
+        __syncthreads();
+    }
+    T *r = S + A.ro;
+    for (int l = A.l0; l < last; l++) {
+        const LV<T> &L = A.lv[l];
+        T *x = S + A.xo[l];
+        const T *b = S + A.bo[l];
+        const int n = L.nx * L.ny * L.nz;
+        if (A.pre > 0) {
+            block_sweep(L, x, b, 0, true);
+            block_sweep(L, x, b, 1, false);
+            for (int s = 1; s < A.pre; s++) {
+                block_sweep(L, x, b, 0, false);
+                block_sweep(L, x, b, 1, false);
+            }
+        } else {
+            for (int q = threadIdx.x; q < n; q += blockDim.x) x[q] = (T)0;
+            __syncthreads();
+        }
+        block_cells(L.nx, L.ny, L.nz, [&](int i, int j, int k) { resid_cell(L, (const T *)x, b, r, i, j, k); });
+        __syncthreads();
+        const LV<T> &C = A.lv[l + 1];
+        T *bc = S + A.bo[l + 1];
+        block_cells(C.nx, C.ny, C.nz, [&](int I, int J, int K) {
+            restrict_cell(L, C, A.cx[l], A.cy[l], A.cz[l], (const T *)r, bc, I, J, K);
+        });
+        __syncthreads();
+    }
+    coarse_solve(A.Minv, A.coarse_n, (const T *)(S + A.bo[last]), S + A.xo[last], sh, bb, mean_s);
+    for (int l = last - 1; l >= A.l0; l--) {
+        const LV<T> &L = A.lv[l];
+        const LV<T> &C = A.lv[l + 1];
+        T *x = S + A.xo[l];
+        const T *b = S + A.bo[l];
+        block_cells(L.nx, L.ny, L.nz, [&](int i, int j, int k) {
+            prolong_cell(L, C, A.cx[l], A.cy[l], A.cz[l], (const T *)(S + A.xo[l + 1]), (const T *)x, x, i, j, k);
+        });
+        __syncthreads();
+        for (int s = 0; s < A.post; s++) {
+            block_sweep(L, x, b, 1, false);
+            block_sweep(L, x, b, 0, false);
+        }
+    }
+    {
+        const LV<T> &L = A.lv[A.l0];
+        const T *x0 = S + A.xo[A.l0];
+        block_cells(L.nx, L.ny, L.nz, [&](int i, int j, int k) {
+            A.gx0[lidx(A.g0, i, j, k)] = x0[(k * L.ny + j) * L.nx + i];
+        });
+    }
+}
+
+// Mid-level smoothing in one launch.  Each block owns an output box of the
 // level and runs NP red-black sweep pairs on it in LDS, recomputing the
 // 2*NP-cell halo its last half sweep depends on, so no block reads what
 // another writes: src and dst are distinct buffers.  Half sweep m = 1 ..
@@ -830,9 +1064,7 @@ __device__ inline void block_cells(int nx, int ny, int nz, F f) {
 // box grown by 2*NP - m cells, which is every cell a later half sweep of the
 // box reads.  ZERO: the sweeps start from x = 0 and read only b (the
 // pre-smoother).  PROL: the starting iterate is src + P xc, the coarse
-// level's correction prolonged on the fly (the post-smoother), and the box's
-// partial sums of b . x, x and b go to part (r . z, sum z and sum r of the
-// Krylov method around the cycle).  Every cell
+// level's correction prolonged on the fly (the post-smoother).  Every cell
 // value is formed by the expressions of rb_value and prolong_sum, so the
 // result equals the launch-per-half-sweep sequence bit for bit.
 constexpr int BLK_THREADS = 1024;
@@ -841,8 +1073,8 @@ constexpr int BLK_LDS_BYTES = 150 * 1024;    // one block per CU
 constexpr int BLK_MIN_BOXES = 128;
 // Above this many cells the halo recomputation (about 5x the cells of a box
 // for two pairs) makes the blocked launch slower than its half sweeps,
-// whose ~5 us launches it exists to save (measured: a 1M-cell level 62 us
-// blocked against 47, a 65k-cell level 17 against 42).
+// whose ~5 us launches it exists to save (measured at 512x256x128: the
+// 1M-cell level 62 us blocked against 47, the 65k-cell level 17 against 42).
 constexpr long BLK_MAX_CELLS = 1L << 18;
 
 struct BlkShape {
@@ -855,7 +1087,7 @@ struct BlkShape {
 template <typename T, int NP, bool ZERO, bool PROL, int FIRST>
 __global__ void __launch_bounds__(BLK_THREADS) k_rbgs_blk(LV<T> L, const T *__restrict__ src, const T *__restrict__ b,
                                                           T *__restrict__ dst, BlkShape S, LV<T> C, int cx, int cy,
-                                                          int cz, const T *__restrict__ xc, double *part) {
+                                                          int cz, const T *__restrict__ xc) {
     extern __shared__ double smem_blk[];
     constexpr int H = 2 * NP;
     const int rx = S.bx + 2 * H, ry = S.by + 2 * H, rz = S.bz + 2 * H;
@@ -926,24 +1158,10 @@ __global__ void __launch_bounds__(BLK_THREADS) k_rbgs_blk(LV<T> L, const T *__re
         });
         __syncthreads();
     }
-    double acc[3] = {0.0, 0.0, 0.0};
     block_cells(min(S.bx, L.nx - ox), min(S.by, L.ny - oy), min(S.bz, L.nz - oz), [&](int a, int e, int f) {
         const int i = ox + a, j = oy + e, k = oz + f;
-        const int q = ((k - gz) * ry + (j - gy)) * rx + (i - gx);
-        const T v = xs[q];
-        dst[lidx(L, i, j, k)] = v;
-        if (PROL) {
-            acc[0] += (double)bs[q] * (double)v;
-            acc[1] += (double)v;
-            acc[2] += (double)bs[q];
-        }
+        dst[lidx(L, i, j, k)] = xs[((k - gz) * ry + (j - gy)) * rx + (i - gx)];
     });
-    if (PROL) {
-        __syncthreads();   // the box is read; its LDS takes the wave sums
-        block_sum<3>(acc, smem_blk);
-        if (threadIdx.x == 0)
-            for (int a = 0; a < 3; a++) part[a * RED_MAX_BLOCKS + lt] = acc[a];
-    }
 }
 
 // LDS bytes of k_rbgs_blk for box (bx, by, bz) on level L (coarsened by its
@@ -958,7 +1176,7 @@ static long blk_lds(const Level &L, int np, size_t tsize, const int *bx, int *cn
     return (long)tsize * (2L * r[0] * r[1] * r[2] + (long)cn[0] * cn[1] * cn[2]);
 }
 
-// box of the blocked smoother: start from 32 x 16 x 8 and halve the
+// box of the mid-level smoother: start from 32 x 16 x 8 and halve the
 // largest side (not below 8) until the LDS fits two blocks per CU (else one)
 // and there are at least BLK_MIN_BOXES boxes; false if no box fits
 static bool blk_shape_cap(const Level &L, int np, size_t tsize, long cap, BlkShape &S, int &lds);
@@ -1024,32 +1242,40 @@ static int choose(const Level &L, int &cx, int &cy, int &cz) {
     return any;
 }
 
-// whether every direction that should be halved can be: where one cannot (an
-// odd cell count), halving only the others leaves a strong coupling that
-// point smoothing does not reach (28 CG iterations at 200 x 72 x 36)
-static bool halves_cleanly(const Level &L) {
-    const int n[3] = {L.nx, L.ny, L.nz};
-    const double h[3] = {L.hx, L.hy, L.hz};
-    const double hmax = std::max(h[0], std::max(h[1], h[2]));
-    bool want[3], any = false;
-    for (int a = 0; a < 3; a++) any |= want[a] = 2.0 * h[a] <= hmax * (1.0 + 1e-9);
-    for (int a = 0; a < 3; a++)
-        if ((want[a] || !any) && (n[a] % 2 || n[a] < 4)) return false;
-    return true;
+static void level_apply_host(const Level &L, const double *x, double *y) {
+    double cx = 1.0 / (L.hx * L.hx), cy = 1.0 / (L.hy * L.hy), cz = 1.0 / (L.hz * L.hz);
+    long pl = (long)L.nx * L.ny;
+    for (int k = 0; k < L.nz; k++)
+        for (int j = 0; j < L.ny; j++)
+            for (int i = 0; i < L.nx; i++) {
+                long id = ((long)k * L.ny + j) * L.nx + i;
+                double xc = x[id], s = 0.0;
+                if (i > 0) s += cx * (xc - x[id - 1]);
+                if (i < L.nx - 1) s += cx * (xc - x[id + 1]);
+                if (j > 0) s += cy * (xc - x[id - L.nx]);
+                if (j < L.ny - 1) s += cy * (xc - x[id + L.nx]);
+                if (k > 0) s += cz * (xc - x[id - pl]);
+                if (k < L.nz - 1) s += cz * (xc - x[id + pl]);
+                y[id] = s;
+            }
 }
 
 void tb_mg_free(tb_ctx *c) {
     for (int l = 0; l < c->nlev; l++) {
         Level &L = c->lev[l];
         if (l > 0) { hipFree(L.x64); hipFree(L.b64); hipFree(L.r64); }
-        hipFree(L.a64);
+        hipFree(L.x32); hipFree(L.b32); hipFree(L.r32);
+        hipFree(L.a64); hipFree(L.a32);
         L.x64 = L.b64 = L.r64 = L.a64 = nullptr;
-        tb_spec_free(L);
+        L.x32 = L.b32 = L.r32 = L.a32 = nullptr;
     }
-    hipFree(c->x32); hipFree(c->r32);
-    c->x32 = c->r32 = nullptr;
-    if (c->vc_exec) hipGraphExecDestroy(c->vc_exec);
-    c->vc_exec = nullptr;
+    hipFree(c->coarse_inv64); hipFree(c->coarse_inv32);
+    c->coarse_inv64 = nullptr; c->coarse_inv32 = nullptr;
+    for (int a = 0; a < 2; a++) {
+        if (c->vc_exec[a]) hipGraphExecDestroy(c->vc_exec[a]);
+        c->vc_exec[a] = nullptr;
+    }
+    for (int a = 0; a < 3; a++) { hipFree(c->cg32[a]); c->cg32[a] = nullptr; }
     c->nlev = 0;
     c->mg_built = false;
 }
@@ -1061,18 +1287,14 @@ int tb_mg_build(tb_ctx *c) {
     L0.nx = c->ncx; L0.ny = c->ncy; L0.nz = c->ncz;
     L0.px = c->d.px; L0.plane = c->d.plane; L0.ntot = c->d.ntot;
     L0.hx = c->cfg.lx / c->ncx; L0.hy = c->cfg.ly / c->ncy; L0.hz = c->cfg.lz / c->ncz;
-    c->nlev = 1;
-    c->spec32 = tb_spec_usable<float>(L0);
-    // one coarser level, or more where its axes are too long for the direct
-    // solve; none where the grid does not halve cleanly
-    while (c->nlev < 16) {
-        Level &L = c->lev[c->nlev - 1];
-        const bool direct = tb_spec_usable<double>(L);
-        if (direct && (c->nlev > 1 || !halves_cleanly(L))) break;
+    int nl = 1;
+    while (nl < 16) {
+        Level &L = c->lev[nl - 1];
+        if ((long)L.nx * L.ny * L.nz <= COARSEST_CELLS) break;
         int cx, cy, cz;
         if (!choose(L, cx, cy, cz)) break;
         L.cx = cx; L.cy = cy; L.cz = cz;
-        Level &C = c->lev[c->nlev];
+        Level &C = c->lev[nl];
         C = Level();
         C.nx = cx ? L.nx / 2 : L.nx; C.hx = cx ? 2.0 * L.hx : L.hx;
         C.ny = cy ? L.ny / 2 : L.ny; C.hy = cy ? 2.0 * L.hy : L.hy;
@@ -1080,48 +1302,148 @@ int tb_mg_build(tb_ctx *c) {
         C.px = (C.nx + 15) / 16 * 16;
         C.plane = (long)C.px * C.ny;
         C.ntot = C.plane * C.nz;
-        c->nlev++;
+        nl++;
     }
-    for (int l = 0; l < c->nlev; l++) {
+    c->nlev = nl;
+    for (int l = 0; l < nl; l++) {
         Level &L = c->lev[l];
-        if (l > 0)
-            for (double **p : {&L.x64, &L.b64, &L.r64}) {
-                TB_CHECK(c, hipMalloc((void **)p, sizeof(double) * L.ntot));
-                TB_CHECK(c, hipMemsetAsync(*p, 0, sizeof(double) * L.ntot, c->s));
-                c->bytes += sizeof(double) * L.ntot;
-            }
-        // second iterate buffer of the fused sweep pairs
-        L.pairs = l < c->nlev - 1 && (long)L.nx * L.ny * L.nz >= PAIR_LEVEL_CELLS && L.ntot < (1L << 31);
+        if (l > 0) {
+            TB_CHECK(c, hipMalloc((void **)&L.x64, sizeof(double) * L.ntot));
+            TB_CHECK(c, hipMalloc((void **)&L.b64, sizeof(double) * L.ntot));
+            TB_CHECK(c, hipMalloc((void **)&L.r64, sizeof(double) * L.ntot));
+            TB_CHECK(c, hipMemsetAsync(L.x64, 0, sizeof(double) * L.ntot, c->s));
+            TB_CHECK(c, hipMemsetAsync(L.b64, 0, sizeof(double) * L.ntot, c->s));
+            TB_CHECK(c, hipMemsetAsync(L.r64, 0, sizeof(double) * L.ntot, c->s));
+            c->bytes += 3 * sizeof(double) * L.ntot;
+        }
+        // second iterate buffers of the fused sweep pairs (both precisions;
+        // with two barriers per plane the FP32 pair beats two half sweeps
+        // even though those find their arrays in the 256 MB Infinity Cache)
+        L.pairs = (long)L.nx * L.ny * L.nz >= PAIR_LEVEL_CELLS && L.ntot < (1L << 31);
         if (L.pairs) {
             TB_CHECK(c, hipMalloc((void **)&L.a64, sizeof(double) * L.ntot));
             TB_CHECK(c, hipMemsetAsync(L.a64, 0, sizeof(double) * L.ntot, c->s));
-            c->bytes += sizeof(double) * L.ntot;
+            TB_CHECK(c, hipMalloc((void **)&L.a32, sizeof(float) * L.ntot));
+            TB_CHECK(c, hipMemsetAsync(L.a32, 0, sizeof(float) * L.ntot, c->s));
+            c->bytes += (sizeof(double) + sizeof(float)) * L.ntot;
         }
+        TB_CHECK(c, hipMalloc((void **)&L.x32, sizeof(float) * L.ntot));
+        TB_CHECK(c, hipMalloc((void **)&L.b32, sizeof(float) * L.ntot));
+        TB_CHECK(c, hipMalloc((void **)&L.r32, sizeof(float) * L.ntot));
+        TB_CHECK(c, hipMemsetAsync(L.x32, 0, sizeof(float) * L.ntot, c->s));
+        TB_CHECK(c, hipMemsetAsync(L.b32, 0, sizeof(float) * L.ntot, c->s));
+        TB_CHECK(c, hipMemsetAsync(L.r32, 0, sizeof(float) * L.ntot, c->s));
+        c->bytes += 3 * sizeof(float) * L.ntot;
     }
-    // the mixed solve's correction and residual; entries outside the interior
-    // cells stay 0
-    for (float **p : {&c->x32, &c->r32}) {
-        TB_CHECK(c, hipMalloc((void **)p, sizeof(float) * L0.ntot));
-        TB_CHECK(c, hipMemsetAsync(*p, 0, sizeof(float) * L0.ntot, c->s));
+    // vectors of the FP32 inner CG; entries outside the interior cells stay 0
+    for (int a = 0; a < 3; a++) {
+        TB_CHECK(c, hipMalloc((void **)&c->cg32[a], sizeof(float) * L0.ntot));
+        TB_CHECK(c, hipMemsetAsync(c->cg32[a], 0, sizeof(float) * L0.ntot, c->s));
         c->bytes += sizeof(float) * L0.ntot;
     }
-    if (c->spec32 && tb_spec_build<float>(c, L0)) return -1;
-    Level &Lc = c->lev[c->nlev - 1];
-    c->coarse_direct = tb_spec_usable<double>(Lc);
-    if (c->coarse_direct && tb_spec_build<double>(c, Lc)) return -1;
-    for (const void *k : {(const void *)k_rbgs_blk<double, 1, true, false, 0>, (const void *)k_rbgs_blk<double, 2, true, false, 0>,
-                          (const void *)k_rbgs_blk<double, 1, false, true, 1>, (const void *)k_rbgs_blk<double, 2, false, true, 1>})
-        TB_CHECK(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, BLK_LDS_BYTES));
+    // The coarsest level is solved by its dense inverse when it has at most
+    // 1024 cells.  Grid dimensions that stop halving (an odd number of
+    // cells) can leave a larger one: it then takes COARSE_SWEEPS symmetric
+    // sweep pairs from zero (the oracle's rule) and no LDS cycle is used.
+    Level &Lc = c->lev[nl - 1];
+    const long nc = (long)Lc.nx * Lc.ny * Lc.nz;
+    c->coarse_dense = nc <= 1024;
+    c->coarse_n = (int)(nc < (1L << 30) ? nc : (1L << 30));
+    // first level of the LDS-resident small cycle, per precision
+    for (int a = 0; a < 2 && !c->coarse_dense; a++) c->small_l0[a] = nl;
+    for (int a = 0; a < 2 && c->coarse_dense; a++) {
+        int l0 = nl - 1;
+        while (l0 > 0) {
+            const Level &P = c->lev[l0 - 1];
+            const int bytes = a ? small_lds_bytes<double>(c, l0 - 1) : small_lds_bytes<float>(c, l0 - 1);
+            if ((long)P.nx * P.ny * P.nz > SMALL_LEVEL_CELLS || bytes > SMALL_LDS_BYTES) break;
+            l0--;
+        }
+        c->small_l0[a] = l0;
+        const int bytes = a ? small_lds_bytes<double>(c, l0) : small_lds_bytes<float>(c, l0);
+        if (bytes > SMALL_LDS_BYTES) { c->err = "multigrid: coarsest levels exceed the LDS budget"; return -1; }
+    }
+    TB_CHECK(c, hipFuncSetAttribute((const void *)k_small_cycle<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    SMALL_LDS_BYTES));
+    TB_CHECK(c, hipFuncSetAttribute((const void *)k_small_cycle<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    SMALL_LDS_BYTES));
+    {
+        const void *blk[8] = {
+            (const void *)k_rbgs_blk<float, 1, true, false, 0>, (const void *)k_rbgs_blk<float, 2, true, false, 0>,
+            (const void *)k_rbgs_blk<float, 1, false, true, 1>, (const void *)k_rbgs_blk<float, 2, false, true, 1>,
+            (const void *)k_rbgs_blk<double, 1, true, false, 0>, (const void *)k_rbgs_blk<double, 2, true, false, 0>,
+            (const void *)k_rbgs_blk<double, 1, false, true, 1>, (const void *)k_rbgs_blk<double, 2, false, true, 1>};
+        for (int a = 0; a < 8; a++)
+            TB_CHECK(c, hipFuncSetAttribute(blk[a], hipFuncAttributeMaxDynamicSharedMemorySize, BLK_LDS_BYTES));
+    }
+    if (!c->coarse_dense) {
+        TB_CHECK(c, hipStreamSynchronize(c->s));
+        c->mg_built = true;
+        return 0;
+    }
+    // dense inverse of (A_c + J/n) on the coarsest level (Gauss-Jordan,
+    // partial pivoting), FP64 on the host
+    const int n = (int)nc;
+    std::vector<double> A((size_t)n * n), I((size_t)n * n, 0.0), e(n), col(n);
+    for (int a = 0; a < n; a++) {
+        std::fill(e.begin(), e.end(), 0.0);
+        e[a] = 1.0;
+        level_apply_host(Lc, e.data(), col.data());
+        for (int r = 0; r < n; r++) A[(size_t)r * n + a] = col[r] + 1.0 / n;
+        I[(size_t)a * n + a] = 1.0;
+    }
+    for (int cc = 0; cc < n; cc++) {
+        int piv = cc;
+        for (int r = cc + 1; r < n; r++) if (fabs(A[(size_t)r * n + cc]) > fabs(A[(size_t)piv * n + cc])) piv = r;
+        if (piv != cc)
+            for (int k = 0; k < n; k++) {
+                std::swap(A[(size_t)cc * n + k], A[(size_t)piv * n + k]);
+                std::swap(I[(size_t)cc * n + k], I[(size_t)piv * n + k]);
+            }
+        double dd = 1.0 / A[(size_t)cc * n + cc];
+        for (int k = 0; k < n; k++) { A[(size_t)cc * n + k] *= dd; I[(size_t)cc * n + k] *= dd; }
+        for (int r = 0; r < n; r++) {
+            if (r == cc) continue;
+            double f = A[(size_t)r * n + cc];
+            if (f == 0.0) continue;
+            for (int k = 0; k < n; k++) { A[(size_t)r * n + k] -= f * A[(size_t)cc * n + k]; I[(size_t)r * n + k] -= f * I[(size_t)cc * n + k]; }
+        }
+    }
+    // stored transposed (column cc contiguous) so that the threads of the
+    // coarse solve, one per row, read consecutive addresses
+    std::vector<double> IT((size_t)n * n);
+    for (int r = 0; r < n; r++)
+        for (int cc = 0; cc < n; cc++) IT[(size_t)cc * n + r] = I[(size_t)r * n + cc];
+    I.swap(IT);
+    std::vector<float> I32((size_t)n * n);
+    for (size_t a = 0; a < I.size(); a++) I32[a] = (float)I[a];
+    TB_CHECK(c, hipMalloc((void **)&c->coarse_inv64, sizeof(double) * (size_t)n * n));
+    TB_CHECK(c, hipMalloc((void **)&c->coarse_inv32, sizeof(float) * (size_t)n * n));
+    TB_CHECK(c, hipMemcpy(c->coarse_inv64, I.data(), sizeof(double) * (size_t)n * n, hipMemcpyHostToDevice));
+    TB_CHECK(c, hipMemcpy(c->coarse_inv32, I32.data(), sizeof(float) * (size_t)n * n, hipMemcpyHostToDevice));
     TB_CHECK(c, hipStreamSynchronize(c->s));
     c->mg_built = true;
     return 0;
 }
 
+template <typename T>
 struct MGBuf {
-    double *x, *b, *r, *a;   // a: second iterate buffer of the fused-pair levels, else null
+    T *x, *b, *r, *a;   // a: second iterate buffer of the fused-pair levels, else null
 };
 
-static MGBuf bufs(tb_ctx *c, int l) { return {c->lev[l].x64, c->lev[l].b64, c->lev[l].r64, c->lev[l].a64}; }
+template <typename T>
+static MGBuf<T> bufs(tb_ctx *c, int l);
+template <>
+MGBuf<double> bufs<double>(tb_ctx *c, int l) { return {c->lev[l].x64, c->lev[l].b64, c->lev[l].r64, c->lev[l].a64}; }
+template <>
+MGBuf<float> bufs<float>(tb_ctx *c, int l) { return {c->lev[l].x32, c->lev[l].b32, c->lev[l].r32, c->lev[l].a32}; }
+
+template <typename T>
+static const T *coarse_inv(tb_ctx *c);
+template <>
+const double *coarse_inv<double>(tb_ctx *c) { return c->coarse_inv64; }
+template <>
+const float *coarse_inv<float>(tb_ctx *c) { return c->coarse_inv32; }
 
 // the column-walking transfer kernels serve large levels coarsened in y and
 // z (on small ones their plane-by-plane chains cost more than two launches)
@@ -1132,11 +1454,12 @@ static bool transfer_011(const Level &L) {
 }
 
 // x_f = x_in + P x_c from level l+1 to level l
-static void prolong(tb_ctx *c, int l, const double *xc, const double *xin, double *xf) {
+template <typename T>
+static void prolong(tb_ctx *c, int l, const T *xc, const T *xin, T *xf) {
     const Level &L = c->lev[l];
-    LV<double> lv = lv_of<double>(L);
+    LV<T> lv = lv_of<T>(L);
     const Level &Cl = c->lev[l + 1];
-    LV<double> cv = lv_of<double>(Cl);
+    LV<T> cv = lv_of<T>(Cl);
     if (transfer_011(L)) {
         KTiles t;
         t.nx = L.nx; t.ny = L.ny; t.nz = L.nz;
@@ -1145,23 +1468,23 @@ static void prolong(tb_ctx *c, int l, const double *xc, const double *xin, doubl
         t.kc = (L.nz + PR_KC - 1) / PR_KC;
         t.n = (long)t.tx * t.ty * t.kc;
         t.per_xcd = (t.n + NXCD - 1) / NXCD;
-        hipLaunchKernelGGL(k_prolong_011<double>, ktiles_grid(t), tiles_block(), 0, c->s, lv, cv, xc, xin, xf, t);
+        hipLaunchKernelGGL(k_prolong_011<T>, ktiles_grid(t), tiles_block(), 0, c->s, lv, cv, xc, xin, xf, t);
         return;
     }
     Tiles all = make_tiles(L.nx, L.ny, L.nz);
-    hipLaunchKernelGGL(k_prolong<double>, tiles_grid(all), tiles_block(), 0, c->s, lv, cv, L.cx, L.cy, L.cz, xc, xin, xf,
+    hipLaunchKernelGGL(k_prolong<T>, tiles_grid(all), tiles_block(), 0, c->s, lv, cv, L.cx, L.cy, L.cz, xc, xin, xf,
                        all);
 }
 
-// b of level l+1 from the residual of x on level l (fused for (0, 1, 1), else
-// through the buffer r)
-static void resid_restrict(tb_ctx *c, int l, const double *x, double *r) {
+// b of level l+1 from the residual of x on level l (fused for (0, 1, 1))
+template <typename T>
+static void resid_restrict(tb_ctx *c, int l, const T *x) {
     const Level &L = c->lev[l];
-    MGBuf B = bufs(c, l);
-    LV<double> lv = lv_of<double>(L);
+    MGBuf<T> B = bufs<T>(c, l);
+    LV<T> lv = lv_of<T>(L);
     const Level &Cl = c->lev[l + 1];
-    MGBuf CB = bufs(c, l + 1);
-    LV<double> cv = lv_of<double>(Cl);
+    MGBuf<T> CB = bufs<T>(c, l + 1);
+    LV<T> cv = lv_of<T>(Cl);
     if (transfer_011(L)) {
         KTiles t;
         t.nx = Cl.nx; t.ny = Cl.ny; t.nz = Cl.nz;
@@ -1170,226 +1493,309 @@ static void resid_restrict(tb_ctx *c, int l, const double *x, double *r) {
         t.kc = (Cl.nz + RR_KC - 1) / RR_KC;
         t.n = (long)t.tx * t.ty * t.kc;
         t.per_xcd = (t.n + NXCD - 1) / NXCD;
-        hipLaunchKernelGGL(k_resid_restrict_011<double>, ktiles_grid(t), tiles_block(), 0, c->s, lv, cv, x,
-                           (const double *)B.b, CB.b, t);
+        hipLaunchKernelGGL(k_resid_restrict_011<T>, ktiles_grid(t), tiles_block(), 0, c->s, lv, cv, x,
+                           (const T *)B.b, CB.b, t);
         return;
     }
     Tiles all = make_tiles(L.nx, L.ny, L.nz);
-    hipLaunchKernelGGL(k_mg_resid<double>, tiles_grid(all), tiles_block(), 0, c->s, lv, x, (const double *)B.b, r, all);
+    hipLaunchKernelGGL(k_mg_resid<T>, tiles_grid(all), tiles_block(), 0, c->s, lv, x, (const T *)B.b, B.r, all);
     Tiles call = make_tiles(Cl.nx, Cl.ny, Cl.nz);
-    const double *rc = r;
+    const T *r = B.r;
     const dim3 g = tiles_grid(call), blk = tiles_block();
     switch (L.cx * 4 + L.cy * 2 + L.cz) {
-    case 1: hipLaunchKernelGGL((k_restrict_t<double, 0, 0, 1>), g, blk, 0, c->s, lv, cv, rc, CB.b, call); break;
-    case 2: hipLaunchKernelGGL((k_restrict_t<double, 0, 1, 0>), g, blk, 0, c->s, lv, cv, rc, CB.b, call); break;
-    case 3: hipLaunchKernelGGL((k_restrict_t<double, 0, 1, 1>), g, blk, 0, c->s, lv, cv, rc, CB.b, call); break;
-    case 4: hipLaunchKernelGGL((k_restrict_t<double, 1, 0, 0>), g, blk, 0, c->s, lv, cv, rc, CB.b, call); break;
-    case 5: hipLaunchKernelGGL((k_restrict_t<double, 1, 0, 1>), g, blk, 0, c->s, lv, cv, rc, CB.b, call); break;
-    case 6: hipLaunchKernelGGL((k_restrict_t<double, 1, 1, 0>), g, blk, 0, c->s, lv, cv, rc, CB.b, call); break;
-    case 7: hipLaunchKernelGGL((k_restrict_t<double, 1, 1, 1>), g, blk, 0, c->s, lv, cv, rc, CB.b, call); break;
+    case 1: hipLaunchKernelGGL((k_restrict_t<T, 0, 0, 1>), g, blk, 0, c->s, lv, cv, r, CB.b, call); break;
+    case 2: hipLaunchKernelGGL((k_restrict_t<T, 0, 1, 0>), g, blk, 0, c->s, lv, cv, r, CB.b, call); break;
+    case 3: hipLaunchKernelGGL((k_restrict_t<T, 0, 1, 1>), g, blk, 0, c->s, lv, cv, r, CB.b, call); break;
+    case 4: hipLaunchKernelGGL((k_restrict_t<T, 1, 0, 0>), g, blk, 0, c->s, lv, cv, r, CB.b, call); break;
+    case 5: hipLaunchKernelGGL((k_restrict_t<T, 1, 0, 1>), g, blk, 0, c->s, lv, cv, r, CB.b, call); break;
+    case 6: hipLaunchKernelGGL((k_restrict_t<T, 1, 1, 0>), g, blk, 0, c->s, lv, cv, r, CB.b, call); break;
+    case 7: hipLaunchKernelGGL((k_restrict_t<T, 1, 1, 1>), g, blk, 0, c->s, lv, cv, r, CB.b, call); break;
+    default:
+        hipLaunchKernelGGL(k_restrict<T>, g, blk, 0, c->s, lv, cv, L.cx, L.cy, L.cz, r, CB.b, call);
+        break;
     }
 }
 
 // symmetric sweep pairs from zero on a coarsest level too large for the
-// direct solve (tb_spec_usable): forward pairs, then as many backward ones
+// dense inverse (mg_build): forward pairs, then as many backward ones
 constexpr int COARSE_SWEEPS = 50;
 
 // the two kinds of blocked launch: pre-smoothing from zero, prolongation +
 // post-smoothing
 enum { BLK_ZERO = 0, BLK_PROL };
 
-template <int NP>
-static void launch_blk_np(tb_ctx *c, const dim3 &grid, int lds, int kind, const LV<double> &lv, const double *src,
-                          const double *b, double *dst, const BlkShape &S, const LV<double> &cv, const Level &L,
-                          const double *xc) {
+template <typename T, int NP>
+static void launch_blk_np(tb_ctx *c, const dim3 &grid, int lds, int kind, const LV<T> &lv, const T *src,
+                          const T *b, T *dst, const BlkShape &S, const LV<T> &cv, const Level &L, const T *xc) {
     const dim3 blk(BLK_THREADS);
     if (kind == BLK_ZERO)
-        hipLaunchKernelGGL((k_rbgs_blk<double, NP, true, false, 0>), grid, blk, lds, c->s, lv, src, b, dst, S, cv,
-                           L.cx, L.cy, L.cz, xc, nullptr);
+        hipLaunchKernelGGL((k_rbgs_blk<T, NP, true, false, 0>), grid, blk, lds, c->s, lv, src, b, dst, S, cv, L.cx,
+                           L.cy, L.cz, xc);
     else
-        hipLaunchKernelGGL((k_rbgs_blk<double, NP, false, true, 1>), grid, blk, lds, c->s, lv, src, b, dst, S, cv,
-                           L.cx, L.cy, L.cz, xc, c->red);
+        hipLaunchKernelGGL((k_rbgs_blk<T, NP, false, true, 1>), grid, blk, lds, c->s, lv, src, b, dst, S, cv, L.cx,
+                           L.cy, L.cz, xc);
 }
 
-// returns the number of boxes
-static int launch_blk(tb_ctx *c, int l, int np, int kind, const double *src, double *dst, const double *xc) {
+template <typename T>
+static void launch_blk(tb_ctx *c, int l, int np, int kind, const T *src, T *dst, const T *xc) {
     const Level &L = c->lev[l];
-    const LV<double> lv = lv_of<double>(L), cv = lv_of<double>(c->lev[l + 1]);
-    const double *b = L.b64;
+    MGBuf<T> B = bufs<T>(c, l);
+    LV<T> lv = lv_of<T>(L);
+    const Level &Cl = c->lev[l + 1];
+    LV<T> cv = lv_of<T>(Cl);
     BlkShape S;
     int lds = 0;
-    blk_shape(L, np, sizeof(double), S, lds);   // checked by blk_usable
+    blk_shape(L, np, sizeof(T), S, lds);   // checked by blk_usable
     const dim3 grid((unsigned)(S.per_xcd * NXCD));
-    if (np == 1) launch_blk_np<1>(c, grid, lds, kind, lv, src, b, dst, S, cv, L, xc);
-    else launch_blk_np<2>(c, grid, lds, kind, lv, src, b, dst, S, cv, L, xc);
-    return S.nb;
+    if (np == 1) launch_blk_np<T, 1>(c, grid, lds, kind, lv, src, (const T *)B.b, dst, S, cv, L, xc);
+    else launch_blk_np<T, 2>(c, grid, lds, kind, lv, src, (const T *)B.b, dst, S, cv, L, xc);
 }
 
-// the blocked smoother serves a finest level of at most BLK_MAX_CELLS cells,
-// with 1 or 2 sweep pairs per side and a box whose LDS fits
-static bool blk_usable(const tb_ctx *c, int l, int pre, int post) {
-    if (!c->mg_blocked || l != 0 || pre < 1 || pre > 2 || post < 1 || post > 2 || c->lev[l].pairs) return false;
+// the blocked smoother serves a level below the finest without fused pairs
+// that has at most BLK_MAX_CELLS cells, with 1 or 2 sweep pairs per side and
+// a box whose LDS fits
+static bool blk_usable(const tb_ctx *c, int l, int pre, int post, size_t tsize) {
+    if (!c->mg_blocked || l == 0 || pre < 1 || pre > 2 || post < 1 || post > 2 || c->lev[l].pairs) return false;
     if ((long)c->lev[l].nx * c->lev[l].ny * c->lev[l].nz > BLK_MAX_CELLS) return false;
     BlkShape S;
     int lds = 0;
-    return blk_shape(c->lev[l], pre, sizeof(double), S, lds) && blk_shape(c->lev[l], post, sizeof(double), S, lds);
+    return blk_shape(c->lev[l], pre, tsize, S, lds) && blk_shape(c->lev[l], post, tsize, S, lds);
 }
 
-// One V-cycle from level l down, b64 -> x64.
-static int vcycle_level(tb_ctx *c, int l) {
+// One V-cycle from level l down; *res receives the buffer that holds the
+// level's result (x, or r for the blocked smoother, whose post-smoother
+// cannot overwrite the x its neighbours' halos read).
+template <typename T>
+static int vcycle_level(tb_ctx *c, int l, const T **res) {
     const Level &L = c->lev[l];
-    const MGBuf B = bufs(c, l);
-    const LV<double> lv = lv_of<double>(L);
-    if (l == 0) c->vc_dot_blocks = 0;
-    const Tiles half = make_tiles((L.nx + 1) / 2, L.ny, L.nz);
-    const int kid = (l == 0) ? TB_K_RBGS0 : TB_K_MG_LEVELS;
-    auto sweep = [&](int id, int color, int zero_init) {
-        TB_PROF(c, id,
-                hipLaunchKernelGGL(k_rbgs<double>, tiles_grid(half), tiles_block(), 0, c->s, lv, B.x,
-                                   (const double *)B.b, color, zero_init, half));
-    };
-    if (l == c->nlev - 1) {
-        if (c->coarse_direct) {
-            if (c->prof_on) tb_prof_begin(c, TB_K_MG_SMALL);
-            if (tb_spec_solve<double>(c, L, B.b, B.x)) return -1;
-            if (c->prof_on) tb_prof_end(c, TB_K_MG_SMALL);
-            return 0;
-        }
-        sweep(TB_K_MG_SMALL, 0, 1);
-        sweep(TB_K_MG_SMALL, 1, 0);
+    MGBuf<T> B = bufs<T>(c, l);
+    LV<T> lv = lv_of<T>(L);
+    if (l == 0) c->vc_dot_blocks[sizeof(T) == 8 ? 1 : 0] = 0;
+    if (l == c->nlev - 1 && !c->coarse_dense) {
+        const Tiles half = make_tiles((L.nx + 1) / 2, L.ny, L.nz);
+        auto sweep = [&](int color, int zero_init) {
+            TB_PROF(c, TB_K_MG_SMALL,
+                    hipLaunchKernelGGL(k_rbgs<T>, tiles_grid(half), tiles_block(), 0, c->s, lv, B.x, (const T *)B.b,
+                                       color, zero_init, half));
+        };
+        sweep(0, 1);
+        sweep(1, 0);
         for (int s = 1; s < COARSE_SWEEPS; s++) {
-            sweep(TB_K_MG_SMALL, 0, 0);
-            sweep(TB_K_MG_SMALL, 1, 0);
+            sweep(0, 0);
+            sweep(1, 0);
         }
         for (int s = 0; s < COARSE_SWEEPS; s++) {
-            sweep(TB_K_MG_SMALL, 1, 0);
-            sweep(TB_K_MG_SMALL, 0, 0);
+            sweep(1, 0);
+            sweep(0, 0);
         }
         TB_LAUNCH_CHECK(c);
+        *res = B.x;
         return 0;
     }
-    const double *xc = c->lev[l + 1].x64;
-    const int pre = (l == 0 && c->mg_pre0 > 0) ? c->mg_pre0 : c->cfg.mg_pre;
-    const int post = (l == 0 && c->mg_post0 > 0) ? c->mg_post0 : c->cfg.mg_post;
+    if (l == c->small_l0[sizeof(T) == 8 ? 1 : 0]) {
+        SmallCycle<T> A;
+        A.l0 = l;
+        A.nl = c->nlev;
+        A.pre = c->cfg.mg_pre;
+        A.post = c->cfg.mg_post;
+        A.coarse_n = c->coarse_n;
+        A.Minv = coarse_inv<T>(c);
+        A.g0 = lv;
+        A.gx0 = B.x;
+        A.gb0 = B.b;
+        int off = 0;
+        for (int m = l; m < c->nlev; m++) {
+            const Level &Lm = c->lev[m];
+            LV<T> v = lv_of<T>(Lm);
+            v.px = Lm.nx;
+            v.py = Lm.ny;
+            A.lv[m] = v;
+            A.xo[m] = off; off += Lm.nx * Lm.ny * Lm.nz;
+            A.bo[m] = off; off += Lm.nx * Lm.ny * Lm.nz;
+            A.cx[m] = Lm.cx; A.cy[m] = Lm.cy; A.cz[m] = Lm.cz;
+        }
+        A.ro = off;
+        TB_PROF(c, TB_K_MG_SMALL,
+                hipLaunchKernelGGL(k_small_cycle<T>, dim3(1), dim3(1024), small_lds_bytes<T>(c, l), c->s, A));
+        TB_LAUNCH_CHECK(c);
+        *res = B.x;
+        return 0;
+    }
+    Tiles all = make_tiles(L.nx, L.ny, L.nz);
+    Tiles half = make_tiles((L.nx + 1) / 2, L.ny, L.nz);
+    const int kid = (l == 0) ? (sizeof(T) == 8 ? TB_K_RBGS0 : TB_K_RBGS0_F32) : TB_K_MG_LEVELS;
+    const int prec = sizeof(T) == 8 ? 1 : 0;
+    const int pre = (l == 0 && c->mg_pre0[prec] > 0) ? c->mg_pre0[prec] : c->cfg.mg_pre;
+    const int post = (l == 0 && c->mg_post0[prec] > 0) ? c->mg_post0[prec] : c->cfg.mg_post;
     // large levels: fused sweep pairs alternating between x and the level's
     // second buffer; cur is the buffer holding the current iterate
-    if (L.pairs) {
+    const bool pairs = L.pairs;
+    T *cur = B.x;
+    if (pairs) {
         const PairTiles P = make_pair_tiles(L.nx, L.ny, L.nz, pair_chunk(L));
         const dim3 grid(P.per_xcd * NXCD), blk(PAIR_THREADS);
-        double *cur = B.x;
-        auto pair = [&](int first, bool zero, bool dot) {
-            double *dst = zero ? B.x : (cur == B.x ? B.a : B.x);
-            const double *src = cur, *bb = B.b;
-            if (c->prof_on) tb_prof_begin(c, kid);
-            if (zero) hipLaunchKernelGGL((k_rbgs_pair<double, 0, true, false>), grid, blk, 0, c->s, lv, src, dst, bb, P, nullptr);
-            else if (first == 0) hipLaunchKernelGGL((k_rbgs_pair<double, 0, false, false>), grid, blk, 0, c->s, lv, src, dst, bb, P, nullptr);
-            else if (!dot) hipLaunchKernelGGL((k_rbgs_pair<double, 1, false, false>), grid, blk, 0, c->s, lv, src, dst, bb, P, nullptr);
-            else hipLaunchKernelGGL((k_rbgs_pair<double, 1, false, true>), grid, blk, 0, c->s, lv, src, dst, bb, P, c->red);
-            if (c->prof_on) tb_prof_end(c, kid);
+        // the first post pair forms the prolongation itself on (0, 1, 1)
+        // levels; the pairs then write pre + post times, so the first one
+        // goes to the buffer that makes the last one land in x
+        const bool fuse = sizeof(T) == 4 && c->mg_blocked && transfer_011(L) && pre > 0 && post > 0;
+        T *zdst = (fuse && (pre + post) % 2 == 0) ? B.a : B.x;
+        const Level &Cl = c->lev[l + 1];
+        const LV<T> cv = lv_of<T>(Cl);
+        auto pair = [&](int first, bool zero, bool dot, const T *pxc) {
+            T *dst = zero ? zdst : (cur == B.x ? B.a : B.x);
+            const T *src = cur;
+            const T *bb = B.b;
+            if (c->prof_on && kid >= 0) tb_prof_begin(c, kid);
+            if (zero) hipLaunchKernelGGL((k_rbgs_pair<T, 0, true, false>), grid, blk, 0, c->s, lv, src, dst, bb, P, nullptr, lv, nullptr);
+            else if (first == 0) hipLaunchKernelGGL((k_rbgs_pair<T, 0, false, false>), grid, blk, 0, c->s, lv, src, dst, bb, P, nullptr, lv, nullptr);
+            else if (pxc) {
+                // FP32 only: the FP64 form needs more registers than two blocks per CU leave
+                if constexpr (sizeof(T) == 4) {
+                    if (!dot) hipLaunchKernelGGL((k_rbgs_pair<T, 1, false, false, true>), grid, blk, 0, c->s, lv, src, dst, bb, P, nullptr, cv, pxc);
+                    else hipLaunchKernelGGL((k_rbgs_pair<T, 1, false, true, true>), grid, blk, 0, c->s, lv, src, dst, bb, P, c->red, cv, pxc);
+                }
+            } else if (!dot) hipLaunchKernelGGL((k_rbgs_pair<T, 1, false, false>), grid, blk, 0, c->s, lv, src, dst, bb, P, nullptr, lv, nullptr);
+            else hipLaunchKernelGGL((k_rbgs_pair<T, 1, false, true>), grid, blk, 0, c->s, lv, src, dst, bb, P, c->red, lv, nullptr);
+            if (c->prof_on && kid >= 0) tb_prof_end(c, kid);
             cur = dst;
         };
-        pair(0, true, false);
-        for (int s = 1; s < pre; s++) pair(0, false, false);
-        TB_PROF(c, TB_K_MG_TRANSFER, resid_restrict(c, l, cur, B.r));
+        if (pre > 0) {
+            pair(0, true, false, nullptr);
+            for (int s = 1; s < pre; s++) pair(0, false, false, nullptr);
+        } else {
+            hipLaunchKernelGGL(k_zero<T>, tiles_grid(all), tiles_block(), 0, c->s, lv, B.x, all);
+        }
+        TB_PROF(c, TB_K_MG_TRANSFER, resid_restrict<T>(c, l, (const T *)cur));
         TB_LAUNCH_CHECK(c);
-        if (vcycle_level(c, l + 1)) return -1;
-        // the post pairs alternate buffers, so the prolonged iterate goes
-        // to the buffer from which they end in x
-        double *dst = (post % 2 == 0) ? B.x : B.a;
-        TB_PROF(c, TB_K_MG_TRANSFER, prolong(c, l, xc, cur, dst));
-        cur = dst;
+        const T *xc = nullptr;
+        if (vcycle_level<T>(c, l + 1, &xc)) return -1;
+        if (!fuse) {
+            // the post pairs alternate buffers, so the prolonged iterate goes
+            // to the buffer from which they end in x
+            T *dst = (post % 2 == 0) ? B.x : B.a;
+            TB_PROF(c, TB_K_MG_TRANSFER, prolong<T>(c, l, xc, (const T *)cur, dst));
+            cur = dst;
+        }
         // on the finest level the last pair also forms the partial sums of
-        // r . z (b . x), z and r for the Krylov method around the cycle
-        for (int s = 0; s < post; s++) pair(1, false, l == 0 && s == post - 1);
-        if (l == 0) c->vc_dot_blocks = (int)(P.per_xcd * NXCD);
+        // r . z (b . x) for the Krylov method around the cycle
+        const bool dot = l == 0 && post > 0;
+        for (int s = 0; s < post; s++) pair(1, false, dot && s == post - 1, (fuse && s == 0) ? xc : nullptr);
+        if (l == 0) {
+            c->vc_dot_blocks[sizeof(T) == 8 ? 1 : 0] = dot ? (int)(P.per_xcd * NXCD) : 0;
+        }
         TB_LAUNCH_CHECK(c);
+        *res = B.x;
         return 0;
     }
-    if (blk_usable(c, l, pre, post)) {
-        // pre-smoother from x = 0 into r (the residual goes to kv[5]), then
-        // prolongation + post-smoother from r into x: its neighbours' halos
-        // read r, so it cannot work in place
-        TB_PROF(c, kid, launch_blk(c, l, pre, BLK_ZERO, nullptr, B.r, nullptr));
-        TB_PROF(c, TB_K_MG_TRANSFER, resid_restrict(c, l, B.r, c->kv[5]));
+    if (blk_usable(c, l, pre, post, sizeof(T))) {
+        // pre-smoother from x = 0 into x, residual and restriction, the
+        // coarse levels, then prolongation + post-smoother from x into r
+        TB_PROF(c, kid, launch_blk<T>(c, l, pre, BLK_ZERO, nullptr, B.x, nullptr));
+        TB_PROF(c, TB_K_MG_TRANSFER, resid_restrict<T>(c, l, (const T *)B.x));
         TB_LAUNCH_CHECK(c);
-        if (vcycle_level(c, l + 1)) return -1;
-        TB_PROF(c, kid, c->vc_dot_blocks = launch_blk(c, l, post, BLK_PROL, B.r, B.x, xc));
+        const T *xc = nullptr;
+        if (vcycle_level<T>(c, l + 1, &xc)) return -1;
+        TB_PROF(c, kid, launch_blk<T>(c, l, post, BLK_PROL, (const T *)B.x, B.r, xc));
         TB_LAUNCH_CHECK(c);
+        *res = B.r;
         return 0;
     }
+    auto smooth = [&](int color, int zero_init) {
+        if (c->prof_on && kid >= 0) tb_prof_begin(c, kid);
+        hipLaunchKernelGGL(k_rbgs<T>, tiles_grid(half), tiles_block(), 0, c->s, lv, B.x, (const T *)B.b, color,
+                           zero_init, half);
+        if (c->prof_on && kid >= 0) tb_prof_end(c, kid);
+    };
     // zero initial guess: the first red half sweep reads no neighbour and
     // the black one only red cells, so x needs no clearing pass
-    sweep(kid, 0, 1);
-    sweep(kid, 1, 0);
-    for (int s = 1; s < pre; s++) {
-        sweep(kid, 0, 0);
-        sweep(kid, 1, 0);
+    if (pre > 0) {
+        smooth(0, 1);
+        smooth(1, 0);
+        for (int s = 1; s < pre; s++) {
+            smooth(0, 0);
+            smooth(1, 0);
+        }
+    } else {
+        hipLaunchKernelGGL(k_zero<T>, tiles_grid(all), tiles_block(), 0, c->s, lv, B.x, all);
     }
-    TB_PROF(c, TB_K_MG_TRANSFER, resid_restrict(c, l, B.x, B.r));
+    TB_PROF(c, TB_K_MG_TRANSFER, resid_restrict<T>(c, l, (const T *)B.x));
     TB_LAUNCH_CHECK(c);
-    if (vcycle_level(c, l + 1)) return -1;
-    TB_PROF(c, TB_K_MG_TRANSFER, prolong(c, l, xc, B.x, B.x));
+    const T *xc = nullptr;
+    if (vcycle_level<T>(c, l + 1, &xc)) return -1;
+    TB_PROF(c, TB_K_MG_TRANSFER, prolong<T>(c, l, xc, (const T *)B.x, B.x));
     for (int s = 0; s < post; s++) {
-        sweep(kid, 1, 0);
-        sweep(kid, 0, 0);
+        smooth(1, 0);
+        smooth(0, 0);
     }
     TB_LAUNCH_CHECK(c);
+    *res = B.x;
     return 0;
 }
 
-static void drop_graph(tb_ctx *c) {
-    if (c->vc_exec) hipGraphExecDestroy(c->vc_exec);
-    c->vc_exec = nullptr;
-}
-
-// z = V(r) in FP64 with level 0 aliased onto the padded vectors.  The cycle
-// is captured once into a HIP graph and replayed with one launch (kernels
-// only, no memset nodes).  Profiling runs launch the kernels directly, so
-// their events are recorded.
-int tb_vcycle64(tb_ctx *c, const double *r_pad, double *z_pad) {
-    if (tb_mg_build(c)) return -1;
-    Level &L0 = c->lev[0];
-    const bool same = L0.b64 == r_pad && L0.x64 == z_pad && L0.r64 == c->kv[4];
-    if (!same) drop_graph(c);            // captured with other level-0 vectors
-    L0.b64 = const_cast<double *>(r_pad);
-    L0.x64 = z_pad;
-    L0.r64 = c->kv[4];
-    if (!c->use_graphs || c->prof_on) return vcycle_level(c, 0);
-    if (!c->vc_exec) {
+// z = V(r) in FP64 with level 0 aliased onto the padded vectors
+// A V-cycle is ~10 levels x ~12 launches, most of them on grids far too
+// small to fill the chip, so it is captured once into a HIP graph and
+// replayed with one launch.  The graph holds kernels only (no memset nodes).
+// Profiling runs launch the kernels directly, so their events are recorded.
+template <typename T>
+static int vcycle_run(tb_ctx *c, int which) {
+    const T *res = nullptr;
+    if (!c->use_graphs || c->prof_on) return vcycle_level<T>(c, 0, &res);
+    if (!c->vc_exec[which]) {
         hipGraph_t g = nullptr;
         TB_CHECK(c, hipStreamBeginCapture(c->s, hipStreamCaptureModeThreadLocal));
-        const int rc = vcycle_level(c, 0);
+        const int rc = vcycle_level<T>(c, 0, &res);
         const hipError_t e = hipStreamEndCapture(c->s, &g);
         if (rc || e != hipSuccess) {
             if (e == hipSuccess && g) hipGraphDestroy(g);
             if (!rc) c->err = std::string("V-cycle capture: ") + hipGetErrorString(e);
             return -1;
         }
-        const hipError_t ei = hipGraphInstantiate(&c->vc_exec, g, nullptr, nullptr, 0);
+        hipGraphExec_t ex = nullptr;
+        const hipError_t ei = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
         hipGraphDestroy(g);
-        if (ei != hipSuccess) {
-            c->vc_exec = nullptr;
-            c->err = std::string("V-cycle graph: ") + hipGetErrorString(ei);
-            return -1;
-        }
+        if (ei != hipSuccess) { c->err = std::string("V-cycle graph: ") + hipGetErrorString(ei); return -1; }
+        c->vc_exec[which] = ex;
     }
-    TB_CHECK(c, hipGraphLaunch(c->vc_exec, c->s));
+    TB_CHECK(c, hipGraphLaunch(c->vc_exec[which], c->s));
     return 0;
 }
 
-// sweeps (or sweep pairs) on the finest level of the V-cycle; 0 keeps
-// cfg.mg_pre / cfg.mg_post there.  The FP32 pair of numbers is checked and
-// has no effect: the mixed solve's FP32 part is direct.  A captured V-cycle is
-// dropped.
+int tb_vcycle64(tb_ctx *c, const double *r_pad, double *z_pad) {
+    if (tb_mg_build(c)) return -1;
+    const bool same = c->lev[0].b64 == r_pad && c->lev[0].x64 == z_pad && c->lev[0].r64 == c->kv[4];
+    if (!same && c->vc_exec[0]) {        // captured with other level-0 vectors
+        hipGraphExecDestroy(c->vc_exec[0]);
+        c->vc_exec[0] = nullptr;
+    }
+    c->lev[0].b64 = const_cast<double *>(r_pad);
+    c->lev[0].x64 = z_pad;
+    c->lev[0].r64 = c->kv[4];
+    return vcycle_run<double>(c, 0);
+}
+
+// lev[0].x32 = V(lev[0].b32) in FP32
+int tb_vcycle32(tb_ctx *c) {
+    if (tb_mg_build(c)) return -1;
+    return vcycle_run<float>(c, 1);
+}
+
+// sweeps (or sweep pairs) on the finest level of the FP32 / FP64 V-cycles;
+// 0 keeps cfg.mg_pre / cfg.mg_post there.  Captured V-cycles are dropped.
 extern "C" int tb_set_mg_finest_sweeps(tb_ctx *c, int pre32, int post32, int pre64, int post64) {
     if (!c) return -1;
     if (pre32 < 0 || post32 < 0 || pre64 < 0 || post64 < 0 || pre32 > 8 || post32 > 8 || pre64 > 8 || post64 > 8) {
         c->err = "tb_set_mg_finest_sweeps: sweeps must be 0..8";
         return -1;
     }
-    c->mg_pre0 = pre64;
-    c->mg_post0 = post64;
-    drop_graph(c);
+    c->mg_pre0[0] = pre32;
+    c->mg_post0[0] = post32;
+    c->mg_pre0[1] = pre64;
+    c->mg_post0[1] = post64;
+    for (int a = 0; a < 2; a++) {
+        if (c->vc_exec[a]) hipGraphExecDestroy(c->vc_exec[a]);
+        c->vc_exec[a] = nullptr;
+    }
     return 0;
 }
 
@@ -1400,7 +1806,10 @@ extern "C" int tb_set_mg_smoother(tb_ctx *c, int blocked) {
         return -1;
     }
     c->mg_blocked = blocked != 0;
-    drop_graph(c);
+    for (int a = 0; a < 2; a++) {
+        if (c->vc_exec[a]) hipGraphExecDestroy(c->vc_exec[a]);
+        c->vc_exec[a] = nullptr;
+    }
     return 0;
 }
 
@@ -1415,180 +1824,12 @@ extern "C" int tb_set_graphs(tb_ctx *c, int on) {
 constexpr int PB = 1024;
 constexpr int PT = 256;
 
-// Up to this many partial sums are added up by every block that needs the
-// total instead of a launch of its own (5 us and a gap against about 1 us of
-// loads from L2 at 512).
-constexpr int SUM_INLINE = 512;
-
-// the totals of nb partial sums of NV of red's arrays in every thread
-// (a 256-thread block; sh: NV * 16 doubles)
-template <int NV>
-__device__ inline void inline_sum(const double *red, int nb, double (&v)[NV], double *sh) {
-#pragma unroll
-    for (int a = 0; a < NV; a++) {
-        v[a] = 0.0;
-        for (int b = threadIdx.y * blockDim.x + threadIdx.x; b < nb; b += 256) v[a] += red[a * (long)RED_MAX_BLOCKS + b];
-    }
-    block_sum<NV>(v, sh);
-    if (threadIdx.x == 0 && threadIdx.y == 0)
-#pragma unroll
-        for (int a = 0; a < NV; a++) sh[a * 16] = v[a];
-    __syncthreads();
-#pragma unroll
-    for (int a = 0; a < NV; a++) v[a] = sh[a * 16];
-    __syncthreads();   // sh is free again
-}
-
-// red's array of the partial sums of p . q: blocks of the kernel that writes
-// it may still read the first three
-constexpr int PQ_ARRAY = 3;
-
-// beta of the direction update p = (z - mean z) + beta p from the sums of
-// r . z, z and r: rz_new / rz_old with rz_new = r . (z - mean z), stored in the
-// scalar slot rz_new (another one than rz_old, which every block reads).  The
-// V-cycle's output has an arbitrary mean and the operator does not see it:
-// left in, it lets the rounding of r's own mean into beta, and solves whose
-// right-hand side is small stagnated (200 iterations instead of 11 at
-// 64x16x16).
-__device__ inline void pcg_beta(const double (&sums)[3], double *s, int rz_old, int rz_new, bool first, double ncell,
-                                bool store, double &mean, double &beta) {
-    mean = sums[1] / ncell;
-    const double rzn = sums[0] - mean * sums[2];
-    beta = first || s[rz_old] == 0.0 ? 0.0 : rzn / s[rz_old];
-    if (store) s[rz_new] = rzn;
-}
-
-// the same by one block into the slots S_MEAN and S_BETA, for more than
-// SUM_INLINE partial sums; the many blocks of a large grid then start from two
-// loads (with the totals' loads and the divisions in each block the update
-// below took 107 us at 512x128x128)
-__global__ void __launch_bounds__(1024) k_pcg_beta(const double *__restrict__ part, int nb, double *s, int rz_old,
-                                                   int rz_new, int first, double ncell) {
-    __shared__ double sh[48];
-    double v[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-        for (int b = threadIdx.x; b < nb; b += 1024) v[a] += part[a * (long)RED_MAX_BLOCKS + b];
-    block_sum<3>(v, sh);
-    if (threadIdx.x != 0) return;
-    double mean, beta;
-    pcg_beta(v, s, rz_old, rz_new, first != 0, ncell, true, mean, beta);
-    s[S_MEAN] = mean;
-    s[S_BETA] = beta;
-}
-
-// The direction update on the cells, in place (no p term when first), from
-// S_MEAN and S_BETA
-__global__ void __launch_bounds__(256) k_pcg_p(Dims d, const double *__restrict__ z, double *__restrict__ p,
-                                               const double *__restrict__ s, int first, Tiles t) {
-    const double mean = s[S_MEAN], beta = s[S_BETA];
-    int i, j, k;
-    if (!tile_point(t, i, j, k)) return;
-    const long id = gidx(d, i, j, k);
-    const double v = z[id] - mean;
-    p[id] = first ? v : v + beta * p[id];
-}
-
-// Cells up to which the direction update and the operator are one pass: it
-// forms each neighbour's p again, twice the operator's loads, for a launch
-// fewer.  Steps with the sums added up in place, fused and in two passes: 1.34
-// and 1.49 ms at 64x16x16, 2.28 / 2.36 at 128x64x32, 2.85 / 2.87 at 192x64x64,
-// 8.20 / 8.05 at 512x128x64, 13.08 / 12.94 at 512x128x128.
-constexpr long PCG_FUSED_CELLS = 1L << 20;
-
-// The direction update and the operator in one pass:
-// p = (z - mean z) + beta po on the cells (0 on the half-cell planes; no po
-// term when FIRST), q = A p, partial p . q.  A neighbour's p is formed from z
-// and po by the same expression; po and p are two buffers.
-template <bool FIRST, bool INLINE>
-__global__ void __launch_bounds__(256) k_pcg_pa(PoisOp P, const double *__restrict__ z, const double *__restrict__ po,
-                                                double *__restrict__ p, double *__restrict__ q, int nsum, double *s,
-                                                int rz_old, int rz_new, double ncell, double *red, KTiles t) {
-    __shared__ double sh[48];
-    double mean, beta;
-    if (INLINE) {
-        double sums[3];
-        inline_sum<3>(red, nsum, sums, sh);
-        pcg_beta(sums, s, rz_old, rz_new, FIRST, ncell, blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0, mean,
-                 beta);
-    } else {
-        mean = s[S_MEAN];
-        beta = s[S_BETA];
-    }
-    double acc[1] = {0.0};
-    int i, j, k0, k1;
-    bool act;
-    ktile_column(t, i, j, k0, k1, act);
-    if (act) {
-        const Dims &d = P.d;
-        const GridDev &g = P.g;
-        const int NI = d.NX - 1, NJ = d.NY - 1, NK = d.NZ - 1;
-        const bool bnd_col = (i == NI) || (j == NJ);
-        const double Cx = P.Cx, Cy = P.Cy, Cz = P.Cz;
-        const int ip1 = i + 1 <= NI ? i + 1 : NI, jp1 = j + 1 <= NJ ? j + 1 : NJ;
-        const double mpx = g.mxc[i], mex = g.mxu[ip1], mwx = g.mxu[i];
-        const double mpy = g.myc[j], mny = g.myv[jp1], msy = g.myv[j];
-        const double axy = -Cx * mpx * (mex + mwx) - Cy * mpy * (mny + msy);
-        const double aw = Cx * mpx * mwx, ae = Cx * mpx * mex, an = Cy * mpy * mny, as = Cy * mpy * msy;
-        const bool hs = j > 0, hw = i > 0, he = i < NI - 1, hn = j < NJ - 1;
-        // absent neighbours are clamped to the point itself (zero coefficient
-        // below), so all loads are issued unconditionally
-        const long os = hs ? d.px : 0, on = hn ? d.px : 0, ow = hw ? 1 : 0, oe = he ? 1 : 0;
-        auto dir = [&](long e) {
-            const double v = z[e] - mean;
-            return FIRST ? v : v + beta * po[e];
-        };
-        long id = gidx(d, i, j, k0);
-        double xm = dir(id - ((k0 > 0) ? d.plane : 0)), xc = dir(id);
-        for (int k = k0; k < k1; k++) {
-            const double xp = dir(id + ((k + 1 < NK) ? d.plane : 0));
-            const double xs = dir(id - os), xw = dir(id - ow), xe = dir(id + oe), xn = dir(id + on);
-            if (bnd_col || k == NK) {
-                p[id] = 0.0;
-                st_stream(&q[id], 0.0);
-            } else {
-                const double mpz = g.mzc[k], mfz = g.mzw[k + 1], mbz = g.mzw[k];
-                double ap = axy - Cz * mpz * (mbz + mfz);
-                const double ab = Cz * mpz * mbz, af = Cz * mpz * mfz;
-                const bool hb = k > 0, hf = k < NK - 1;
-                if (!hb) ap += ab;
-                if (!hs) ap += as;
-                if (!hw) ap += aw;
-                if (!he) ap += ae;
-                if (!hn) ap += an;
-                if (!hf) ap += af;
-                double r = 0.0;
-                r = hb ? r + ab * xm : r;
-                r = hs ? r + as * xs : r;
-                r = hw ? r + aw * xw : r;
-                r += ap * xc;
-                r = he ? r + ae * xe : r;
-                r = hn ? r + an * xn : r;
-                r = hf ? r + af * xp : r;
-                p[id] = xc;
-                st_stream(&q[id], r);
-                acc[0] += xc * r;
-            }
-            xm = xc;
-            xc = xp;
-            id += d.plane;
-        }
-    }
-    block_sum<1>(acc, sh);
-    if (threadIdx.x == 0 && threadIdx.y == 0) red[PQ_ARRAY * (long)RED_MAX_BLOCKS + blockIdx.x] = acc[0];
-}
-
-// x += alpha p ; r -= alpha q ; partial r.r      (alpha = rz / pq; 0 where the
-// direction vanishes, r then being a constant the operator cannot reduce)
-template <bool INLINE>
-__global__ void __launch_bounds__(PT) k_pcg_xr(long n, double *__restrict__ x, double *__restrict__ r,
-                                               const double *__restrict__ p, const double *__restrict__ q, int nsum,
-                                               const double *__restrict__ s, int rz, double *red) {
+// x += alpha p ; r -= alpha q ; partial r.r      (alpha = rz / pq)
+__global__ void k_pcg_xr(long n, double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
+                         const double *__restrict__ q, const double *__restrict__ s, double *part) {
     __shared__ double sh[16];
-    double acc[1];
-    if (INLINE) inline_sum<1>(red + PQ_ARRAY * (long)RED_MAX_BLOCKS, nsum, acc, sh);
-    const double pq = INLINE ? acc[0] : s[S_PQ], alpha = pq == 0.0 ? 0.0 : s[rz] / pq;
-    acc[0] = 0.0;
+    double alpha = s[S_RZ] / s[S_PQ];
+    double acc[1] = {0.0};
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         x[i] += alpha * p[i];
         double ri = r[i] - alpha * q[i];
@@ -1596,22 +1837,19 @@ __global__ void __launch_bounds__(PT) k_pcg_xr(long n, double *__restrict__ x, d
         acc[0] += ri * ri;
     }
     block_sum<1>(acc, sh);
-    if (threadIdx.x == 0) red[blockIdx.x] = acc[0];
+    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
 }
 
-// partial sums of r . z, z and r
-__global__ void k_pcg_rz(long n, const double *__restrict__ r, const double *__restrict__ z, double *part) {
-    __shared__ double sh[48];
-    double acc[3] = {0.0, 0.0, 0.0};
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const double ri = r[i], zi = z[i];
-        acc[0] += ri * zi;
-        acc[1] += zi;
-        acc[2] += ri;
-    }
-    block_sum<3>(acc, sh);
-    if (threadIdx.x == 0)
-        for (int a = 0; a < 3; a++) part[a * RED_MAX_BLOCKS + blockIdx.x] = acc[a];
+// p = z + beta p with beta = rz_new / rz ; rz <- rz_new (thread 0 of block 0
+// writes it after every block has read the old value: done by the next launch)
+__global__ void k_pcg_p(long n, const double *__restrict__ z, double *__restrict__ p, const double *__restrict__ s) {
+    double beta = s[S_TMP0] / s[S_RZ];
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+        p[i] = z[i] + beta * p[i];
+}
+
+__global__ void k_copy_scalar(double *s, int dst, int src) {
+    if (threadIdx.x == 0) s[dst] = s[src];
 }
 
 // x -= x[corner] on non-boundary cells ; boundary entries set to 0
@@ -1684,23 +1922,14 @@ static int residual(tb_ctx *c, const PoisCtx &P, bool neumann, const double *x, 
 
 // FP64 GMG-preconditioned CG from the current x; returns iterations
 // rr_known: x is already pinned and kv[0] holds its residual, of squared norm
-// *rr_known; the first shift and residual are skipped.  The recursive
-// residual is read back (a stall of the stream for a host round trip) only
-// from two iterations before the count of the last solve on, and after
-// PCG_SKIP_MAX - 2 at the latest (far past convergence the recursive residual
-// underflows).
-constexpr int PCG_SKIP_MAX = 16;
+// *rr_known; the first shift and residual are skipped.
 static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double bn, double rtol, int maxit,
                  int &its, int &vcy, double &res, const double *rr_known) {
     long n = c->d.ntot;
-    double *r = c->kv[0], *z = c->kv[1], *p = c->kv[2], *q = c->kv[3], *po = c->kv[6];
-    const double ncell = (double)c->ncx * c->ncy * c->ncz;
-    const bool fused = (long)c->ncx * c->ncy * c->ncz <= PCG_FUSED_CELLS;
+    double *r = c->kv[0], *z = c->kv[1], *p = c->kv[2], *q = c->kv[3];
     double rr, bb;
-    // the V-cycle and k_pcg_p write interior cells only; keep the half-cell
-    // planes of z and p at 0
+    // the V-cycle writes interior cells only; keep z's half-cell planes at 0
     TB_CHECK(c, hipMemsetAsync(z, 0, sizeof(double) * n, c->s));
-    if (!fused) TB_CHECK(c, hipMemsetAsync(p, 0, sizeof(double) * n, c->s));
     if (rr_known) {
         rr = *rr_known;
     } else {
@@ -1708,90 +1937,194 @@ static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double
         if (residual(c, P, false, x, b, r, nullptr, rr, bb)) return -1;
     }
     res = sqrt(rr) / bn;
-    int slot = 0;
-    const int nvb = (int)std::min<long>(PB, (n + PT - 1) / PT);   // blocks of the vector kernels
-    // z = V(r), then p = z + beta p, q = A p and the partial sums of p . q
-    auto direction = [&](bool first) -> int {
+    // r . z of the V-cycle just run: from its last pair's partial sums, or a
+    // separate pass when the finest level has no pairs
+    auto rz = [&](int slot) -> int {
+        if (c->vc_dot_blocks[1] > 0) return tb_reduce_finish(c, c->vc_dot_blocks[1], 1, slot);
+        return tb_dot(c, r, z, slot);
+    };
+    while (res > rtol && its < maxit) {
         if (tb_vcycle64(c, r, z)) return -1;
         vcy++;
-        // the sums of r . z, z and r: the V-cycle's last smoothing launch's,
-        // or a separate pass when the finest level has no such
-        int nb = c->vc_dot_blocks;
-        if (nb == 0) {
-            nb = nvb;
-            hipLaunchKernelGGL(k_pcg_rz, dim3(nvb), dim3(PT), 0, c->s, n, (const double *)r, (const double *)z, c->red);
-            TB_LAUNCH_CHECK(c);
-        }
-        const int old = S_RZ + slot;
-        slot ^= 1;
-        const bool in = fused && nb <= SUM_INLINE;
-        if (!in)
-            hipLaunchKernelGGL(k_pcg_beta, dim3(1), dim3(1024), 0, c->s, (const double *)c->red, nb, c->scal, old,
-                               S_RZ + slot, first ? 1 : 0, ncell);
-        if (fused) {
-            std::swap(p, po);
-            const auto k = first ? (in ? k_pcg_pa<true, true> : k_pcg_pa<true, false>)
-                                 : (in ? k_pcg_pa<false, true> : k_pcg_pa<false, false>);
-            TB_PROF(c, TB_K_POIS_OP,
-                    hipLaunchKernelGGL(k, ktiles_grid(P.kt), tiles_block(), 0, c->s, P.Pn, (const double *)z,
-                                       (const double *)po, p, q, nb, c->scal, old, S_RZ + slot, ncell, c->red, P.kt));
-        } else {
-            hipLaunchKernelGGL(k_pcg_p, tiles_grid(P.cells), tiles_block(), 0, c->s, c->d, (const double *)z, p,
-                               (const double *)c->scal, first ? 1 : 0, P.cells);
-            TB_PROF(c, TB_K_POIS_OP,
-                    hipLaunchKernelGGL(k_pois_km<0>, ktiles_grid(P.kt), tiles_block(), 0, c->s, P.Pn,
-                                       (const double *)p, (const double *)nullptr, q, (float *)nullptr,
-                                       c->red + PQ_ARRAY * (long)RED_MAX_BLOCKS, P.kt));
-        }
-        TB_LAUNCH_CHECK(c);
-        return 0;
-    };
-    const int skip = c->pcg_its > 2 ? std::min(c->pcg_its, PCG_SKIP_MAX) - 2 : 0;
-    const int its0 = its;
-    // the recursive residual is followed no further than FP64's reach: beyond,
-    // the iteration only adds rounding to x (a residual of 6e-10 after 200
-    // iterations, from 2e-11 after 10, at 128x96x100 with a tolerance of 1e-18)
-    const double stop = std::max(0.5 * rtol, 1e-15);
-    // the passes that may leave the true residual above half of what it was
-    // before the tolerance counts as out of reach of FP64
-    int stalls = 3;
-    while (res > rtol && its < maxit) {
-        const double prev = res;
-        if (direction(true)) return -1;
+        TB_CHECK(c, hipMemcpyAsync(p, z, sizeof(double) * n, hipMemcpyDeviceToDevice, c->s));
+        if (rz(S_RZ)) return -1;
         int inner = 0;
         while (its < maxit) {
-            const bool in = P.nblk <= SUM_INLINE;
-            if (!in && tb_reduce_finish(c, (int)P.nblk, 1, S_PQ, PQ_ARRAY)) return -1;
-            TB_PROF(c, TB_K_PCG_UPD,
-                    hipLaunchKernelGGL(in ? k_pcg_xr<true> : k_pcg_xr<false>, dim3(nvb), dim3(PT), 0, c->s, n, x, r,
-                                       (const double *)p, (const double *)q, (int)P.nblk, (const double *)c->scal,
-                                       S_RZ + slot, c->red));
+            TB_PROF(c, TB_K_POIS_OP,
+                    hipLaunchKernelGGL(k_pois_km<0>, ktiles_grid(P.kt), tiles_block(), 0, c->s, P.Pn,
+                                       (const double *)p, (const double *)nullptr, q, (float *)nullptr, c->red, P.kt));
             TB_LAUNCH_CHECK(c);
+            if (tb_reduce_finish(c, (int)P.nblk, 1, S_PQ)) return -1;
+            TB_PROF(c, TB_K_PCG_UPD,
+                    hipLaunchKernelGGL(k_pcg_xr, dim3(PB), dim3(PT), 0, c->s, n, x, r, (const double *)p,
+                                       (const double *)q, (const double *)c->scal, c->red));
+            TB_LAUNCH_CHECK(c);
+            if (tb_reduce_read(c, PB, 1, S_RR)) return -1;
             its++;
             inner++;
-            if (inner >= 200) break;
-            if (its - its0 > skip && its < maxit) {
-                if (tb_reduce_read(c, nvb, 1, S_RR)) return -1;
-                double rrel = sqrt(c->hscal[S_RR]) / bn;
-                if (!(rrel == rrel)) { c->err = "Poisson CG produced NaN"; return -1; }
-                if (rrel <= stop) break;
-            }
-            if (its < maxit && direction(false)) return -1;
+            double rrel = sqrt(c->hscal[S_RR]) / bn;
+            if (!(rrel == rrel)) { c->err = "Poisson CG produced NaN"; return -1; }
+            if (rrel <= 0.5 * rtol || inner >= 200) break;
+            if (tb_vcycle64(c, r, z)) return -1;
+            vcy++;
+            if (rz(S_TMP0)) return -1;
+            hipLaunchKernelGGL(k_pcg_p, dim3(PB), dim3(PT), 0, c->s, n, (const double *)z, p, (const double *)c->scal);
+            hipLaunchKernelGGL(k_copy_scalar, dim3(1), dim3(64), 0, c->s, c->scal, S_RZ, S_TMP0);
+            TB_LAUNCH_CHECK(c);
         }
         if (shift_corner(c, P, x)) return -1;
         if (residual(c, P, false, x, b, r, nullptr, rr, bb)) return -1;
         res = sqrt(rr) / bn;
-        if (!(res == res)) { c->err = "Poisson CG produced NaN"; return -1; }
-        if (res > 0.5 * prev && --stalls == 0) break;
     }
-    if (res <= rtol) c->pcg_its = its - its0;
     return 0;
 }
 
 // ---------------------------------------------------------------------------
-// tb_set_mixed_inner: the cap of 0 leaves the refinement passes without FP32
-// work, so every mixed solve hands over to FP64 GMG-PCG at once; the reduction
-// floor is checked and kept, the direct FP32 solve has no target to stop at.
+// FP32 inner CG of the mixed-precision solve.  Vectors live in the level-0
+// layout (the padded field layout); every entry outside the interior cells is
+// 0 and stays 0, so the vector kernels sweep the whole array as float4.  Dot
+// products accumulate in FP64.
+
+// q = A p (Neumann -Laplacian of level 0) with the partial p.q
+__global__ void __launch_bounds__(256) k_cg32_apply(LV<float> L, const float *__restrict__ p, float *__restrict__ q,
+                                                    double *part, KTiles t) {
+    __shared__ double sh[16];
+    double acc[1] = {0.0};
+    int i, j, k0, k1;
+    bool act;
+    ktile_column(t, i, j, k0, k1, act);
+    if (act) {
+        const long pl = (long)L.px * L.py;
+        // absent neighbours are clamped to the cell itself and contribute 0
+        const long ow = i > 0 ? 1 : 0, oe = i < L.nx - 1 ? 1 : 0;
+        const long os = j > 0 ? L.px : 0, on = j < L.ny - 1 ? L.px : 0;
+        long id = lidx(L, i, j, k0);
+        float pm = p[id - (k0 > 0 ? pl : 0)];
+        float pc = p[id];
+        for (int k = k0; k < k1; k++) {
+            const float pp = p[id + (k < L.nz - 1 ? pl : 0)];
+            const float pw = p[id - ow], pe = p[id + oe], ps = p[id - os], pn = p[id + on];
+            const float v = L.cx * (pc - pw) + L.cx * (pc - pe) + L.cy * (pc - ps) + L.cy * (pc - pn) +
+                            L.cz * (pc - pm) + L.cz * (pc - pp);
+            st_stream(&q[id], v);
+            acc[0] += (double)pc * (double)v;
+            pm = pc;
+            pc = pp;
+            id += pl;
+        }
+    }
+    block_sum<1>(acc, sh);
+    if (threadIdx.x == 0 && threadIdx.y == 0) part[blockIdx.x] = acc[0];
+}
+
+// e += alpha p ; r -= alpha q ; partial r.r      (alpha = rz / pq)
+__global__ void __launch_bounds__(PT) k_cg32_xr(long n4, float4 *__restrict__ e, float4 *__restrict__ r,
+                                                const float4 *__restrict__ p, const float4 *__restrict__ q,
+                                                const double *__restrict__ s, double *part) {
+    __shared__ double sh[16];
+    const float alpha = (float)(s[S_RZ] / s[S_PQ]);
+    double acc[1] = {0.0};
+    for (long a = blockIdx.x * (long)blockDim.x + threadIdx.x; a < n4; a += (long)gridDim.x * blockDim.x) {
+        const float4 pv = p[a], qv = q[a];
+        float4 ev = e[a], rv = r[a];
+        ev.x += alpha * pv.x; ev.y += alpha * pv.y; ev.z += alpha * pv.z; ev.w += alpha * pv.w;
+        rv.x -= alpha * qv.x; rv.y -= alpha * qv.y; rv.z -= alpha * qv.z; rv.w -= alpha * qv.w;
+        e[a] = ev;
+        r[a] = rv;
+        acc[0] += (double)rv.x * rv.x + (double)rv.y * rv.y + (double)rv.z * rv.z + (double)rv.w * rv.w;
+    }
+    block_sum<1>(acc, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
+}
+
+__global__ void __launch_bounds__(PT) k_dot32(long n4, const float4 *__restrict__ a, const float4 *__restrict__ b,
+                                              double *part) {
+    __shared__ double sh[16];
+    double acc[1] = {0.0};
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n4; i += (long)gridDim.x * blockDim.x) {
+        const float4 u = a[i], v = b[i];
+        acc[0] += (double)u.x * v.x + (double)u.y * v.y + (double)u.z * v.z + (double)u.w * v.w;
+    }
+    block_sum<1>(acc, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
+}
+
+// p = z + beta p, beta = rz_new / rz
+__global__ void __launch_bounds__(PT) k_cg32_p(long n4, const float4 *__restrict__ z, float4 *__restrict__ p,
+                                               const double *__restrict__ s) {
+    const float beta = (float)(s[S_TMP0] / s[S_RZ]);
+    for (long a = blockIdx.x * (long)blockDim.x + threadIdx.x; a < n4; a += (long)gridDim.x * blockDim.x) {
+        const float4 zv = z[a];
+        float4 pv = p[a];
+        pv.x = zv.x + beta * pv.x; pv.y = zv.y + beta * pv.y; pv.z = zv.z + beta * pv.z; pv.w = zv.w + beta * pv.w;
+        p[a] = pv;
+    }
+}
+
+// Inner solve A e = r on level 0 by FP32 CG preconditioned with FP32
+// V-cycles, from e = 0, until ||r|| <= tol_rel * ||r0|| or maxit iterations.
+// r is lev[0].b32 (updated in place), z is lev[0].x32, e is cg32[2].
+// The first `skip` iterations run without reading their residual back (each
+// read-back stalls the stream for a host round trip); the caller takes skip
+// from the iterations an earlier solve needed.
+static int cg32_inner(tb_ctx *c, const KTiles &kt, double r0n, double tol_rel, int maxit, int skip, int &its,
+                      int &vcy) {
+    Level &L0 = c->lev[0];
+    const long n4 = L0.ntot / 4;
+    float *r = L0.b32, *z = L0.x32, *p = c->cg32[0], *q = c->cg32[1], *e = c->cg32[2];
+    const LV<float> lv = lv_of<float>(L0);
+    const int nblk = (int)(kt.per_xcd * NXCD);
+    TB_CHECK(c, hipMemsetAsync(e, 0, sizeof(float) * L0.ntot, c->s));
+    // r . z of the V-cycle just run: from its last pair's partial sums, or
+    // a separate pass when the finest level has no pairs
+    auto rz = [&](int slot) -> int {
+        if (c->vc_dot_blocks[0] > 0) return tb_reduce_finish(c, c->vc_dot_blocks[0], 1, slot);
+        hipLaunchKernelGGL(k_dot32, dim3(PB), dim3(PT), 0, c->s, n4, (const float4 *)r, (const float4 *)z, c->red);
+        TB_LAUNCH_CHECK(c);
+        return tb_reduce_finish(c, PB, 1, slot);
+    };
+    if (tb_vcycle32(c)) return -1;
+    vcy++;
+    TB_CHECK(c, hipMemcpyAsync(p, z, sizeof(float) * L0.ntot, hipMemcpyDeviceToDevice, c->s));
+    if (rz(S_RZ)) return -1;
+    int inner = 0;
+    while (inner < maxit) {
+        TB_PROF(c, TB_K_CG32_OP,
+                hipLaunchKernelGGL(k_cg32_apply, ktiles_grid(kt), tiles_block(), 0, c->s, lv, (const float *)p, q,
+                                   c->red, kt));
+        TB_LAUNCH_CHECK(c);
+        if (tb_reduce_finish(c, nblk, 1, S_PQ)) return -1;
+        TB_PROF(c, TB_K_CG32_UPD,
+                hipLaunchKernelGGL(k_cg32_xr, dim3(PB), dim3(PT), 0, c->s, n4, (float4 *)e, (float4 *)r,
+                                   (const float4 *)p, (const float4 *)q, (const double *)c->scal, c->red));
+        TB_LAUNCH_CHECK(c);
+        if (tb_reduce_finish(c, PB, 1, S_RR)) return -1;
+        inner++;
+        its++;
+        if (inner >= maxit) break;
+        if (inner > skip) {
+            if (read_s(c, S_RR, 1)) return -1;
+            const double rel = sqrt(c->hscal[S_RR]) / r0n;
+            if (!(rel == rel)) { c->err = "Poisson FP32 CG produced NaN"; return -1; }
+            if (rel <= tol_rel) break;
+        }
+        if (tb_vcycle32(c)) return -1;
+        vcy++;
+        if (rz(S_TMP0)) return -1;
+        hipLaunchKernelGGL(k_cg32_p, dim3(PB), dim3(PT), 0, c->s, n4, (const float4 *)z, (float4 *)p,
+                           (const double *)c->scal);
+        hipLaunchKernelGGL(k_copy_scalar, dim3(1), dim3(64), 0, c->s, c->scal, S_RZ, S_TMP0);
+        TB_LAUNCH_CHECK(c);
+    }
+    return 0;
+}
+
+// Mixed precision: FP64 iterative refinement (true residual r = b - A x in
+// FP64, rounded to FP32) around the FP32 inner CG, x += e in FP64.  Each inner
+// solve asks for the residual reduction still missing (times 0.5), but never
+// less than c->ir_floor (default 1e-5, which FP32 reaches reliably).  Stops at
+// rtol, at maxit inner iterations, or when an outer pass reduces the FP64
+// residual by less than half (stalled: the caller falls back to FP64 PCG).
 extern "C" int tb_set_mixed_inner(tb_ctx *c, double reduction_floor, int maxit) {
     if (!c || !(reduction_floor > 0.0 && reduction_floor < 1.0) || maxit < 0) {
         if (c) c->err = "tb_set_mixed_inner: bad argument";
@@ -1802,15 +2135,8 @@ extern "C" int tb_set_mixed_inner(tb_ctx *c, double reduction_floor, int maxit) 
     return 0;
 }
 
-// Mixed precision: FP64 iterative refinement (true residual r = b - A x in
-// FP64, rounded to FP32) around the direct FP32 solve of the Neumann operator
-// in cosine modes, x += e in FP64.  One pass reduces the residual to FP32's
-// rounding of the correction (1e-4 to 1e-6 of it); stops at rtol, at maxit
-// passes, or when a pass reduces the FP64 residual by less than half
-// (stalled: the caller falls back to FP64 PCG, as it does for a grid too long
-// for the direct solve).
-// rr_known: x is already pinned (corner exactly 0) and r32 holds its FP32
-// residual, of squared norm *rr_known; the first shift and residual are
+// rr_known: x is already pinned (corner exactly 0) and lev[0].b32 holds its
+// FP32 residual, of squared norm *rr_known; the first shift and residual are
 // skipped.  Every refinement pass adds the correction and pins x in one
 // kernel, so its residual (Neumann rows, with x[corner] = 0 the same vector
 // as the pinned one) is the true residual of the result: no further pass
@@ -1819,33 +2145,41 @@ extern "C" int tb_set_mixed_inner(tb_ctx *c, double reduction_floor, int maxit) 
 static int mixed_ir(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double bn, double rtol, int maxit,
                     int &its, int &vcy, double &res, bool &stalled, const double *rr_known) {
     double *r = nullptr;   // only the FP32 copy of the residual and its norms are needed
+    Level &L0 = c->lev[0];
     double rr, bb;
     stalled = false;
     if (tb_mg_build(c)) return -1;
+    const KTiles kt0 = make_ktiles(L0.nx, L0.ny, L0.nz);
+    if (kt0.per_xcd * NXCD > RED_MAX_BLOCKS) { c->err = "grid too large for the reduction buffer"; return -1; }
     if (rr_known) {
         rr = *rr_known;
     } else {
         if (shift_corner(c, P, x)) return -1;
-        if (residual(c, P, true, x, b, r, c->r32, rr, bb)) return -1;
+        if (residual(c, P, true, x, b, r, L0.b32, rr, bb)) return -1;
     }
     res = sqrt(rr) / bn;
-    if ((c->ir_maxit == 0 || !c->spec32) && res > rtol) {
-        stalled = true;   // a pass would leave x as it is
+    if (c->ir_maxit == 0 && res > rtol) {
+        // no FP32 work allowed: the first pass would leave x as it is
+        stalled = true;
         return 0;
     }
     while (res > rtol && its < maxit) {
         const double prev = res;
-        if (c->prof_on) tb_prof_begin(c, TB_K_MG_SMALL);
-        if (tb_spec_solve<float>(c, c->lev[0], c->r32, c->x32)) return -1;
-        if (c->prof_on) tb_prof_end(c, TB_K_MG_SMALL);
-        its++;
-        vcy++;
-        hipLaunchKernelGGL(k_corner_after_add, dim3(1), dim3(64), 0, c->s, (const double *)x, (const float *)c->x32,
-                           P.corner, c->scal);
-        hipLaunchKernelGGL(k_add32_pin, tiles_grid(P.cells), tiles_block(), 0, c->s, c->d, x, (const float *)c->x32,
-                           (const double *)c->scal, P.cells);
+        double want = 0.5 * rtol / res;
+        if (want < c->ir_floor) want = c->ir_floor;
+        int room = maxit - its;
+        // the first pass skips the tests of all but the last two iterations
+        // the previous solve's first pass needed
+        const int skip = (its == 0 && c->ir_first_its > 2) ? c->ir_first_its - 2 : 0;
+        const int its_before = its;
+        if (cg32_inner(c, kt0, sqrt(rr), want, room < c->ir_maxit ? room : c->ir_maxit, skip, its, vcy)) return -1;
+        if (its_before == 0) c->ir_first_its = its;
+        hipLaunchKernelGGL(k_corner_after_add, dim3(1), dim3(64), 0, c->s, (const double *)x,
+                           (const float *)c->cg32[2], P.corner, c->scal);
+        hipLaunchKernelGGL(k_add32_pin, tiles_grid(P.cells), tiles_block(), 0, c->s, c->d, x,
+                           (const float *)c->cg32[2], (const double *)c->scal, P.cells);
         TB_LAUNCH_CHECK(c);
-        if (residual(c, P, true, x, b, r, c->r32, rr, bb)) return -1;
+        if (residual(c, P, true, x, b, r, L0.b32, rr, bb)) return -1;
         res = sqrt(rr) / bn;
         if (!(res == res)) { c->err = "Poisson IR produced NaN"; return -1; }
         if (res > 0.5 * prev) { stalled = true; break; }
@@ -2008,7 +2342,7 @@ static void launch_dots(tb_ctx *c, long n, const Dirs &D, const double *b, const
     else hipLaunchKernelGGL((k_guess_dots<H, false>), dim3(PB), dim3(PT), 0, c->s, n, D, b, d, q, c->red);
 }
 
-// On return with ndir > 0, x is pinned and r32 holds the FP32 copy of
+// On return with ndir > 0, x is pinned and lev[0].b32 holds the FP32 copy of
 // its residual, whose squared norm is rrg (and that of b bbg); with ndir = 0
 // x is untouched.  c->guess_r / guess_nr receive the products phi_k . b for
 // the Galerkin matrix of the next solve.
@@ -2103,7 +2437,7 @@ static int learned_guess(tb_ctx *c, const PoisCtx &P, double *x, const double *b
     // vector (the rows differ only in the corner's own coefficient): one
     // pass gives the guess's residual norm, the norm of b and the FP32
     // residual the mixed solve starts from.
-    if (residual(c, P, true, x, b, nullptr, c->r32, rrg, bbg)) return -1;
+    if (residual(c, P, true, x, b, nullptr, c->lev[0].b32, rrg, bbg)) return -1;
     return 0;
 }
 
@@ -2222,7 +2556,7 @@ static int poisson_solve(tb_ctx *c, tb_solve_stats *st, int guess_f, bool output
         } else {
             TB_CHECK(c, hipMemcpyAsync(x, c->f[guess_f], sizeof(double) * c->d.ntot, hipMemcpyDeviceToDevice, c->s));
             if (shift_corner(c, P, x)) return -1;
-            if (residual(c, P, !plain, x, b, plain ? c->kv[0] : nullptr, plain ? nullptr : c->r32, rr_g, bb_g))
+            if (residual(c, P, !plain, x, b, plain ? c->kv[0] : nullptr, plain ? nullptr : c->lev[0].b32, rr_g, bb_g))
                 return -1;
             ndir = 1;
         }
@@ -2245,7 +2579,7 @@ static int poisson_solve(tb_ctx *c, tb_solve_stats *st, int guess_f, bool output
             c->phi_pinned = true;
         }
     }
-    double rr_top = 0.0, rr_first = rr;
+    double rr_top = 0.0;
     if (!guess_resid) {
         // the field left by the previous solve is pinned already (the shift
         // would subtract exactly 0)
@@ -2254,16 +2588,8 @@ static int poisson_solve(tb_ctx *c, tb_solve_stats *st, int guess_f, bool output
         // FP64 PCG takes r (kv[0]), the mixed solve its FP32 copy (x is
         // pinned, so the Neumann and the pinned residual are the same vector)
         double *r_top = plain ? c->kv[0] : nullptr;
-        float *r32_top = plain ? nullptr : c->r32;
+        float *r32_top = plain ? nullptr : c->lev[0].b32;
         if (residual(c, P, !plain, x, b, r_top, r32_top, rr, bb)) return -1;
-        // the increments of the two RK stages differ in size (their right-hand
-        // sides by up to 400 times at 64x16x16): where the field left by the
-        // last solve starts further off than zero does, zero it is
-        rr_first = rr;
-        if (rr > bb && std::isfinite(rr)) {
-            TB_CHECK(c, hipMemsetAsync(x, 0, sizeof(double) * c->d.ntot, c->s));
-            if (residual(c, P, !plain, x, b, r_top, r32_top, rr, bb)) return -1;
-        }
     }
     rr_top = rr;
     c->phi_pinned = false;
@@ -2273,7 +2599,7 @@ static int poisson_solve(tb_ctx *c, tb_solve_stats *st, int guess_f, bool output
         TB_CHECK(c, hipMemsetAsync(x, 0, sizeof(double) * c->d.ntot, c->s));
         loc.converged = 1;
     } else {
-        loc.res0 = sqrt(rr_first) / bn;
+        loc.res0 = sqrt(rr) / bn;
         if (plain) {
             if (pcg64(c, P, x, b, bn, rtol, maxit, its, vcy, res, &rr_top)) return -1;
         } else {
