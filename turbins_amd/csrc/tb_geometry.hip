@@ -591,7 +591,8 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
     if (c->has_geometry) {
         // the Krylov vectors are free here; kv[4] alone may be written outside
         // the box points (the others' row padding stays 0): it holds the
-        // heights first, then the second iterate
+        // heights first, then the second iterate, whose padding is cleared of
+        // what transfers left there, since the whole rows may become sdf_c's
         double *p0 = c->kv[0], *dh = c->kv[4], *sgn = c->kv[2], *dist = c->kv[3], *alt = c->kv[4], *part = c->red;
         const bool own_part = all.per_xcd * NXCD > (long)RED_SLOTS * RED_MAX_BLOCKS;
         if (own_part) TB_CHECK(c, hipMalloc((void **)&part, sizeof(double) * (size_t)(all.per_xcd * NXCD)));
@@ -599,6 +600,7 @@ int tb_geometry_run(tb_ctx *c, const double *h_xz) {
         double offset = c->cfg.bottom_offset ? c->hgrid[13][0] * 2.001 : 0.0;   // Grid.c:913
         hipLaunchKernelGGL(k_sdf_guess, tiles_grid(all), tiles_block(), 0, c->s, d, c->g, dh, offset, p0, sdf_c, all);
         TB_LAUNCH_CHECK(c);
+        TB_CHECK(c, hipMemsetAsync(alt, 0, sizeof(double) * d.ntot, c->s));
         // Levelset_compute_fictitious_time (Levelset.c:590-637)
         double dmin_[3] = {1000.0, 1000.0, 1000.0};
         for (int a = 0; a < d.NX - 1; a++) if (c->hgrid[12][a] < dmin_[0]) dmin_[0] = c->hgrid[12][a];
