@@ -154,3 +154,29 @@ def test_trained_network_gain():
         assert worth > 0.5 * g["net_ms_per_call"]
     else:
         assert worth < 1.5 * g["net_ms_per_call"]
+
+
+def test_inference_holds_no_weight_gradient_buffers():
+    """A first forward pass on a new size takes the activations; the operand
+    copies of the weight gradients (48 BF16 channels per voxel at least) come
+    with the first backward pass."""
+    import ctypes
+    n = Net(seed=2)
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert n.L.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    shape = (96, 96, 96)
+    in3 = np.zeros(shape + (3,), dtype=np.float32)
+    tgt = np.zeros(shape, dtype=np.float32)
+    n.forward(in3[:8, :8, :8])
+    n.gradient(in3[:8, :8, :8], tgt[:8, :8, :8])
+    n.forward(in3)
+    before = free()
+    n.gradient(in3, tgt)
+    taken = before - free()
+    print("memory the first backward pass takes", taken)
+    assert taken >= 96 * tgt.size
+    n.close()

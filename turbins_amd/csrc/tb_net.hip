@@ -920,22 +920,28 @@ static int acts_ensure(tb_net *net, Acts &A, int nx, int ny, int nz, bool train)
             {&A.gp1, A.v2 * 32}, {&A.gx1, A.v1 * 32}, {&A.gp0, A.v1 * 16}};
         for (auto &e : gb)
             if (net_alloc(net, A, (void **)e.p, b2 * e.n)) return -1;
-        long px = 0, pg = 0, pp = 0;
-        for (int l = 0; l < NLAYER; l++) {
-            const int lev = LAYER_LEVEL[l];
-            const WgShape w = wg_shape(nx >> lev, ny >> lev, nz >> lev, LAYERS[l].cin, LAYERS[l].cout);
-            px = std::max(px, w.plane * LAYERS[l].cin);
-            pg = std::max(pg, w.plane * std::max(LAYERS[l].cout, 3));
-            pp = std::max(pp, (long)w.pairs * w.nblk * WG_ELEMS);
-        }
-        if (net_alloc(net, A, (void **)&A.plx, b2 * px) || net_alloc(net, A, (void **)&A.plg, b2 * pg) ||
-            net_alloc(net, A, (void **)&A.wpart, sizeof(float) * pp))
-            return -1;
         if (net_alloc(net, A, (void **)&A.tgt, sizeof(float) * A.v0)) return -1;
         if (net_alloc(net, A, (void **)&A.gout, sizeof(float) * A.v0)) return -1;
     }
     A.nx = nx; A.ny = ny; A.nz = nz; A.train = train;   // last: a set that was cut short is made anew
     return 0;
+}
+
+// the weight gradients' buffers of a training set, which only a backward pass
+// needs (128 bytes or more per voxel: an inference goes without)
+static int wgrad_ensure(tb_net *net, Acts &A) {
+    if (A.wpart) return 0;
+    long px = 0, pg = 0, pp = 0;
+    for (int l = 0; l < NLAYER; l++) {
+        const int lev = LAYER_LEVEL[l];
+        const WgShape w = wg_shape(A.nx >> lev, A.ny >> lev, A.nz >> lev, LAYERS[l].cin, LAYERS[l].cout);
+        px = std::max(px, w.plane * LAYERS[l].cin);
+        pg = std::max(pg, w.plane * std::max(LAYERS[l].cout, 3));
+        pp = std::max(pp, (long)w.pairs * w.nblk * WG_ELEMS);
+    }
+    if (!A.plx && net_alloc(net, A, (void **)&A.plx, sizeof(bf16_t) * px)) return -1;
+    if (!A.plg && net_alloc(net, A, (void **)&A.plg, sizeof(bf16_t) * pg)) return -1;
+    return net_alloc(net, A, (void **)&A.wpart, sizeof(float) * pp);
 }
 
 static int pack_frags(tb_net *net) {
@@ -1231,7 +1237,7 @@ extern "C" int tb_net_forward(tb_net *net, const float *in3, int nx, int ny, int
     if (!net || !in3 || !out) return -1;
     if (acts_ensure(net, net->trn, nx, ny, nz, true)) return -1;
     Acts &A = net->trn;
-    float *d3 = (float *)A.plx;   // at least 16 BF16 channels per voxel, free until a backward pass
+    float *d3 = (float *)A.du0;   // 48 BF16 channels per voxel, free until a backward pass
     if (tb_xfer(net->xfer, net->s, net->err, const_cast<float *>(in3), d3, sizeof(float) * 3 * A.v0, true)) return -1;
     hipLaunchKernelGGL(k_expand3, grid1d(A.v0), dim3(256), 0, net->s, (const float *)d3, A.v0, A.in16);
     if (forward(net, net->s, A)) return -1;
@@ -1242,9 +1248,9 @@ extern "C" int tb_net_forward(tb_net *net, const float *in3, int nx, int ny, int
 extern "C" int tb_net_gradient(tb_net *net, const float *in3, const float *target, int nx, int ny, int nz,
                                double *loss, float *grad) {
     if (!net || !in3 || !target || !grad) return -1;
-    if (acts_ensure(net, net->trn, nx, ny, nz, true)) return -1;
+    if (acts_ensure(net, net->trn, nx, ny, nz, true) || wgrad_ensure(net, net->trn)) return -1;
     Acts &A = net->trn;
-    float *d3 = (float *)A.plx;
+    float *d3 = (float *)A.du0;
     if (tb_xfer(net->xfer, net->s, net->err, const_cast<float *>(in3), d3, sizeof(float) * 3 * A.v0, true) ||
         tb_xfer(net->xfer, net->s, net->err, const_cast<float *>(target), A.tgt, sizeof(float) * A.v0, true))
         return -1;
@@ -1294,13 +1300,13 @@ extern "C" int tb_net_train(tb_net *net, int steps, int batch, int cx, int cy, i
                             double *loss_first, double *loss_last) {
     if (!net || net->count < 1 || steps < 0 || batch < 1) { if (net) net->err = "tb_net_train: no snapshots"; return -1; }
     if (cx > net->sx || cy > net->sy || cz > net->sz) { net->err = "crop larger than the snapshots"; return -1; }
-    if (acts_ensure(net, net->trn, cx, cy, cz, true)) return -1;
+    if (acts_ensure(net, net->trn, cx, cy, cz, true) || wgrad_ensure(net, net->trn)) return -1;
     int lanes = net->trn.v0 <= TRAIN_LANE_VOXELS ? std::min(batch, TRAIN_LANES) : 1;
     for (int a = 0; a < lanes; a++) {
         if (!net->lane_ev[a]) NET_CHECK(net, hipEventCreateWithFlags(&net->lane_ev[a], hipEventDisableTiming));
         if (a == 0) continue;
         if (!net->lane_s[a - 1]) NET_CHECK(net, hipStreamCreate(&net->lane_s[a - 1]));
-        if (acts_ensure(net, net->lane_a[a - 1], cx, cy, cz, true)) {
+        if (acts_ensure(net, net->lane_a[a - 1], cx, cy, cz, true) || wgrad_ensure(net, net->lane_a[a - 1])) {
             // no memory for more lanes: those that there are take all crops
             acts_free(net->lane_a[a - 1]);
             (void)hipGetLastError();
