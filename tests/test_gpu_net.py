@@ -180,3 +180,23 @@ def test_inference_holds_no_weight_gradient_buffers():
     print("memory the first backward pass takes", taken)
     assert taken >= 96 * tgt.size
     n.close()
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3.4e38])
+def test_overflowed_gradient_keeps_its_kind(bad):
+    """The head's bias gradient is the plain sum of the output gradient,
+    2 (out - target) / n: an infinite target makes it infinite, not NaN, and
+    one near the largest float leaves it finite (n = 512 divides it first)."""
+    n = Net(seed=4)
+    tgt = np.zeros((8, 8, 8), dtype=np.float32)
+    tgt[3, 4, 5] = bad
+    _, g = n.gradient(np.ones((8, 8, 8, 3), dtype=np.float32), tgt)
+    db = g[_layer_slices()[15]][0]
+    print("bias gradient", bad, db)
+    if np.isnan(bad):
+        assert np.isnan(db)
+    elif np.isinf(bad):
+        assert db == -bad
+    else:
+        assert abs(db + 2.0 * 3.4e38 / 512) <= 1e-6 * 2.0 * 3.4e38 / 512
+    n.close()

@@ -346,7 +346,8 @@ __global__ void __launch_bounds__(256) k_planar(Src s, int nx, int ny, int nz, i
 }
 
 // an FP32 field as three planar BF16 channels whose sum is exact (8 + 8 + 8
-// significant bits)
+// significant bits; an infinity or NaN is the first one alone, and a value
+// that would round up to infinity is cut off instead)
 __global__ void __launch_bounds__(256) k_planar_split(const float *__restrict__ g, int nx, int ny, int nz, int nx8,
                                                       bf16_t *__restrict__ out) {
     const long total = (long)nx8 * ny * nz, plane = 8 * total;
@@ -360,9 +361,10 @@ __global__ void __launch_bounds__(256) k_planar_split(const float *__restrict__ 
             float v = x < nx ? g[((long)z * ny + y) * nx + x] : 0.f;
 #pragma unroll
             for (int a = 0; a < 3; a++) {
-                const bf16_t b = f2bf(v);
+                bf16_t b = f2bf(v);
+                if (isinf(bf2f(b)) && isfinite(v)) b = (bf16_t)(__float_as_uint(v) >> 16);
                 h[a][i >> 1] |= (uint32_t)b << (16 * (i & 1));
-                v -= bf2f(b);
+                v = isfinite(v) ? v - bf2f(b) : 0.f;
             }
         }
 #pragma unroll
