@@ -62,3 +62,45 @@ def test_set_matches_bicgstab(name, dims, kind):
             assert d <= 1e-9
     a.close()
     b.close()
+
+
+def _by_entry_points(g, dt):
+    """tb_step through the public entry points, its predictor systems one by one."""
+    g.store_old()
+    helm = []
+    for stage in range(2):
+        g.eno_conv_rhs(dt)
+        helm.append([g.helmholtz_solve(q, dt) for q in range(4)])
+        g.poisson_rhs(dt)
+        g.poisson_solve()
+        g.project(dt)
+    g.rk_average(0.5, 0.5)
+    return helm
+
+
+@pytest.mark.parametrize("name,dims,steps", [
+    ("bump_small", (65, 17, 33), 3),             # a set
+    ("turbidity1024", (1024, 256, 128), 1),      # above 2^25 points (rows padded to 16): one by one in the step too
+])
+def test_step_matches_entry_points(name, dims, steps):
+    """The sets share launches, not arithmetic: a step gives the bits, the pairs
+    and the residuals of the quantities solved by calls of their own."""
+    c = W.case(name, **dict(zip(("nx", "ny", "nz"), dims)))
+    prof = 0.5 * (1.0 - np.tanh((W.cell_centres(dims[0], c["lx"]) - 1.0) / 0.1))
+    out = []
+    for split in (False, True):
+        print("step", name, dims, "by entry points" if split else "", flush=True)
+        g = Solver(W.config_for(c))
+        g.setup_geometry(W.topography(c))
+        conc = np.tile(prof, (dims[1] + 1) * (dims[2] + 1))
+        conc[g.flags(3) != abi.FLUID] = 0.0
+        g.upload("C", conc)
+        for _ in range(steps):
+            helm = _by_entry_points(g, c["dt"]) if split else g.step(c["dt"]).helm
+        out.append(([[(h.iterations, h.res, h.fallback) for h in st] for st in helm],
+                    {n: g.download(n) for n in ("U", "V", "W", "C", "DPDX")}))
+        g.close()
+    print(out[0][0], flush=True)
+    assert out[0][0] == out[1][0]
+    for n, a in out[0][1].items():
+        assert np.array_equal(a, out[1][1][n]), n

@@ -58,7 +58,10 @@ struct GsSet {   // a kernel argument: at most 4 KB
     __device__ const GsView &mine() const { return v[N == 1 ? 0 : blockIdx.y]; }
 };
 
-static_assert(sizeof(GsSet<HELM_SET>) <= 4096 - 64, "kernel arguments");
+// k_helm_check's argument list is the longest; the runtime's own arguments
+// follow in the same segment
+static_assert(sizeof(GsSet<HELM_SET>) + sizeof(double *) + sizeof(long) + sizeof(KTiles) <= 4096 - 256,
+              "kernel arguments");
 
 // wall rule applied to ap when a neighbour is absent:
 // 0 nothing (normal component on the wall), 1 no-slip (ap -= a),
