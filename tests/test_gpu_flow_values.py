@@ -32,6 +32,9 @@ FLOWS = {
     # three grain sizes with hindered settling
     "grains92": dict(nx=92, ny=32, nz=32, re=2000.0, mode=abi.POIS_MIXED_IR, bump="gauss8", grains=3, open=False,
                      steps=5),
+    # the predictor systems by BiCGStab
+    "bicg67": dict(nx=67, ny=19, nz=13, re=2000.0, mode=abi.POIS_MIXED_IR, bump="gauss8", helm=abi.HELM_BICGSTAB,
+                   open=False, steps=4),
     # a finest level of 1.6 million cells
     "box256": dict(nx=256, ny=96, nz=64, re=2000.0, mode=abi.POIS_MIXED_IR, open=False, steps=2),
 }
@@ -42,6 +45,7 @@ def flow_samples(name):
     c = W.case("bump512x128", nx=f["nx"], ny=f["ny"], nz=f["nz"], re=f["re"], particle=True, v_settle=0.02,
                eno_order=f.get("eno_order", 2), bump=f.get("bump", "gauss1"))
     g = Solver(W.config_for(c, pois_rtol=1e-10, helm_rtol=1e-12, pois_mode=f["mode"]))
+    g.set_helmholtz_method(f.get("helm", abi.HELM_GS))
     g.setup_geometry(W.topography(c))
     init = W.initial_fields(c, [g.flags(q) for q in range(4)])
     for n, a in init.items():

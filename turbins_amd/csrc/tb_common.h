@@ -120,11 +120,12 @@ __device__ inline bool tile_point_kfast(const Tiles &t, int &i, int &j, int &k) 
 // column 512 and row 256) are listed 256 to a block, and the last k chunk
 // takes up to KCHUNK/2 extra planes (129 planes: 8 chunks, not 9).  Each
 // block is a chain of plane steps, so nearly empty tiles would cost as much
-// time as full ones; for the same reason the Helmholtz kernels, whose sums
-// only decide when a solve stops, walk grids with fewer than KTILES_BLOCKS
-// blocks (four per CU) in shorter chunks.  The Poisson operator keeps whole
-// chunks: its partial sums enter the conjugate gradient's steps, and their
-// order is part of what a solve to a finite tolerance returns.
+// time as full ones; for the same reason the Gauss-Seidel solves' residual
+// check, whose sums only decide when a solve stops, walks grids with fewer
+// than KTILES_BLOCKS blocks (four per CU) in shorter chunks (`shorten`).  The
+// operators inside conjugate gradient and BiCGStab keep whole chunks: their
+// partial sums enter the iterations' steps, and the order of those sums is
+// part of what a solve to a finite tolerance returns.
 constexpr int KCHUNK = 16;
 constexpr int KTILES_BLOCKS = 1024;
 

@@ -295,7 +295,7 @@ static int helm_apply(tb_ctx *c, const HelmOp &H, const double *x, double *y, bo
     if (c->nib[q] > 0)
         hipLaunchKernelGGL(k_ib_apply, dim3((c->nib[q] + 255) / 256), dim3(256), 0, c->s, c->ib_row[q], c->ib_cnt[q],
                            c->ib_col[q], c->ib_val[q], c->nib[q], x, y, scaled ? H.mod : 0.0);
-    KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ, true);
+    KTiles t = make_ktiles(c->d.NX, c->d.NY, c->d.NZ);
     if (c->prof_on) tb_prof_begin(c, TB_K_HELM_OP);
     if (mode == 0)
         hipLaunchKernelGGL(k_helm_km<0>, ktiles_grid(t), tiles_block(), 0, c->s, H, x, y, w, c->red, t);
