@@ -10,9 +10,8 @@ Helmholtz solve to 1e-12.  Two device paths are timed on the same state:
   headline -- learned mode: Galerkin guess on the last eight solutions and
               the trained network's direction (the network is dropped at
               run time if its saved iterations cost more than its
-              inference), then a direct FP32 solve in cosine modes inside
-              FP64 iterative refinement (FP64 GMG-PCG takes over if it
-              stalls)
+              inference), then FP32 CG with FP32 V-cycles inside FP64
+              iterative refinement (FP64 GMG-PCG takes over if it stalls)
 The JSON line's `value` is the headline path's timesteps/s.  Inputs are
 resident in HBM before the timed region; each library step ends with a
 device synchronisation, so the wall clock brackets exactly K steps.
@@ -54,14 +53,15 @@ BYTES_PER_POINT = {
     # momentum u, v, w, three flags, three pressure gradients and c in, three
     # right-hand sides out; concentration c, u, v, w and a flag in, one out
     "ENO_MOM": 83, "ENO_CONC": 41, "PROJECT": 115, "BICG_UPD": 56, "PCG_UPD": 48, "POIS_OP": 16,
+    "CG32_OP": 8, "CG32_UPD": 24,
 }
 WEIGHTS = os.path.join(ROOT, "turbins_amd", "weights", "poisson_guess.f32")
 # HBM bytes per instrumented launch measured with rocprofv3 FETCH_SIZE /
 # WRITE_SIZE on this workload, scaled by a plain copy of known size
 # (profiles/hbm_traffic_bump512x256.md); only valid for the kernels as built.
-# HELM_GS: the sweep pair, and the first pair of a solve, which also reads
-# the last solve's increment
-MEASURED_TRAFFIC = {"HELM_GS": 463.8e6, "HELM_GS_FIRST": 552.2e6}
+# HELM_GS: one solve's sweep pair in a launch of four, and the first pair of a
+# solve, which also reads the last solve's increment
+MEASURED_TRAFFIC = {"HELM_GS": 469.2e6, "HELM_GS_FIRST": 565.1e6}
 
 
 def log(*a):
@@ -148,7 +148,8 @@ def roofline(prof, stats, c):
         elif name == "HELM_OP":
             # the Gauss-Seidel solves' residual checks, at least one each: x,
             # b, the field it started from and the status in, the FP32
-            # increment out
+            # increment out.  A solve checked twice counts once: the rate
+            # is a lower bound
             total = 29 * NT * n_first
         elif name == "HELM_GS":
             # one fused red+black sweep pair: x, b and the status byte read
@@ -158,6 +159,8 @@ def roofline(prof, stats, c):
             total = 25 * NT * helm_its + 4 * NT * n_first
         elif name == "RBGS0":
             total = 24 * ncell * n      # FP64 fused pair: x, b read, x written
+        elif name == "RBGS0_F32":
+            total = 12 * ncell * n      # FP32 fused pair: x, b read, x written
         else:
             continue
         if best is None or ms > best[1]:
@@ -349,7 +352,7 @@ def main():
             "helmholtz_rtol": 1e-12,
             "headline_path": "Galerkin guess from the last eight solutions"
                              + (" + network direction while its gate is open" if learned else "")
-                             + ", direct FP32 solve inside FP64 iterative refinement",
+                             + ", FP32 CG + FP32 V-cycles inside FP64 iterative refinement",
             "learned_guess_loaded": learned,
             # what the timed headline steps ran: the network's direction
             # only while its run-time gate was open
@@ -368,7 +371,7 @@ def main():
             "solve_ms_per_step_plain": phase_ms(st_plain),
             "headline_vs_fp64_step_rel_l2": mixed_err,
             "solve_ms_per_step_headline": phase_ms(st_head),
-            "precision": "FP64 fields/ENO/Helmholtz/outer Poisson; FP32 direct solve in the headline path",
+            "precision": "FP64 fields/ENO/Helmholtz/outer Poisson; FP32 multigrid in the headline path",
         },
         "roofline": rl,
     }
