@@ -1852,6 +1852,47 @@ __global__ void k_copy_scalar(double *s, int dst, int src) {
     if (threadIdx.x == 0) s[dst] = s[src];
 }
 
+// The projected iteration's pieces (pcg64_projected): partial sums of r . z, z
+// and r ...
+__global__ void __launch_bounds__(PT) k_proj_sums(long n, const double *__restrict__ r, const double *__restrict__ z,
+                                                  double *part) {
+    __shared__ double sh[48];
+    double acc[3] = {0.0, 0.0, 0.0};
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        const double ri = r[i], zi = z[i];
+        acc[0] += ri * zi;
+        acc[1] += zi;
+        acc[2] += ri;
+    }
+    block_sum<3>(acc, sh);
+    if (threadIdx.x == 0)
+        for (int a = 0; a < 3; a++) part[a * RED_MAX_BLOCKS + blockIdx.x] = acc[a];
+}
+
+// ... p = (z - mean) + beta p on the cells (z and p may be one vector) ...
+__global__ void __launch_bounds__(256) k_proj_p(Dims d, const double *z, double *p, double mean, double beta, Tiles t) {
+    int i, j, k;
+    if (!tile_point(t, i, j, k)) return;
+    const long id = gidx(d, i, j, k);
+    p[id] = (z[id] - mean) + beta * p[id];
+}
+
+// ... x += alpha p ; r -= alpha q ; partial r.r
+__global__ void __launch_bounds__(PT) k_proj_xr(long n, double *__restrict__ x, double *__restrict__ r,
+                                                const double *__restrict__ p, const double *__restrict__ q, double alpha,
+                                                double *part) {
+    __shared__ double sh[16];
+    double acc[1] = {0.0};
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        x[i] += alpha * p[i];
+        const double ri = r[i] - alpha * q[i];
+        r[i] = ri;
+        acc[0] += ri * ri;
+    }
+    block_sum<1>(acc, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
+}
+
 // x -= x[corner] on non-boundary cells ; boundary entries set to 0
 __global__ void __launch_bounds__(256) k_shift(Dims d, double *__restrict__ x, const double *__restrict__ s, Tiles t) {
     int i, j, k;
@@ -1920,7 +1961,80 @@ static int residual(tb_ctx *c, const PoisCtx &P, bool neumann, const double *x, 
     return 0;
 }
 
-// FP64 GMG-preconditioned CG from the current x; returns iterations
+// CG on the zero-mean space, for a solve that broke down (NaN).  The operator's
+// null space is the constant: the V-cycle's output has an arbitrary mean that
+// the operator does not see but r . z does, and where a right-hand side is
+// small or not quite compatible (the mean of its rounding, open faces) that
+// spoils beta until the directions overflow.  Here the residual starts without
+// its mean, z's mean is taken out of the direction and of r . z, and a
+// vanishing direction ends nothing (alpha = 0).  pcg64 and the FP32 iteration
+// stay without the projection: what they return, converged or at their cap,
+// they return to the last bit as ever.  The scalars go through the host
+// (three read-backs an iteration).  From the current x, or from zero if that is
+// no better; at most `more` iterations.
+static int pcg64_projected(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double bn, double rtol, int more,
+                           int &its, int &vcy, double &res) {
+    const long n = c->d.ntot;
+    double *r = c->kv[0], *z = c->kv[1], *p = c->kv[2], *q = c->kv[3];
+    const double ncell = (double)c->ncx * c->ncy * c->ncz;
+    // a breakdown leaves NaN in the row padding too, which the vector kernels
+    // sweep and nothing else writes
+    for (double *v : {r, z, p, q}) TB_CHECK(c, hipMemsetAsync(v, 0, sizeof(double) * n, c->s));
+    if (!(res < 1.0)) TB_CHECK(c, hipMemsetAsync(x, 0, sizeof(double) * n, c->s));
+    double rr, bb;
+    if (residual(c, P, false, x, b, r, nullptr, rr, bb)) return -1;
+    res = sqrt(rr) / bn;
+    // below FP64's reach the iteration only adds rounding to x
+    const double stop = std::max(0.5 * rtol, 1e-15);
+    const int last = its + more;
+    int stalls = 3;   // passes that may leave more than half of the residual
+    while (res > rtol && its < last) {
+        const double prev = res;
+        double rz_old = 0.0;
+        TB_CHECK(c, hipMemsetAsync(z, 0, sizeof(double) * n, c->s));
+        TB_CHECK(c, hipMemsetAsync(p, 0, sizeof(double) * n, c->s));
+        hipLaunchKernelGGL(k_proj_sums, dim3(PB), dim3(PT), 0, c->s, n, (const double *)r, (const double *)z, c->red);
+        TB_LAUNCH_CHECK(c);
+        if (tb_reduce_read(c, PB, 3, S_TMP0)) return -1;
+        // r = (r - mean) + 0 * r
+        hipLaunchKernelGGL(k_proj_p, tiles_grid(P.cells), tiles_block(), 0, c->s, c->d, (const double *)r, r,
+                           c->hscal[S_TMP2] / ncell, 0.0, P.cells);
+        for (int inner = 0; its < last && inner < 200; inner++) {
+            if (tb_vcycle64(c, r, z)) return -1;
+            vcy++;
+            hipLaunchKernelGGL(k_proj_sums, dim3(PB), dim3(PT), 0, c->s, n, (const double *)r, (const double *)z, c->red);
+            TB_LAUNCH_CHECK(c);
+            if (tb_reduce_read(c, PB, 3, S_TMP0)) return -1;
+            const double mean = c->hscal[S_TMP1] / ncell, rz = c->hscal[S_TMP0] - mean * c->hscal[S_TMP2];
+            hipLaunchKernelGGL(k_proj_p, tiles_grid(P.cells), tiles_block(), 0, c->s, c->d, (const double *)z, p, mean,
+                               rz_old == 0.0 ? 0.0 : rz / rz_old, P.cells);
+            TB_PROF(c, TB_K_POIS_OP,
+                    hipLaunchKernelGGL(k_pois_km<0>, ktiles_grid(P.kt), tiles_block(), 0, c->s, P.Pn,
+                                       (const double *)p, (const double *)nullptr, q, (float *)nullptr, c->red, P.kt));
+            TB_LAUNCH_CHECK(c);
+            if (tb_reduce_read(c, (int)P.nblk, 1, S_PQ)) return -1;
+            const double pq = c->hscal[S_PQ];
+            hipLaunchKernelGGL(k_proj_xr, dim3(PB), dim3(PT), 0, c->s, n, x, r, (const double *)p, (const double *)q,
+                               pq == 0.0 ? 0.0 : rz / pq, c->red);
+            TB_LAUNCH_CHECK(c);
+            if (tb_reduce_read(c, PB, 1, S_RR)) return -1;
+            rz_old = rz;
+            its++;
+            const double rrel = sqrt(c->hscal[S_RR]) / bn;
+            if (!(rrel == rrel)) { c->err = "Poisson CG produced NaN"; return -1; }
+            if (rrel <= stop) break;
+        }
+        if (shift_corner(c, P, x)) return -1;
+        if (residual(c, P, false, x, b, r, nullptr, rr, bb)) return -1;
+        res = sqrt(rr) / bn;
+        if (!(res == res)) { c->err = "Poisson CG produced NaN"; return -1; }
+        if (res > 0.5 * prev && --stalls == 0) break;
+    }
+    return 0;
+}
+
+// FP64 GMG-preconditioned CG from the current x; returns iterations.  Where it
+// breaks down pcg64_projected takes over, with up to maxit more.
 // rr_known: x is already pinned and kv[0] holds its residual, of squared norm
 // *rr_known; the first shift and residual are skipped.
 static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double bn, double rtol, int maxit,
@@ -1943,6 +2057,7 @@ static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double
         if (c->vc_dot_blocks[1] > 0) return tb_reduce_finish(c, c->vc_dot_blocks[1], 1, slot);
         return tb_dot(c, r, z, slot);
     };
+    bool broken = false;
     while (res > rtol && its < maxit) {
         if (tb_vcycle64(c, r, z)) return -1;
         vcy++;
@@ -1963,7 +2078,7 @@ static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double
             its++;
             inner++;
             double rrel = sqrt(c->hscal[S_RR]) / bn;
-            if (!(rrel == rrel)) { c->err = "Poisson CG produced NaN"; return -1; }
+            if (!(rrel == rrel)) { broken = true; break; }
             if (rrel <= 0.5 * rtol || inner >= 200) break;
             if (tb_vcycle64(c, r, z)) return -1;
             vcy++;
@@ -1972,6 +2087,7 @@ static int pcg64(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double
             hipLaunchKernelGGL(k_copy_scalar, dim3(1), dim3(64), 0, c->s, c->scal, S_RZ, S_TMP0);
             TB_LAUNCH_CHECK(c);
         }
+        if (broken) return pcg64_projected(c, P, x, b, bn, rtol, maxit, its, vcy, res = INFINITY);
         if (shift_corner(c, P, x)) return -1;
         if (residual(c, P, false, x, b, r, nullptr, rr, bb)) return -1;
         res = sqrt(rr) / bn;
@@ -2066,9 +2182,11 @@ __global__ void __launch_bounds__(PT) k_cg32_p(long n4, const float4 *__restrict
 // r is lev[0].b32 (updated in place), z is lev[0].x32, e is cg32[2].
 // The first `skip` iterations run without reading their residual back (each
 // read-back stalls the stream for a host round trip); the caller takes skip
-// from the iterations an earlier solve needed.
+// from the iterations an earlier solve needed.  broken: the iteration broke
+// down (see pcg64_projected) and e holds nothing of use; r is then cleared, whose
+// row padding the vector kernels sweep.
 static int cg32_inner(tb_ctx *c, const KTiles &kt, double r0n, double tol_rel, int maxit, int skip, int &its,
-                      int &vcy) {
+                      int &vcy, bool &broken) {
     Level &L0 = c->lev[0];
     const long n4 = L0.ntot / 4;
     float *r = L0.b32, *z = L0.x32, *p = c->cg32[0], *q = c->cg32[1], *e = c->cg32[2];
@@ -2101,12 +2219,15 @@ static int cg32_inner(tb_ctx *c, const KTiles &kt, double r0n, double tol_rel, i
         if (tb_reduce_finish(c, PB, 1, S_RR)) return -1;
         inner++;
         its++;
-        if (inner >= maxit) break;
-        if (inner > skip) {
+        if (inner > skip || inner >= maxit) {
             if (read_s(c, S_RR, 1)) return -1;
             const double rel = sqrt(c->hscal[S_RR]) / r0n;
-            if (!(rel == rel)) { c->err = "Poisson FP32 CG produced NaN"; return -1; }
-            if (rel <= tol_rel) break;
+            if (!(rel == rel)) {
+                broken = true;
+                TB_CHECK(c, hipMemsetAsync(r, 0, sizeof(float) * L0.ntot, c->s));
+                break;
+            }
+            if (rel <= tol_rel || inner >= maxit) break;
         }
         if (tb_vcycle32(c)) return -1;
         vcy++;
@@ -2125,6 +2246,7 @@ static int cg32_inner(tb_ctx *c, const KTiles &kt, double r0n, double tol_rel, i
 // less than c->ir_floor (default 1e-5, which FP32 reaches reliably).  Stops at
 // rtol, at maxit inner iterations, or when an outer pass reduces the FP64
 // residual by less than half (stalled: the caller falls back to FP64 PCG).
+// broken: the FP32 iteration broke down and pcg64_projected finished the solve.
 extern "C" int tb_set_mixed_inner(tb_ctx *c, double reduction_floor, int maxit) {
     if (!c || !(reduction_floor > 0.0 && reduction_floor < 1.0) || maxit < 0) {
         if (c) c->err = "tb_set_mixed_inner: bad argument";
@@ -2143,11 +2265,11 @@ extern "C" int tb_set_mixed_inner(tb_ctx *c, double reduction_floor, int maxit) 
 // follows the last one.  On return x is pinned, res is its pinned relative
 // residual and the last residual pass ran on x.
 static int mixed_ir(tb_ctx *c, const PoisCtx &P, double *x, const double *b, double bn, double rtol, int maxit,
-                    int &its, int &vcy, double &res, bool &stalled, const double *rr_known) {
+                    int &its, int &vcy, double &res, bool &stalled, bool &broken, const double *rr_known) {
     double *r = nullptr;   // only the FP32 copy of the residual and its norms are needed
     Level &L0 = c->lev[0];
     double rr, bb;
-    stalled = false;
+    stalled = broken = false;
     if (tb_mg_build(c)) return -1;
     const KTiles kt0 = make_ktiles(L0.nx, L0.ny, L0.nz);
     if (kt0.per_xcd * NXCD > RED_MAX_BLOCKS) { c->err = "grid too large for the reduction buffer"; return -1; }
@@ -2172,7 +2294,13 @@ static int mixed_ir(tb_ctx *c, const PoisCtx &P, double *x, const double *b, dou
         // the previous solve's first pass needed
         const int skip = (its == 0 && c->ir_first_its > 2) ? c->ir_first_its - 2 : 0;
         const int its_before = its;
-        if (cg32_inner(c, kt0, sqrt(rr), want, room < c->ir_maxit ? room : c->ir_maxit, skip, its, vcy)) return -1;
+        if (cg32_inner(c, kt0, sqrt(rr), want, room < c->ir_maxit ? room : c->ir_maxit, skip, its, vcy, broken)) return -1;
+        if (broken) {
+            // x is as it was; the next solve reads every iteration's residual
+            // until it knows their number again
+            c->ir_first_its = 0;
+            return pcg64_projected(c, P, x, b, bn, rtol, maxit, its, vcy, res);
+        }
         if (its_before == 0) c->ir_first_its = its;
         hipLaunchKernelGGL(k_corner_after_add, dim3(1), dim3(64), 0, c->s, (const double *)x,
                            (const float *)c->cg32[2], P.corner, c->scal);
@@ -2603,9 +2731,11 @@ static int poisson_solve(tb_ctx *c, tb_solve_stats *st, int guess_f, bool output
         if (plain) {
             if (pcg64(c, P, x, b, bn, rtol, maxit, its, vcy, res, &rr_top)) return -1;
         } else {
-            bool stalled = false;
-            if (mixed_ir(c, P, x, b, bn, rtol, maxit, its, vcy, res, stalled, &rr_top)) return -1;
-            if (res > rtol) {
+            bool stalled, broken;
+            if (mixed_ir(c, P, x, b, bn, rtol, maxit, its, vcy, res, stalled, broken, &rr_top)) return -1;
+            if (broken) {
+                loc.fallback |= 1;       // the FP64 iteration for breakdowns took over
+            } else if (res > rtol) {
                 loc.fallback |= 1;   // plain FP64 GMG-PCG takes over
                 if (pcg64(c, P, x, b, bn, rtol, maxit, its, vcy, res, nullptr)) return -1;
             }
